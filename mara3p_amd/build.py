@@ -63,7 +63,7 @@ def build_hip(verbose=False, jobs=None):
 def build_oracle(verbose=False):
     oracle = os.path.join(ROOT, "oracle")
     _run(["make", "-s", "-C", oracle, os.path.join(oracle, "liboracle.so")], verbose)
-    if os.path.isdir(REFERENCE):
+    if os.path.isfile(os.path.join(REFERENCE, "problems", "minidisk_scheme.cpp")):
         _run(["make", "-s", "-C", oracle, "REFERENCE=" + REFERENCE, "ref"], verbose)
 
 
