@@ -323,9 +323,12 @@ int m3p_srhd_riemann_array(const double* pl, const double* pr, double* f, long n
 
 /* Tile selection and autotuning (no reference counterpart: the reference runs
  * one closure per block on a CPU thread pool).  A 2D stage workgroup owns TJ
- * contiguous columns of a block and marches down H rows; the compiled
- * variants are TJ x H in {256x32, 256x16, 128x32, 64x64, 64x32, 64x16, 32x32,
- * 16x16}.  The choice is per process, per (kind, precision). */
+ * contiguous columns of a block and marches down H rows (tiles narrower than
+ * 64 columns as 64 / TJ strips side by side); the compiled variants are TJ x H
+ * in {256x128, 256x64, 256x32, 256x16, 128x64, 128x32, 64x64, 64x32, 64x16,
+ * 64x8, 64x4, 64x2, 32x32, 32x16, 32x8, 32x4, 16x16, 16x8}.  Without a choice
+ * the library picks by the size of the mesh; a choice holds for the process,
+ * per (kind, precision), where it divides the block size. */
 int m3p_set_stage2d_tile(int kind, int precision, int tj, int h);
 int m3p_get_stage2d_tile(int kind, int precision, int* tj /* host */, int* h /* host */);
 /* Time every variant that fits on the caller's mesh (u -> out, `reps`

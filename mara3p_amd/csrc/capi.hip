@@ -197,8 +197,9 @@ struct Lease {
 
 // ---------------------------------------------------------------------------
 // 2D launch dispatch.  The variant used for each (scheme kind, precision) is
-// a per-process setting (an index into kTileVariants) chosen by
-// m3p_set_stage2d_tile or m3p_autotune_*; it is read and written atomically.
+// chosen by the size of the mesh (pick_tile), unless a caller has chosen one
+// for the process with m3p_set_stage2d_tile or m3p_autotune_* (an index into
+// kTileVariants, read and written atomically).
 constexpr int kNumKinds = 3;
 constexpr int tile_index(int tj, int h)
 {
@@ -206,30 +207,50 @@ constexpr int tile_index(int tj, int h)
         if (kTileVariants[i].tj == tj && kTileVariants[i].h == h) return i;
     return -1;
 }
-// [kind][precision]: defaults from sweeps of the benchmark meshes; the tree
-// kind runs 64^2 leaves, where 64 x 16 tiles give the most workgroups.
-std::atomic<int> g_tile[kNumKinds][2] = { { tile_index(256, 16), tile_index(256, 16) },
-                                          { tile_index(256, 16), tile_index(256, 16) },
-                                          { tile_index(64, 16), tile_index(64, 16) } };
+// [kind][precision]: the shape of meshes that fill the device, from sweeps of
+// the benchmark meshes (the tree kind runs 64^2 leaves); g_tile holds a
+// caller's choice, or -1.
+constexpr TileShape kLargeTile[kNumKinds] = { {256, 16}, {256, 16}, {64, 16} };
+std::atomic<int> g_tile[kNumKinds][2] = { { -1, -1 }, { -1, -1 }, { -1, -1 } };
 
 bool tile_fits(TileShape v, int n) { return n % v.tj == 0 && n % v.h == 0 && v.h <= n; }
 
-TileShape pick_tile(int kind, int precision, int n)
+// The tile of a stage over nblk blocks of n x n zones: the caller's choice
+// where it fits, else by the size of the mesh.  A wave marches the rows of
+// its strip in series (2 to 3 us a row for FP64 Euler), so a mesh of few
+// zones is bound by that chain and wants short strips; every strip also
+// recovers four extra rows and computes one extra row of x fluxes, so a mesh
+// that fills the device wants long ones.  The lines are from sweeps of both
+// stages on meshes of 64^2 to 4096^2 zones: two-row strips below 2048 waves
+// of four rows (FP64 Euler, 256^2 zones in 32^2 blocks: 24 us a step, 32 with
+// four rows, 92 with sixteen), four rows up to 2048 waves of eight, eight up
+// to 4096 waves of sixteen (1024^2 zones in 64^2 blocks: FP64 95 us against
+// 115 with sixteen rows, mixed 47 against 65).  Beyond that sixteen rows in
+// FP64 (2048^2: 325 us against 339 with eight), eight in mixed (153 against
+// 169) and on quad-trees (1408 leaves of 64^2, mixed: 223 against 233).
+TileShape pick_tile(int kind, int precision, int n, int nblk)
 {
-    TileShape want = kTileVariants[g_tile[kind][precision].load(std::memory_order_relaxed)];
-    if (tile_fits(want, n)) return want;
-    // widest fitting tile, then the fewest rows (most workgroups)
-    TileShape best{0, 0};
-    for (auto v : kTileVariants)
-        if (tile_fits(v, n) && (v.tj > best.tj || (v.tj == best.tj && v.h < best.h))) best = v;
-    return best;
+    const int chosen = g_tile[kind][precision].load(std::memory_order_relaxed);
+    if (chosen >= 0 && tile_fits(kTileVariants[chosen], n)) return kTileVariants[chosen];
+    const double zones = (double)nblk * n * n;
+    auto waves = [&] (int rows) { return zones / (64.0 * rows); };
+    int rows = waves(16) >= 4096 ? 16 : waves(8) >= 2048 ? 8 : waves(4) >= 2048 ? 4 : 2;
+    if (rows == 16 && kind != M3P_KIND_AMR_EULER2D) {
+        if (tile_fits(kLargeTile[kind], n)) return kLargeTile[kind];
+        if (precision == M3P_MIXED && n % 128 == 0) return {128, 32};     // 153 us against 163 (64 x 8) at 2048^2
+    }
+    if (rows == 16 && (precision == M3P_MIXED || kind == M3P_KIND_AMR_EULER2D)) rows = 8;
+    if (n % 64 == 0) return {64, rows};
+    if (n % 32 == 0) return {32, 2 * rows};                   // two strips a wave
+    if (n % 16 == 0) return {16, 4 * std::min(rows, 4)};      // four
+    return {0, 0};
 }
 
 template<class S, class Ld>
 int launch_stage2d(int kind, const typename S::Params& prm, const Ld& ld, const StageArgs& a, hipStream_t s)
 {
     const int prec = is_fp64<typename S::Real>::value ? M3P_FP64 : M3P_MIXED;
-    const TileShape ts = pick_tile(kind, prec, a.n);
+    const TileShape ts = pick_tile(kind, prec, a.n, a.nblk);
     if (ts.tj == 0) return fail(M3P_ERR_BAD_SHAPE, "m3p: 2D block size must be 16, 32 or a multiple of 64 (got " + std::to_string(a.n) + ")");
     return launch_stage2d_shape<S, Ld>(ts, prm, ld, a, s);
 }
@@ -1127,7 +1148,8 @@ int m3p_set_stage2d_tile(int kind, int precision, int tj, int h)
 int m3p_get_stage2d_tile(int kind, int precision, int* tj, int* h)
 {
     if (kind < 0 || kind >= kNumKinds || precision < 0 || precision > 1) return fail(M3P_ERR_BAD_ARGUMENT, "m3p: bad kind/precision");
-    const TileShape v = kTileVariants[g_tile[kind][precision].load(std::memory_order_relaxed)];
+    const int i = g_tile[kind][precision].load(std::memory_order_relaxed);
+    const TileShape v = i >= 0 ? kTileVariants[i] : kLargeTile[kind];
     if (tj) *tj = v.tj;
     if (h) *h = v.h;
     return M3P_OK;

@@ -21,7 +21,8 @@ int launch_status(const char* what);
 // 2D stage tiles: TJ columns x H rows (the compiled variants).
 struct TileShape { int tj, h; };
 constexpr TileShape kTileVariants[] = { {256, 128}, {256, 64}, {256, 32}, {256, 16}, {128, 64}, {128, 32},
-                                        {64, 64}, {64, 32}, {64, 16}, {32, 32}, {16, 16} };
+                                        {64, 64}, {64, 32}, {64, 16}, {64, 8}, {64, 4}, {64, 2}, {32, 32}, {32, 16},
+                                        {32, 8}, {32, 4}, {16, 16}, {16, 8} };
 constexpr int kNumVariants = sizeof(kTileVariants) / sizeof(kTileVariants[0]);
 
 // One 2D stage with tile shape ts (a compiled variant).

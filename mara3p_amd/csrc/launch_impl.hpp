@@ -14,22 +14,29 @@ int launch_stage2d_variant(TileShape ts, const typename S::Params& prm, const Ld
     // and its update; the FP64 kernels (register-bound) re-load it.
     constexpr bool K = !is_fp64<typename S::Real>::value;
     const int n = a.n;
-    auto go = [&] (auto kern) {
+    auto go = [&] (auto kern, int strips) {
         const int grid = a.nblk * (n / ts.h) * (n / ts.tj);
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(ts.tj), 0, s, prm, ld, a);
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(ts.tj * strips), 0, s, prm, ld, a);
         return launch_status("stage2d_kernel");
     };
-    if (ts.tj == 256 && ts.h == 128) return go(stage2d_kernel<S, Ld, 128, 256, K, FIRST>);
-    if (ts.tj == 256 && ts.h == 64) return go(stage2d_kernel<S, Ld, 64, 256, K, FIRST>);
-    if (ts.tj == 256 && ts.h == 32) return go(stage2d_kernel<S, Ld, 32, 256, K, FIRST>);
-    if (ts.tj == 256 && ts.h == 16) return go(stage2d_kernel<S, Ld, 16, 256, K, FIRST>);
-    if (ts.tj == 128 && ts.h == 64) return go(stage2d_kernel<S, Ld, 64, 128, K, FIRST>);
-    if (ts.tj == 128 && ts.h == 32) return go(stage2d_kernel<S, Ld, 32, 128, K, FIRST>);
-    if (ts.tj == 64 && ts.h == 64)  return go(stage2d_kernel<S, Ld, 64, 64, K, FIRST>);
-    if (ts.tj == 64 && ts.h == 32)  return go(stage2d_kernel<S, Ld, 32, 64, K, FIRST>);
-    if (ts.tj == 64 && ts.h == 16)  return go(stage2d_kernel<S, Ld, 16, 64, K, FIRST>);
-    if (ts.tj == 32 && ts.h == 32)  return go(stage2d_kernel<S, Ld, 32, 32, K, FIRST>);
-    if (ts.tj == 16 && ts.h == 16)  return go(stage2d_kernel<S, Ld, 16, 16, K, FIRST>);
+    if (ts.tj == 256 && ts.h == 128) return go(stage2d_kernel<S, Ld, 128, 256, 1, K, FIRST>, 1);
+    if (ts.tj == 256 && ts.h == 64) return go(stage2d_kernel<S, Ld, 64, 256, 1, K, FIRST>, 1);
+    if (ts.tj == 256 && ts.h == 32) return go(stage2d_kernel<S, Ld, 32, 256, 1, K, FIRST>, 1);
+    if (ts.tj == 256 && ts.h == 16) return go(stage2d_kernel<S, Ld, 16, 256, 1, K, FIRST>, 1);
+    if (ts.tj == 128 && ts.h == 64) return go(stage2d_kernel<S, Ld, 64, 128, 1, K, FIRST>, 1);
+    if (ts.tj == 128 && ts.h == 32) return go(stage2d_kernel<S, Ld, 32, 128, 1, K, FIRST>, 1);
+    if (ts.tj == 64 && ts.h == 64)  return go(stage2d_kernel<S, Ld, 64, 64, 1, K, FIRST>, 1);
+    if (ts.tj == 64 && ts.h == 32)  return go(stage2d_kernel<S, Ld, 32, 64, 1, K, FIRST>, 1);
+    if (ts.tj == 64 && ts.h == 16)  return go(stage2d_kernel<S, Ld, 16, 64, 1, K, FIRST>, 1);
+    if (ts.tj == 64 && ts.h == 8)   return go(stage2d_kernel<S, Ld, 8, 64, 1, K, FIRST>, 1);
+    if (ts.tj == 64 && ts.h == 4)   return go(stage2d_kernel<S, Ld, 4, 64, 1, K, FIRST>, 1);
+    if (ts.tj == 64 && ts.h == 2)   return go(stage2d_kernel<S, Ld, 2, 64, 1, K, FIRST>, 1);
+    if (ts.tj == 32 && ts.h == 32)  return go(stage2d_kernel<S, Ld, 32, 32, 2, K, FIRST>, 2);
+    if (ts.tj == 32 && ts.h == 16)  return go(stage2d_kernel<S, Ld, 16, 32, 2, K, FIRST>, 2);
+    if (ts.tj == 32 && ts.h == 8)   return go(stage2d_kernel<S, Ld, 8, 32, 2, K, FIRST>, 2);
+    if (ts.tj == 32 && ts.h == 4)   return go(stage2d_kernel<S, Ld, 4, 32, 2, K, FIRST>, 2);
+    if (ts.tj == 16 && ts.h == 16)  return go(stage2d_kernel<S, Ld, 16, 16, 4, K, FIRST>, 4);
+    if (ts.tj == 16 && ts.h == 8)   return go(stage2d_kernel<S, Ld, 8, 16, 4, K, FIRST>, 4);
     return fail(M3P_ERR_BAD_SHAPE, "m3p: 2D block size must be 16, 32 or a multiple of 64 (got " + std::to_string(n) + ")");
 }
 

@@ -305,11 +305,22 @@ __device__ __forceinline__ void store_edge_flux(double* reg, int b, int e, int n
 // at the update (fewer registers).  FIRST: a stage without a base state
 // (a.u0 == nullptr is then assumed); it has fewer loads in flight per row, so
 // a scheme may ask it to fetch more rows ahead (S::kPrefetchRows).
-template<class S, class Ld, int H, int TJ, bool KEEPU, bool FIRST = false>
-__global__ void __launch_bounds__(TJ) __attribute__((amdgpu_waves_per_eu(S::kWavesPerEU, 8)))
+//
+// G: a tile of H rows is marched as G strips of H / G rows, by G groups of TJ
+// lanes side by side.  A tile narrower than a wave (TJ = 16 or 32) takes
+// G = 64 / TJ, so that its rows fill the wave.  Its row addresses differ from
+// lane to lane and live in vector registers, so it runs at one wave per SIMD
+// less, where it does not spill (168 VGPRs spill 16 to 32).
+constexpr int stage2d_waves(int waves, int strips) { return strips > 1 && waves > 2 ? waves - 1 : waves; }
+
+template<class S, class Ld, int H, int TJ, int G, bool KEEPU, bool FIRST = false>
+__global__ void __launch_bounds__(TJ * G) __attribute__((amdgpu_waves_per_eu(stage2d_waves(S::kWavesPerEU, G), 8)))
 stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
 {
     constexpr int NC = S::NC;
+    constexpr int NT = TJ * G;                 // lanes of the workgroup
+    constexpr int HS = H / G;                  // rows of a strip
+    static_assert(H % G == 0, "whole strips");
     using R = typename S::Real;
     resolve_params(prm);
 
@@ -331,7 +342,9 @@ stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
     if (a.bcoord) { tc.bi = a.bcoord[2 * tc.b]; tc.bj = a.bcoord[2 * tc.b + 1]; }
     else          { tc.bi = a.bi0; tc.bj = a.bj0; }
 
-    const int t = threadIdx.x;
+    const int lane = threadIdx.x;              // of the workgroup (the pre-pass)
+    const int g = G > 1 ? lane / TJ : 0;       // the lane's strip and its column in the tile
+    const int t = G > 1 ? lane % TJ : lane;
     const int c = tc.c0 + t;
     const int b = tc.b;
     const double dt = a.dt_dev ? *a.dt_dev : a.dt;
@@ -345,15 +358,18 @@ stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
     __shared__ R hraw[7][NC][H];     // pre-pass primitives at 7 edge columns
     __shared__ R hG[NC][H];          // y half slope at column c0-1
     __shared__ R hF[NC][H];          // y flux at face c0+TJ
-    __shared__ R rowP[NC][TJ + 2];   // [t+1] = column c0+t; [0], [TJ+1] from hraw
-    __shared__ R rowG[NC][TJ + 1];   // [t+1] = half slope at column c0+t; [0] from hG
-    __shared__ R rowF[NC][TJ + 1];   // [t] = y flux at face c0+t; [TJ] from hF
+    __shared__ R rowPs[G][NC][TJ + 2];   // [t+1] = column c0+t; [0], [TJ+1] from hraw
+    __shared__ R rowGs[G][NC][TJ + 1];   // [t+1] = half slope at column c0+t; [0] from hG
+    __shared__ R rowFs[G][NC][TJ + 1];   // [t] = y flux at face c0+t; [TJ] from hF
+    R (&rowP)[NC][TJ + 2] = rowPs[g];
+    R (&rowG)[NC][TJ + 1] = rowGs[g];
+    R (&rowF)[NC][TJ + 1] = rowFs[g];
 
     S::setup(td, prm, tc);
     bool ok = true;
 
     // ---- halo pre-pass --------------------------------------------------
-    for (int idx = t; idx < 7 * H; idx += TJ) {
+    for (int idx = lane; idx < 7 * H; idx += NT) {
         const int r = idx / 7, q = idx % 7;
         const int cols[7] = { tc.c0 - 2, tc.c0 - 1, tc.c0, tc.c0 + TJ - 2, tc.c0 + TJ - 1, tc.c0 + TJ, tc.c0 + TJ + 1 };
         R p[NC];
@@ -363,7 +379,7 @@ stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
     }
     __syncthreads();
     const R theta = R(S::theta(prm));
-    for (int r = t; r < H; r += TJ) {
+    for (int r = lane; r < H; r += NT) {
         R pl[NC], pr[NC], f[NC];
 #pragma unroll
         for (int m = 0; m < NC; ++m) {
@@ -396,7 +412,7 @@ stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
     // fewer registers across the row).
     auto march = [&] (auto dir) {
         constexpr int D = decltype(dir)::value;
-        const int kfirst = D > 0 ? tc.k0 : tc.k0 + H - 1;
+        const int kfirst = D > 0 ? tc.k0 + g * HS : tc.k0 + g * HS + HS - 1;
 
         // warm-up: rows kfirst - 2D .. kfirst + D, flux at the face behind kfirst
         R Pa[NC], Pb[NC], ga[NC];   // current row, next row, half slope at the current row
@@ -439,7 +455,7 @@ stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
         // Prefetched raw rows: Unx[i] = row k + (2 + i) D of the iteration
         // that follows, kAhead rows in flight.
         constexpr int kAhead = FIRST ? S::kPrefetchRows : 1;
-        static_assert(kAhead >= 1 && kAhead <= H, "rows ahead within the tile");
+        static_assert(kAhead >= 1 && kAhead <= HS, "rows ahead within the strip");
         double Unx[kAhead][NC] = {};
         if constexpr (Ld::kPrefetch) {
 #pragma unroll
@@ -447,7 +463,7 @@ stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
         }
         constexpr int kRowsPerIter = Ld::kUnroll ? S::kMarchUnroll : 1;
 #pragma unroll kRowsPerIter
-        for (int kk = 0; kk < H; ++kk) {
+        for (int kk = 0; kk < HS; ++kk) {
             const int k = kfirst + D * kk;
             const int kl = k - tc.k0;
             R Pc[NC], gb[NC], pl[NC], pr[NC], Fa[NC], gy[NC], Fy[NC];
@@ -460,8 +476,8 @@ stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
                 for (int i = 0; i + 1 < kAhead; ++i)
 #pragma unroll
                     for (int m = 0; m < NC; ++m) Unx[i][m] = Unx[i + 1][m];
-                // the last row a tile reads is kfirst + (H + 1) D
-                if (kk + kAhead < H) ld.fetch_row(b, k + (2 + kAhead) * D, c, Unx[kAhead - 1]);
+                // the last row a strip reads is kfirst + (HS + 1) D
+                if (kk + kAhead < HS) ld.fetch_row(b, k + (2 + kAhead) * D, c, Unx[kAhead - 1]);
                 if constexpr (!S::kLateBase) {
                     if (!FIRST && a.u0) {
                         const double* z0 = a.u0 + ((size_t)b * NC * n + k) * n + c;
@@ -590,11 +606,12 @@ stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
             }
         }
     };
-    if (((rem / tiles_j) & 1) == 0) march(std::integral_constant<int, 1>{});
-    else                            march(std::integral_constant<int, -1>{});
+    // (the strips of a split tile share a wave, hence one direction)
+    if (G > 1 || ((rem / tiles_j) & 1) == 0) march(std::integral_constant<int, 1>{});
+    else                                     march(std::integral_constant<int, -1>{});
     if (!ok) report_error(a.err, 1, b, 0);
     if constexpr (S::kCfl) {
-        if (a.rate_slot) workgroup_atomic_max<TJ>(rate, a.rate_slot);
+        if (a.rate_slot) workgroup_atomic_max<NT>(rate, a.rate_slot);
     }
 }
 

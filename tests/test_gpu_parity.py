@@ -228,6 +228,39 @@ def test_every_tile_shape_gives_the_same_minidisk_step(precision):
         assert err <= 1e-12, err
 
 
+@pytest.mark.parametrize("n, depth", [(16, 0), (16, 5), (32, 1), (32, 5), (48, 1), (64, 0), (64, 3), (64, 4), (64, 5),
+                                      (96, 2), (128, 4), (192, 1), (192, 3)])
+def test_tile_of_each_mesh_size(n, depth):
+    """The tile that the library picks by the size of the mesh (block sizes of
+    each width, meshes on both sides of each line of the rule): FP64 equals
+    the oracle, mixed the same step of one fixed tile shape."""
+    from mara3p_amd import problems
+    from mara3p_amd._lib import M3P_KIND_EULER2D, M3P_MIXED
+    from mara3p_amd.mesh import to_device_layout, to_reference_layout
+    from mara3p_amd.solvers import Euler2DSolver
+    mesh, u0 = problems.kelvin_helmholtz(depth=depth, block_size=n, seed=5)
+    for precision in ("fp64", "mixed"):
+        s = Euler2DSolver(depth, n, precision=precision)
+        dt = 0.4 * s.dl / 2.0
+        s.set_state(u0)
+        s.step(dt)
+        s.check_errors()
+        got = s.state()
+        if precision == "fp64":
+            ref = to_reference_layout(u0).copy()
+            assert orc().orc_euler2d_mesh_rk2(P(ref), mesh.nb, n, dt, s.dl, 1.5, 5.0 / 3.0, 0, 1, 8) == 0
+            assert np.array_equal(got, to_device_layout(ref))
+        else:
+            tj = 64 if n % 64 == 0 else 32 if n % 32 == 0 else 16
+            restore = _with_tile(M3P_KIND_EULER2D, M3P_MIXED, tj, tj)
+            try:
+                s.set_state(u0)
+                s.step(dt)
+                assert np.array_equal(got, s.state())
+            finally:
+                restore()
+
+
 def test_minidisk_mesh_rk2_fp64():
     from mara3p_amd import MinidiskData, problems
     from mara3p_amd.mesh import to_device_layout, to_reference_layout
