@@ -220,8 +220,8 @@ int m3p_euler1d_stage(const double* u, const double* u0, double* out, const int*
  *   faces stored).
  * With u0 != NULL the RK combine out = base * rk_b + advance * (1 - rk_b) is
  * fused (examples/mhd3d.cpp:77-86 weighted_sum).  work: device scratch of at
- * least m3p_mhd_workspace_bytes(N, precision) bytes (primitives, face fluxes
- * and face fields).  Asynchronous; negative density / pressure are latched
+ * least m3p_mhd_workspace_bytes(N, precision) bytes (primitives and face
+ * fields).  Asynchronous; negative density / pressure are latched
  * (M3P_ERR_NEGATIVE_DENSITY / _PRESSURE, src/physics_mhd.hpp:296-300). */
 long m3p_mhd_workspace_bytes(int N, int precision);
 int  m3p_mhd_advance_ct(const double* uc, const double* bf1, const double* bf2, const double* bf3,
@@ -235,9 +235,8 @@ int  m3p_mhd_advance_ct(const double* uc, const double* bf1, const double* bf2, 
  * m3p_mhd_advance_ct, with no workspace argument: the workspace is a static
  * device array of 48 MiB inside the library (one per GPU, held until the
  * process ends), so N is limited to what fits (m3p_mhd_workspace_bytes(N,
- * precision) <= 48 MiB: N a multiple of 8, whose passes keep no face fluxes,
- * up to 72 in FP64 and 96 mixed; any other N up to 59 and 75); a larger N fails with
- * M3P_ERR_BAD_ARGUMENT.  Kernel errors (negative density or pressure) go to
+ * precision) <= 48 MiB: N up to 76 in FP64 and 96 mixed); a larger N fails
+ * with M3P_ERR_BAD_ARGUMENT.  Kernel errors (negative density or pressure) go to
  * status, a caller's device int[4] (code, block, zone) that the call clears
  * first; m3p_check_errors does not see them.  Nothing is allocated, with
  * hipMalloc, torch or otherwise.  All calls on one GPU share the one array,

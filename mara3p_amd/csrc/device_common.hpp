@@ -194,4 +194,13 @@ __device__ __forceinline__ int xcd_remap(int w, int total)
     return (w % nxcd) * (total / nxcd) + (w / nxcd);
 }
 
+// The same within each run of `chunk` workgroups (a multiple of 8; the
+// workgroups after the last whole run stay): the XCDs advance through the
+// runs together, each on its own contiguous part of the run.
+__device__ __forceinline__ int xcd_remap_chunk(int w, int total, int chunk)
+{
+    const int first = w - w % chunk;
+    return first + chunk <= total ? first + xcd_remap(w - first, chunk) : w;
+}
+
 } // namespace m3p

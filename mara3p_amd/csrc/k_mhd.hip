@@ -4,17 +4,13 @@
 
 namespace m3p {
 
-// Cubes with N % 8 == 0 take the column-tile pass, whose face fluxes never
-// leave the workgroup; other N write them, [5][nf] per face family.
-static bool mhd_tiled(int N) { return N % 8 == 0 && N >= 8; }
-
 long mhd_workspace_bytes(int N, int precision)
 {
     const long N3 = (long)N * N * N, nf = (long)(N + 1) * N * N;
     const long rs = precision == M3P_FP64 ? 8 : 4;
-    // primitives [8][N^3], face fields [2][nf] per family, face fluxes (per-cell
-    // passes only), + alignment, the speed slots and dt
-    return (8 * N3 + 3 * 2 * nf + (mhd_tiled(N) ? 0 : 3 * 5 * nf)) * rs + 1024;
+    // primitives [8 N^3] and face fields [2][nf] per family, the primitive
+    // pass's speeds, dt, and the alignment of the first and the third
+    return (8 * N3 + 3 * 2 * nf) * rs + 8 * kMhdPrimGroups + 8 + 2 * 256;
 }
 
 template<typename R>
@@ -22,63 +18,48 @@ int mhd_advance(MhdArgs a, char* work, hipStream_t s)
 {
     const int N = a.N;
     const long N3 = (long)N * N * N, nf = (long)(N + 1) * N * N;
-    const bool tiled = mhd_tiled(N);
-    R* P = reinterpret_cast<R*>(work);
-    R* E1 = P + 8 * N3;
+    auto align = [] (char* p) { return p + ((256 - (reinterpret_cast<uintptr_t>(p) & 255)) & 255); };
+    auto P = reinterpret_cast<typename MhdPrim<R>::V*>(align(work));
+    R* E1 = reinterpret_cast<R*>(P) + 8 * N3;
     R* E2 = E1 + 2 * nf;
     R* E3 = E2 + 2 * nf;
-    R* F1 = E3 + 2 * nf;                     // per-cell passes only
-    R* F2 = F1 + 5 * nf;
-    R* F3 = F2 + 5 * nf;
-    char* tail = reinterpret_cast<char*>(tiled ? F1 : F3 + 5 * nf);
-    tail += (256 - (reinterpret_cast<uintptr_t>(tail) & 255)) & 255;
-    a.vmax = reinterpret_cast<unsigned long long*>(tail);
-    if (!a.dt) a.dt = reinterpret_cast<double*>(tail + 8 * kRateSlots);
+    a.vmax = reinterpret_cast<double*>(align(reinterpret_cast<char*>(E3 + 2 * nf)));
+    if (!a.dt) a.dt = a.vmax + kMhdPrimGroups;
     const int gc = (int)((N3 + 255) / 256);
-    hipLaunchKernelGGL(fill_u64_kernel, dim3(1), dim3(64), 0, s, a.vmax, kRateSlots, 0ull);
-    hipLaunchKernelGGL(mhd_prim_kernel<R>, dim3(std::min(gc, 4096)), dim3(256), 0, s, a, P);
-    hipLaunchKernelGGL(mhd_dt_kernel, dim3(1), dim3(kRateSlots), 0, s, a);
+    a.nvmax = std::min(gc, kMhdPrimGroups);
+    hipLaunchKernelGGL(mhd_prim_kernel<R>, dim3(a.nvmax), dim3(256), 0, s, a, P);
     FaceE<R> fe{ E1, E2, E3, N, nf };
-    if (tiled) {
-        // column tiles: fluxes and the conserved update in one pass, then the
-        // faces.  FP64 too (236 VGPRs at two waves per SIMD, no spills): at
-        // 256^3 its RK2 step takes 5.77 ms against 7.06 ms through the
-        // per-cell passes below, which write every face flux and read it back.
-        // 16-plane segments: 4096 workgroups at 256^3, four full rounds of
-        // the 1024 resident at four waves per SIMD (32-plane segments run
-        // as fast; 16 x 16 column tiles 10 % slower).  TI must divide N: an
-        // N with N % 16 == 8 takes 8-plane segments.
-        const int TI = N < 64 ? N : (N % 16 == 0 ? 16 : 8);
-        const int segs = N / TI;
+    // Column tiles of 8 x 32 columns: fluxes and the conserved update in one
+    // pass (16 x 16 tiles 0 to 10 % slower at 64 to 256, 8 x 8 tiles 20 to
+    // 40 %).  A workgroup marches TI planes after a warm-up of about one, so
+    // a cube that fills the device takes long segments (FP64, 16 planes:
+    // 4.36 ms a step at 256^3 against 4.45 with 8) and a small one as many
+    // workgroups as it can give (FP64 64^3: 98 us a step with 2 planes, 236
+    // with 16; mixed 100^3: 190 us with 8, 233 with 16).  Mixed keeps to 8
+    // planes (1.37 ms at 200^3 against 1.42 with 16, equal at 256^3).
+    auto tiles = [&] (auto kern) {
+        const int cols = ((N + 7) / 8) * ((N + 31) / 32);
+        const int groups = is_fp64<R>::value ? 640 : 768, cap = is_fp64<R>::value ? 16 : 8;
+        const int TI = (int)std::max(2l, std::min((long)cap, (long)N * cols / groups));
+        hipLaunchKernelGGL(kern, dim3(cols * ((N + TI - 1) / TI)), dim3(256), 0, s, a,
+                           (const typename MhdPrim<R>::V*)P, E1, E2, E3, TI);
+    };
+    if (N % 32 == 0) tiles(mhd_tile_kernel<R, 8, 32, false>);
+    else             tiles(mhd_tile_kernel<R, 8, 32, true>);
+    if (int st = launch_status("mhd_tile_kernel")) return st;
+    // The face fields: FP64 by bricks of 4 x 4 x 32 cells where they divide
+    // the cube (the step 4.41 ms at 256^3 against 4.71 per cell, 626 us
+    // against 672 at 128^3), else per cell (2.50 ms at 200^3 against 2.71 by
+    // bricks of 2 x 4 x 8); mixed per cell, where the FP32 face fields that
+    // the four faces of an edge re-read come from cache (bricks 0.5 % slower).
+    if constexpr (is_fp64<R>::value) {
         if (N % 32 == 0) {
-            const int grid = (N / 8) * (N / 32) * segs;
-            hipLaunchKernelGGL((mhd_tile_kernel<R, 8, 32>), dim3(grid), dim3(256), 0, s, a, (const R*)P, E1, E2, E3, TI);
-        } else {
-            const int grid = (N / 8) * (N / 8) * segs;
-            hipLaunchKernelGGL((mhd_tile_kernel<R, 8, 8>), dim3(grid), dim3(64), 0, s, a, (const R*)P, E1, E2, E3, TI);
+            hipLaunchKernelGGL((mhd_face_b_brick_kernel<R, 4, 4, 32>), dim3((N / 4) * (N / 4) * (N / 32)), dim3(512),
+                               0, s, a, fe);
+            return launch_status("m3p_mhd_advance_ct");
         }
-        if (int st = launch_status("mhd_tile_kernel")) return st;
-        // The face fields: FP64 by bricks of 4 x 4 x 32 cells, each edge field
-        // loaded once per brick (at 256^3 the FP64 RK2 step 5.60 -> 5.31 ms;
-        // bricks of 2 x 4 x 32: 5.34 ms); mixed per cell, where the FP32 face
-        // fields that the four faces of an edge re-read come from cache and
-        // the bricks ran 0.8 % slower.
-        if constexpr (is_fp64<R>::value) {
-            if (N % 32 == 0)
-                hipLaunchKernelGGL((mhd_face_b_brick_kernel<R, 4, 4, 32>), dim3((N / 4) * (N / 4) * (N / 32)), dim3(512),
-                                   0, s, a, fe);
-            else
-                hipLaunchKernelGGL((mhd_face_b_brick_kernel<R, 2, 4, 8>), dim3((N / 2) * (N / 4) * (N / 8)), dim3(64), 0,
-                                   s, a, fe);
-        } else {
-            hipLaunchKernelGGL(mhd_face_b_kernel<R>, dim3(gc), dim3(256), 0, s, a, fe);
-        }
-        return launch_status("m3p_mhd_advance_ct");
     }
-    hipLaunchKernelGGL(mhd_faces_kernel<R>, dim3(gc), dim3(256), 0, s, a, (const R*)P, F1, E1, F2, E2, F3, E3);
-    hipLaunchKernelGGL(mhd_boundary_faces_kernel<R>, dim3((int)((3L * N * N + 255) / 256)), dim3(256), 0, s, a,
-                       (const R*)P, F1, E1, F2, E2, F3, E3);
-    hipLaunchKernelGGL(mhd_update_kernel<R>, dim3(gc), dim3(256), 0, s, a, (const R*)F1, (const R*)F2, (const R*)F3, fe);
+    hipLaunchKernelGGL(mhd_face_b_kernel<R>, dim3(gc), dim3(256), 0, s, a, fe);
     return launch_status("m3p_mhd_advance_ct");
 }
 

@@ -4,22 +4,27 @@
 //   1. mhd_prim_kernel     cell primitives from U and the face-averaged B
 //                          (primitive_array :214-224, face_to_cell
 //                          src/mesh_cartesian_3d.hpp:235-245) + CFL max speed
-//   2. mhd_faces_kernel    PLM face states, HLLE Godunov flux and face electric
-//                          field of the three faces below each cell (and
-//                          mhd_boundary_faces_kernel for the upper planes)
-//                          (godunov_fluxes_plm :152-179,
-//                          mhd::riemann_hlle src/physics_mhd.hpp:358-390)
-//   3. mhd_update_kernel   U - div(F) dt / dl (divergence_difference
-//                          src/mesh_cartesian_3d.hpp:290-301) and, for the
-//                          faces below each cell, B_f - curl(E) dt / dl with
-//                          edge EMFs averaged from the faces
-//                          (edge_emf_from_face :76-98, solenoidal_difference
-//                          src/mesh_cartesian_3d.hpp:265-276)
+//   2. mhd_tile_kernel     PLM face states, HLLE Godunov flux and face electric
+//                          field of every face (godunov_fluxes_plm :152-179,
+//                          mhd::riemann_hlle src/physics_mhd.hpp:358-390), then
+//                          U - div(F) dt / dl (divergence_difference
+//                          src/mesh_cartesian_3d.hpp:290-301)
+//   3. mhd_face_b_kernel   B_f - curl(E) dt / dl with edge EMFs averaged from
+//                          the faces (edge_emf_from_face :76-98,
+//                          solenoidal_difference src/mesh_cartesian_3d.hpp:265-276)
 //
 // Layouts (row-major, last axis fastest, as the reference arrays):
 //   U [5][N][N][N];  B1 [N+1][N][N], B2 [N][N+1][N], B3 [N][N][N+1]
-//   workspace: P [8][N^3], face fluxes F_A [5][nf], face fields E_A [2][nf]
-//   (nf = (N+1) N^2, the transverse E components of axis-A faces).
+//   workspace: P [8 / W][N^3] vectors of W values (MhdPrim), face fields
+//   E_A [2][nf] (nf = (N+1) N^2, the transverse E components of axis-A faces).
+//
+// At 256^3 the mixed passes are bound by HBM: 5.2 to 5.5 TB/s of traffic each
+// (a large copy reaches 5.1), so what they fetch twice is what they lose.
+// Workgroups that share cache lines run on one XCD: each pass advances through
+// the planes in order, every XCD on its own rows of the plane (the primitive
+// pass fetches 1.24 GB, 1.35 in launch order; the face pass 1.02, was 1.44),
+// and the tile pass gives an XCD whole rows of tiles (2.48 GB a stage, was
+// 2.67 with an XCD per strip of 32 cells along k; the RK2 step 2.76 to 2.62 ms).
 #pragma once
 #include "device_common.hpp"
 
@@ -244,31 +249,78 @@ struct MhdArgs {
     double rk_b;
     int N;
     double dl, cfl, theta, gamma;
-    double* dt;                      // device: CFL time step of this call (written by mhd_dt_kernel)
-    unsigned long long* vmax;        // device: kRateSlots partial maxima of the fastest speed (ordered bits)
+    double* dt;                      // device: CFL time step of this call (written by the flux pass)
+    double* vmax;                    // device: the fastest speed of each primitive-pass workgroup
+    int nvmax;
     int* err;
 };
 
 __device__ __forceinline__ int wrapi(int i, int N) { return i < 0 ? i + N : (i >= N ? i - N : i); }
 
-// Grid-stride over cells with a bounded grid, so the speed reduction ends in
-// one atomic per workgroup of a few thousand, spread over kRateSlots slots.
+// (i, j, k) of cell c: 32-bit divisions while N^3 < 2^31
+__device__ __forceinline__ void cell_index(long c, int N, int& i, int& j, int& k)
+{
+    if (N <= 1290) {
+        const unsigned u = (unsigned)c, ij = u / (unsigned)N;
+        k = (int)(u - ij * (unsigned)N);
+        i = (int)(ij / (unsigned)N);
+        j = (int)(ij - (unsigned)i * (unsigned)N);
+    } else {
+        i = (int)(c / ((long)N * N)); j = (int)(c / N % N); k = (int)(c % N);
+    }
+}
+
+// 256-cell workgroups of about one plane, a multiple of 8 (xcd_remap_chunk)
+__device__ __forceinline__ int mhd_plane_groups(int N)
+{
+    return (int)(((long)N * N + 2047) / 2048) * 8;
+}
+
+// Primitives in the workspace: the eight values of a cell as 16-byte vectors,
+// vector v of all cells after vector v - 1 (P[v N^3 + cell]).  A wave's load
+// of one vector is contiguous, and the two halo cells at each end of a tile
+// row cost one or two more cache lines per vector instead of per component.
+template<typename R>
+struct MhdPrim {
+    static constexpr int W = 16 / sizeof(R);       // values of a vector
+    static constexpr int NV = 8 / W;
+    typedef R V __attribute__((ext_vector_type(16 / sizeof(R))));
+    __device__ static __forceinline__ void unpack(const V* x, R* p)
+    {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) p[q] = x[q / W][q % W];
+    }
+    __device__ static __forceinline__ void pack(const R* p, V* x)
+    {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) x[q / W][q % W] = p[q];
+    }
+    __device__ static __forceinline__ void store(V* P, long N3, long c, const R* p)
+    {
+        V x[NV];
+        pack(p, x);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) P[v * N3 + c] = x[v];
+    }
+};
+
+// Grid-stride over cells with a bounded grid: each workgroup leaves its
+// fastest speed in a slot of its own, which every workgroup of the flux pass
+// reduces for itself (no slots to clear, no launch for the time step).
+constexpr int kMhdPrimGroups = 2048;
+
 template<typename R>
 __global__ void __launch_bounds__(256)
-mhd_prim_kernel(MhdArgs a, R* P)
+mhd_prim_kernel(MhdArgs a, typename MhdPrim<R>::V* P)
 {
     const int N = a.N;
     const long N3 = (long)N * N * N;
     const long NN = (long)N * N;
     double s = 0.0;
-    // FP64: each XCD sweeps a contiguous range of the grid's cells, so the
-    // face fields that neighbouring rows and planes share stay in its L2
-    // (step 0.9 % faster at 256^3).  Mixed keeps the hardware order, which
-    // writes the top planes last for the tile pass that starts there (the
-    // remap made its step 1.1 % slower).
-    const long w = is_fp64<R>::value ? xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
+    const long w = xcd_remap_chunk(blockIdx.x, gridDim.x, mhd_plane_groups(N));
     for (long c = w * blockDim.x + threadIdx.x; c < N3; c += (long)gridDim.x * blockDim.x) {
-        const int i = (int)(c / NN), j = (int)(c / N % N), k = (int)(c % N);
+        int i, j, k;
+        cell_index(c, N, i, j, k);
         double b[3] = { 0.5 * (a.b1[(long)i * NN + (long)j * N + k] + a.b1[(long)(i + 1) * NN + (long)j * N + k]),
                         0.5 * (a.b2[((long)i * (N + 1) + j) * N + k] + a.b2[((long)i * (N + 1) + j + 1) * N + k]),
                         0.5 * (a.b3[((long)i * N + j) * (N + 1) + k] + a.b3[((long)i * N + j) * (N + 1) + k + 1]) };
@@ -278,8 +330,7 @@ mhd_prim_kernel(MhdArgs a, R* P)
         if constexpr (is_fp64<R>::value) {
             int st = mhd_recover<true>(u, b, a.gamma, p);
             if (st) report_error(a.err, st == 1 ? 1 : 2, 0, (int)c);
-#pragma unroll
-            for (int q = 0; q < 8; ++q) P[q * N3 + c] = p[q];
+            MhdPrim<R>::store(P, N3, c, p);
             s = fmax(s, mhd_fastest_speed(p, a.gamma));
         } else {
             // mixed: the pressure difference in FP64 (one reciprocal of the
@@ -292,8 +343,7 @@ mhd_prim_kernel(MhdArgs a, R* P)
             if (d < 0.0) report_error(a.err, 1, 0, (int)c);
             else if (pg < 0.0) report_error(a.err, 2, 0, (int)c);
             R pf[8] = { R(d), R(u[1] * id), R(u[2] * id), R(u[3] * id), R(pg), R(b[0]), R(b[1]), R(b[2]) };
-#pragma unroll
-            for (int q = 0; q < 8; ++q) P[q * N3 + c] = pf[q];
+            MhdPrim<R>::store(P, N3, c, pf);
             R m1, q1, m2, q2, m3, q3;
             const R gf = R(a.gamma);
             Mhd<R>::template wavespeeds<1>(pf, gf, m1, q1);
@@ -303,23 +353,13 @@ mhd_prim_kernel(MhdArgs a, R* P)
             s = fmax(s, double(v));
         }
     }
-    workgroup_atomic_max<256>(s, a.vmax);
+    __shared__ double part[4];
+    s = wave_max(s);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) a.vmax[blockIdx.x] = fmax(fmax(part[0], part[1]), fmax(part[2], part[3]));
 }
 
-// dt from the kRateSlots partial maxima (one wave)
-static __global__ void __launch_bounds__(64) mhd_dt_kernel(MhdArgs a)
-{
-    double vmax = wave_max(__longlong_as_double((long long)a.vmax[threadIdx.x]));
-    if (threadIdx.x == 0) *a.dt = a.cfl * a.dl / vmax;
-}
-
-// All three face families in one pass: the thread of cell (i, j, k)
-// computes the lower face of the cell on each axis (the x face at i, the y
-// face at j, the z face at k), and the cells on the last plane of an axis
-// also compute the face at N (periodic: the same cells as face 0).  The
-// primitive stencils of the three axes share the cell's neighbourhood, so
-// the primitives are read once from cache instead of once per axis.  Each
-// face's stencil: cells (m-2, m-1, m, m+1) along the axis for face m, wrapped.
 // Half the PLM slope of the middle value: the reference's 0.5 * plm_gradient
 // in FP64, the three-operand median form in FP32 (the same value).
 template<typename R>
@@ -329,128 +369,92 @@ __device__ __forceinline__ R mhd_half_slope(R c0, R c1, R c2, R theta)
     else return plm_half(c0, c1, c2, theta);
 }
 
-template<typename R, int A>
-__device__ __forceinline__ void mhd_one_face(const MhdArgs& a, const R* P, R* F, R* E, int i, int j, int k)
-{
-    const int N = a.N;
-    const long N3 = (long)N * N * N;
-    const long nf = (long)(N + 1) * N * N;
-    long f;
-    if (A == 1)      f = ((long)i * N + j) * N + k;
-    else if (A == 2) f = ((long)i * (N + 1) + j) * N + k;
-    else             f = ((long)i * N + j) * (N + 1) + k;
-    long cell[4];
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-        const int o = s - 2;
-        int ci = i, cj = j, ck = k;
-        if (A == 1) ci = wrapi(i + o, N);
-        if (A == 2) cj = wrapi(j + o, N);
-        if (A == 3) ck = wrapi(k + o, N);
-        cell[s] = ((long)ci * N + cj) * N + ck;
-    }
-    const R theta = R(a.theta);
-    R pl[8], pr[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-        R c0 = P[q * N3 + cell[0]], c1 = P[q * N3 + cell[1]], c2 = P[q * N3 + cell[2]], c3 = P[q * N3 + cell[3]];
-        pl[q] = c1 + mhd_half_slope(c0, c1, c2, theta);
-        pr[q] = c2 - mhd_half_slope(c1, c2, c3, theta);
-    }
-    const double* bf = A == 1 ? a.b1 : (A == 2 ? a.b2 : a.b3);
-    R fl[5], e[3];
-    Mhd<R>::template riemann<A>(pl, pr, R(bf[f]), R(a.gamma), fl, e);
-#pragma unroll
-    for (int q = 0; q < 5; ++q) F[q * nf + f] = fl[q];
-    E[f] = e[A == 1 ? 1 : 0];
-    E[nf + f] = e[A == 3 ? 1 : 2];
-}
-
-template<typename R>
-__global__ void __launch_bounds__(256)
-mhd_faces_kernel(MhdArgs a, const R* P, R* F1, R* E1, R* F2, R* E2, R* F3, R* E3)
-{
-    const int N = a.N;
-    const long N3 = (long)N * N * N;
-    const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= N3) return;
-    const int i = (int)(c / ((long)N * N)), j = (int)(c / N % N), k = (int)(c % N);
-    mhd_one_face<R, 1>(a, P, F1, E1, i, j, k);
-    mhd_one_face<R, 2>(a, P, F2, E2, i, j, k);
-    mhd_one_face<R, 3>(a, P, F3, E3, i, j, k);
-}
-
-// The faces on the upper boundary planes (i = N, j = N, k = N), one per
-// thread: 3 N^2 faces.  In the per-cell pass the cells next to them would
-// run a fourth, nearly empty face pass (a quarter of all waves, for k = N).
-template<typename R>
-__global__ void __launch_bounds__(256)
-mhd_boundary_faces_kernel(MhdArgs a, const R* P, R* F1, R* E1, R* F2, R* E2, R* F3, R* E3)
-{
-    const int N = a.N;
-    const long NN = (long)N * N;
-    const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= 3 * NN) return;
-    const int axis = (int)(c / NN);
-    const int u = (int)(c % NN / N), v = (int)(c % N);
-    if (axis == 0)      mhd_one_face<R, 1>(a, P, F1, E1, N, u, v);
-    else if (axis == 1) mhd_one_face<R, 2>(a, P, F2, E2, u, N, v);
-    else                mhd_one_face<R, 3>(a, P, F3, E3, u, v, N);
-}
-
-// Column-tile form of the flux pass fused with the conserved update.  A
-// workgroup owns TJ x TK columns (j, k) and marches along i over TI planes
-// of one segment.  Each thread keeps a four-plane window of its column's
-// primitives, so the x face above its cell needs one new load per plane;
-// the y and z faces of the plane come from an LDS copy of the plane with a
-// two-cell halo.  Per plane and thread: the y and z faces below the cell
-// (the tile's upper y and z faces by the last row and by the first TJ
-// threads), the x face above it (after the y and z faces, so the next
-// plane's primitives it needs arrive meanwhile; FP64 needs 34 fewer
-// VGPRs, and the RK2 step at 256^3 is 0.5 % (mixed) and 0.9 % (FP64)
-// faster), then U of the cell from the six face fluxes
-// (divergence_difference, src/mesh_cartesian_3d.hpp:290-301).  Face fluxes
-// never leave the workgroup; the transverse face electric fields go to the
-// E arrays for the face update.  Every face is computed from the same
-// operands in the same order as mhd_one_face, so a face shared by two
-// tiles or segments has one value.
+// The flux pass fused with the conserved
+// update, by column tiles.  A workgroup owns TJ x TK columns (j, k) and
+// marches along i over TI planes of one segment.  Each thread keeps a
+// four-plane window of its column's primitives, so the x face above its cell
+// needs one new load per plane; the y and z faces of the plane come from an
+// LDS copy of the plane with a two-cell halo, as 16-byte vectors like the
+// workspace (a quarter of the LDS instructions of single values).  Per plane
+// and thread: the y and z faces below the cell (the tile's upper y and z faces
+// by the last row and by the first TJ threads), the x face above it (after
+// the y and z faces, so the next plane's primitives it needs arrive
+// meanwhile; FP64 needs 34 fewer VGPRs, and the RK2 step at 256^3 is 0.5 %
+// (mixed) and 0.9 % (FP64) faster), then U of the cell from the six face
+// fluxes (divergence_difference, src/mesh_cartesian_3d.hpp:290-301).  Face
+// fluxes never leave the workgroup; the transverse face electric fields go to
+// the E arrays for the face update.  Every face is computed from the same
+// operands in the same order wherever it is computed, so a face shared by two
+// tiles or segments has one value.  RAGGED: the tiles do not divide the cube
+// (100^3 mixed: 200 us a step, 278 through passes per cell that wrote and
+// re-read every face flux).
 // Mixed: four waves per SIMD, where the register allocator fits the kernel
 // in 128 VGPRs without spills (150 when unconstrained, three waves) and the
 // extra wave hides load latency (11 % faster per RK2 step at 256^3).  FP64:
-// two waves per SIMD (up to 256 VGPRs), the update in the arithmetic and
-// order of mhd_update_kernel.
+// two waves per SIMD (up to 256 VGPRs), the update in the reference's
+// association order.
 template<typename R> struct MhdTileWaves { static constexpr int value = is_fp64<R>::value ? 2 : 4; };
 
-template<typename R, int TJ, int TK>
+template<typename R, int TJ, int TK, bool RAGGED>
 __global__ void __launch_bounds__(TJ * TK) __attribute__((amdgpu_waves_per_eu(MhdTileWaves<R>::value, 8)))
-mhd_tile_kernel(MhdArgs a, const R* P, R* E1, R* E2, R* E3, int TI)
+mhd_tile_kernel(MhdArgs a, const typename MhdPrim<R>::V* P, R* E1, R* E2, R* E3, int TI)
 {
     constexpr int NT = TJ * TK;
     constexpr int EJ = TJ + 4, EK = TK + 4;
+    using Vec = typename MhdPrim<R>::V;
+    constexpr int NV = MhdPrim<R>::NV;
     const int N = a.N;
     const long N3 = (long)N * N * N, nf = (long)(N + 1) * N * N;
-    const int tiles_k = N / TK, tiles_j = N / TJ;
-    int w = blockIdx.x;
-    const int k0 = (w % tiles_k) * TK; w /= tiles_k;
-    const int j0 = (w % tiles_j) * TJ; w /= tiles_j;
+    const int tiles_k = RAGGED ? (N + TK - 1) / TK : N / TK, tiles_j = RAGGED ? (N + TJ - 1) / TJ : N / TJ;
+    const int cols = tiles_k * tiles_j;
+    const int col = xcd_remap(blockIdx.x % cols, cols), w = blockIdx.x / cols;
+    const int k0 = (col % tiles_k) * TK, j0 = (col / tiles_k) * TJ;
     // segments from the top plane down: the primitive pass wrote the high
     // planes last, so they are the likeliest to still be cached
-    const int i0 = (N / TI - 1 - w) * TI;
+    const int i0 = ((N + TI - 1) / TI - 1 - w) * TI;
+    const int ni = min(TI, N - i0);
     const int t = threadIdx.x, jl = t / TK, kl = t % TK;
     const int j = j0 + jl, k = k0 + kl;
+    // A ragged tile reaches past the cube: its lanes there load from the
+    // nearest index inside (jc, kc for cells, clamped face indices below) and
+    // store nothing; the first row and column of them compute the upper
+    // boundary faces, which are the cube's.
+    const int jc = RAGGED ? min(j, N - 1) : j, kc = RAGGED ? min(k, N - 1) : k;
+    const bool in_j = !RAGGED || j < N, in_k = !RAGGED || k < N;
 
-    __shared__ R Pl[8][EJ][EK];       // primitives of plane i, (j0 - 2 .. j0 + TJ + 1) x (k0 - 2 .. k0 + TK + 1)
+    __shared__ Vec Pl[NV][EJ][EK];    // primitives of plane i, (j0 - 2 .. j0 + TJ + 1) x (k0 - 2 .. k0 + TK + 1)
     __shared__ R F2s[5][TJ + 1][TK];  // y-face fluxes of plane i, faces j0 .. j0 + TJ
     __shared__ R F3s[5][TJ][TK + 1];  // z-face fluxes of plane i, faces k0 .. k0 + TK
 
-    const double dt = *a.dt;
+    __shared__ double vpart[NT / 64];  // fastest speed, by wave
+    {
+        double v = 0.0;
+        for (int r = t; r < a.nvmax; r += NT) v = fmax(v, a.vmax[r]);
+        v = wave_max(v);
+        if ((t & 63) == 0) vpart[t >> 6] = v;
+    }
     const R theta = R(a.theta), gamma = R(a.gamma);
     auto cell = [&] (int ii, int jj, int kk) {
+        if (RAGGED) { jj = min(jj, N + 1); kk = min(kk, N + 1); }
         return ((long)wrapi(ii, N) * N + wrapi(jj, N)) * N + wrapi(kk, N);
     };
     auto loadP = [&] (long c, R* p) {
+        Vec x[NV];
 #pragma unroll
-        for (int q = 0; q < 8; ++q) p[q] = P[q * N3 + c];
+        for (int v = 0; v < NV; ++v) x[v] = P[v * N3 + c];
+        MhdPrim<R>::unpack(x, p);
+    };
+    auto putP = [&] (int rj, int rk, const R* p) {
+        Vec x[NV];
+        MhdPrim<R>::pack(p, x);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) Pl[v][rj][rk] = x[v];
+    };
+    auto getP = [&] (int rj, int rk, R* p) {
+        Vec x[NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) x[v] = Pl[v][rj][rk];
+        MhdPrim<R>::unpack(x, p);
     };
     // face states from four cells along the face normal (lower two, upper two)
     auto states = [&] (const R* c0, const R* c1, const R* c2, const R* c3, R* pl, R* pr) {
@@ -477,10 +481,16 @@ mhd_tile_kernel(MhdArgs a, const R* P, R* E1, R* E2, R* E3, int TI)
             pl[q] = Pm[q] + mhd_half_slope(Pm2[q], Pm[q], P0[q], theta);
             pr[q] = P0[q] - g0[q];
         }
-        const long f = ((long)i0 * N + j) * N + k;
+        const long f = ((long)i0 * N + jc) * N + kc;
         Mhd<R>::template riemann<1>(pl, pr, R(a.b1[f]), gamma, Fx_lo, e);
-        if (i0 == 0) { E1[f] = e[1]; E1[nf + f] = e[2]; }
+        if (i0 == 0 && in_j && in_k) { E1[f] = e[1]; E1[nf + f] = e[2]; }
     }
+    __syncthreads();
+    double vmax = vpart[0];
+#pragma unroll
+    for (int r = 1; r < NT / 64; ++r) vmax = fmax(vmax, vpart[r]);
+    const double dt = a.cfl * a.dl / vmax;
+    if (blockIdx.x == 0 && t == 0) *a.dt = dt;
     const double dtdl = dt / a.dl;
 
     // The plane's two-cell halo ring (NH cells): position of ring cell r.
@@ -508,27 +518,25 @@ mhd_tile_kernel(MhdArgs a, const R* P, R* E1, R* E2, R* E3, int TI)
         }
     }
 
-    for (int il = 0; il < TI; ++il) {
+    for (int il = 0; il < ni; ++il) {
         const int i = i0 + il;
         R Pn[8];
         loadP(cell(i + 2, j, k), Pn);
 
         // LDS plane i: interior from the window, halo ring from memory
-#pragma unroll
-        for (int q = 0; q < 8; ++q) Pl[q][jl + 2][kl + 2] = P0[q];
+        putP(jl + 2, kl + 2, P0);
         if constexpr (kRingAhead) {
             if (t < NH) {
-#pragma unroll
-                for (int q = 0; q < 8; ++q) Pl[q][hj][hk] = Hn[q];
-                if (il + 1 < TI) loadP(cell(i + 1, j0 - 2 + hj, k0 - 2 + hk), Hn);
+                putP(hj, hk, Hn);
+                if (il + 1 < ni) loadP(cell(i + 1, j0 - 2 + hj, k0 - 2 + hk), Hn);
             }
         } else {
             for (int r = t; r < NH; r += NT) {
                 int rj, rk;
                 ring(r, rj, rk);
-                const long c = cell(i, j0 - 2 + rj, k0 - 2 + rk);
-#pragma unroll
-                for (int q = 0; q < 8; ++q) Pl[q][rj][rk] = P[q * N3 + c];
+                R h[8];
+                loadP(cell(i, j0 - 2 + rj, k0 - 2 + rk), h);
+                putP(rj, rk, h);
             }
         }
         // FP64: the longitudinal fields of the cell's own y and z faces are
@@ -538,28 +546,25 @@ mhd_tile_kernel(MhdArgs a, const R* P, R* E1, R* E2, R* E3, int TI)
         constexpr bool kPreB = is_fp64<R>::value;
         // the x face's longitudinal field (its face follows the barrier), in
         // both precisions (FP64 step 1.0 % faster, mixed unchanged)
-        const R blx = R(a.b1[((long)(i + 1) * N + j) * N + k]);
+        const R blx = R(a.b1[((long)(i + 1) * N + jc) * N + kc]);
         R bly = R(0), blz = R(0);
         if constexpr (kPreB) {
-            bly = R(a.b2[((long)i * (N + 1) + j) * N + k]);
-            blz = R(a.b3[((long)i * N + j) * (N + 1) + k]);
+            bly = R(a.b2[((long)i * (N + 1) + (RAGGED ? min(j, N) : j)) * N + kc]);
+            blz = R(a.b3[((long)i * N + jc) * (N + 1) + (RAGGED ? min(k, N) : k)]);
         }
         __syncthreads();
 
         // y face below the cell (face j), and the tile's upper y face by the last row
         auto yface = [&] (int jf /* local face row 0..TJ */, bool own) {
             R c0[8], c1[8], c2[8], c3[8], pl[8], pr[8], f[5], e[3];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                c0[q] = Pl[q][jf][kl + 2]; c1[q] = Pl[q][jf + 1][kl + 2];
-                c2[q] = Pl[q][jf + 2][kl + 2]; c3[q] = Pl[q][jf + 3][kl + 2];
-            }
+            getP(jf, kl + 2, c0); getP(jf + 1, kl + 2, c1);
+            getP(jf + 2, kl + 2, c2); getP(jf + 3, kl + 2, c3);
             states(c0, c1, c2, c3, pl, pr);
-            const long fi = ((long)i * (N + 1) + (j0 + jf)) * N + k;
+            const long fi = ((long)i * (N + 1) + (RAGGED ? min(j0 + jf, N) : j0 + jf)) * N + kc;
             Mhd<R>::template riemann<2>(pl, pr, kPreB && own ? bly : R(a.b2[fi]), gamma, f, e);
 #pragma unroll
             for (int q = 0; q < 5; ++q) F2s[q][jf][kl] = f[q];
-            if (jf < TJ || j0 + jf == N) { E2[fi] = e[0]; E2[nf + fi] = e[2]; }
+            if ((jf < TJ || j0 + jf == N) && in_k && (!RAGGED || j0 + jf <= N)) { E2[fi] = e[0]; E2[nf + fi] = e[2]; }
         };
         yface(jl, true);
         if (jl == TJ - 1) yface(TJ, false);
@@ -567,17 +572,15 @@ mhd_tile_kernel(MhdArgs a, const R* P, R* E1, R* E2, R* E3, int TI)
         // z face below the cell (face k), and the tile's upper z faces by threads 0 .. TJ-1
         auto zface = [&] (int row, int kf /* local face column 0..TK */, bool own) {
             R c0[8], c1[8], c2[8], c3[8], pl[8], pr[8], f[5], e[3];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                c0[q] = Pl[q][row + 2][kf]; c1[q] = Pl[q][row + 2][kf + 1];
-                c2[q] = Pl[q][row + 2][kf + 2]; c3[q] = Pl[q][row + 2][kf + 3];
-            }
+            getP(row + 2, kf, c0); getP(row + 2, kf + 1, c1);
+            getP(row + 2, kf + 2, c2); getP(row + 2, kf + 3, c3);
             states(c0, c1, c2, c3, pl, pr);
-            const long fi = ((long)i * N + (j0 + row)) * (N + 1) + (k0 + kf);
+            const long fi = ((long)i * N + (RAGGED ? min(j0 + row, N - 1) : j0 + row)) * (N + 1)
+                          + (RAGGED ? min(k0 + kf, N) : k0 + kf);
             Mhd<R>::template riemann<3>(pl, pr, kPreB && own ? blz : R(a.b3[fi]), gamma, f, e);
 #pragma unroll
             for (int q = 0; q < 5; ++q) F3s[q][row][kf] = f[q];
-            if (kf < TK || k0 + kf == N) { E3[fi] = e[0]; E3[nf + fi] = e[1]; }
+            if ((kf < TK || k0 + kf == N) && (!RAGGED || (j0 + row < N && k0 + kf <= N))) { E3[fi] = e[0]; E3[nf + fi] = e[1]; }
         };
         zface(jl, kl, true);
         if (t < TJ) zface(t, TK, false);
@@ -592,10 +595,9 @@ mhd_tile_kernel(MhdArgs a, const R* P, R* E1, R* E2, R* E3, int TI)
                 pr[q] = Pp[q] - gp;
                 g0[q] = gp;
             }
-            const long f = ((long)(i + 1) * N + j) * N + k;
+            const long f = ((long)(i + 1) * N + jc) * N + kc;
             Mhd<R>::template riemann<1>(pl, pr, blx, gamma, Fx_hi, e);
-            E1[f] = e[1];
-            E1[nf + f] = e[2];
+            if (in_j && in_k) { E1[f] = e[1]; E1[nf + f] = e[2]; }
         }
         // the update's U and RK base, loaded before the barrier (which
         // orders memory, so the compiler keeps loads written after it there)
@@ -603,7 +605,7 @@ mhd_tile_kernel(MhdArgs a, const R* P, R* E1, R* E2, R* E3, int TI)
         // faster mixed, 11.6 % FP64
         double ucv[5], u0v[5] = {};
         {
-            const long c = ((long)i * N + j) * N + k;
+            const long c = ((long)i * N + jc) * N + kc;
 #pragma unroll
             for (int q = 0; q < 5; ++q) ucv[q] = a.uc[q * N3 + c];
             if (a.u0) {
@@ -614,7 +616,7 @@ mhd_tile_kernel(MhdArgs a, const R* P, R* E1, R* E2, R* E3, int TI)
         __syncthreads();
 
         // conserved update of cell (i, j, k)
-        {
+        if (in_j && in_k) {
             const long c = ((long)i * N + j) * N + k;
 #pragma unroll
             for (int q = 0; q < 5; ++q) {
@@ -686,10 +688,6 @@ struct FaceE {
     }
 };
 
-// One pass for the whole update: the thread of cell (i, j, k) updates the
-// cell's conserved state and the lower face of the cell on each axis (plus
-// the faces at N on the last planes), with the arithmetic of
-// mhd_cell_update_kernel and mhd_face_update_kernel<R, A>.
 template<typename R, int A>
 __device__ __forceinline__ void mhd_update_face(const MhdArgs& a, const FaceE<R>& fe, double dt, int i, int j, int k)
 {
@@ -718,38 +716,8 @@ __device__ __forceinline__ void mhd_update_face(const MhdArgs& a, const FaceE<R>
     out[f] = r;
 }
 
-template<typename R>
-__global__ void __launch_bounds__(256)
-mhd_update_kernel(MhdArgs a, const R* F1, const R* F2, const R* F3, FaceE<R> fe)
-{
-    const int N = a.N;
-    const long N3 = (long)N * N * N, nf = (long)(N + 1) * N * N;
-    const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= N3) return;
-    const int i = (int)(c / ((long)N * N)), j = (int)(c / N % N), k = (int)(c % N);
-    const double dt = *a.dt;
-    const long x0 = ((long)i * N + j) * N + k, x1 = x0 + (long)N * N;
-    const long y0 = ((long)i * (N + 1) + j) * N + k, y1 = y0 + N;
-    const long z0 = ((long)i * N + j) * (N + 1) + k, z1 = z0 + 1;
-#pragma unroll
-    for (int q = 0; q < 5; ++q) {
-        double d1 = double(F1[q * nf + x1]) - double(F1[q * nf + x0]);
-        double d2 = double(F2[q * nf + y1]) - double(F2[q * nf + y0]);
-        double d3 = double(F3[q * nf + z1]) - double(F3[q * nf + z0]);
-        double r = a.uc[q * N3 + c] - (d1 + d2 + d3) * (dt / a.dl);
-        if (a.u0) r = a.u0[q * N3 + c] * a.rk_b + r * (1.0 - a.rk_b);
-        a.uo[q * N3 + c] = r;
-    }
-    mhd_update_face<R, 1>(a, fe, dt, i, j, k);
-    mhd_update_face<R, 2>(a, fe, dt, i, j, k);
-    mhd_update_face<R, 3>(a, fe, dt, i, j, k);
-    if (i == N - 1) mhd_update_face<R, 1>(a, fe, dt, N, j, k);
-    if (j == N - 1) mhd_update_face<R, 2>(a, fe, dt, i, N, k);
-    if (k == N - 1) mhd_update_face<R, 3>(a, fe, dt, i, j, N);
-}
-
-// The face part of mhd_update_kernel alone (the conserved update is done by
-// mhd_tile_kernel).
+// The face-field update per cell: the three faces below it (and the faces at
+// N on the last planes).
 template<typename R>
 __global__ void __launch_bounds__(256)
 mhd_face_b_kernel(MhdArgs a, FaceE<R> fe)
@@ -757,9 +725,10 @@ mhd_face_b_kernel(MhdArgs a, FaceE<R> fe)
     const int N = a.N;
     const long N3 = (long)N * N * N;
     // cells from the bottom up: the tile pass wrote the low planes last
-    const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long c = (long)xcd_remap_chunk(blockIdx.x, gridDim.x, mhd_plane_groups(N)) * blockDim.x + threadIdx.x;
     if (c >= N3) return;
-    const int i = (int)(c / ((long)N * N)), j = (int)(c / N % N), k = (int)(c % N);
+    int i, j, k;
+    cell_index(c, N, i, j, k);
     const double dt = *a.dt;
     mhd_update_face<R, 1>(a, fe, dt, i, j, k);
     mhd_update_face<R, 2>(a, fe, dt, i, j, k);
@@ -791,10 +760,10 @@ mhd_face_b_brick_kernel(MhdArgs a, FaceE<R> fe)
     __shared__ double Y2[BI + 1][BJ][BK + 1];           // ee2(i0 + p, j0 + r, k0 + c)
     __shared__ double Z3[BI + 1][BJ + 1][BK];           // ee3(i0 + p, j0 + r, k0 + c)
     const int N = a.N;
-    int w = blockIdx.x;
-    const int k0 = (w % (N / BK)) * BK; w /= N / BK;
-    const int j0 = (w % (N / BJ)) * BJ; w /= N / BJ;
-    const int i0 = w * BI;
+    const int cols = (N / BK) * (N / BJ);
+    const int col = xcd_remap(blockIdx.x % cols, cols);
+    const int k0 = (col % (N / BK)) * BK, j0 = (col / (N / BK)) * BJ;
+    const int i0 = (int)(blockIdx.x / cols) * BI;
     const int t = threadIdx.x;
     const int il = t / (BJ * BK), jl = t / BK % BJ, kl = t % BK;
     const int i = i0 + il, j = j0 + jl, k = k0 + kl;
@@ -858,7 +827,8 @@ mhd_divb_kernel(const double* b1, const double* b2, const double* b3, int N, uns
     const long NN = (long)N * N;
     double v = 0.0;
     for (long c = (long)blockIdx.x * blockDim.x + threadIdx.x; c < N3; c += (long)gridDim.x * blockDim.x) {
-        const int i = (int)(c / NN), j = (int)(c / N % N), k = (int)(c % N);
+        int i, j, k;
+        cell_index(c, N, i, j, k);
         double d1 = b1[(long)(i + 1) * NN + (long)j * N + k] - b1[(long)i * NN + (long)j * N + k];
         double d2 = b2[((long)i * (N + 1) + j + 1) * N + k] - b2[((long)i * (N + 1) + j) * N + k];
         double d3 = b3[((long)i * N + j) * (N + 1) + k + 1] - b3[((long)i * N + j) * (N + 1) + k];

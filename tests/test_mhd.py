@@ -135,6 +135,30 @@ def test_gpu_mhd_advance_ct_fp64_matches_oracle(N):
 
 @pytest.mark.gpu
 @gpu
+@pytest.mark.parametrize("N", [2, 3, 7, 9, 31, 33, 50, 65])
+def test_gpu_mhd_ragged_tiles(N):
+    """Cubes that the 8 x 32 column tiles do not divide: smaller than a tile,
+    one cell more or less than whole tiles, and a short last segment.  FP64
+    against the oracle at the bar of the other sizes; mixed against FP64 at
+    the bar of test_gpu_mhd_mixed_tracks_fp64."""
+    from mara3p_amd.problems import orszag_tang_3d
+    from mara3p_amd.solvers import MhdSolver
+    state = orszag_tang_3d(N, seed=6, perturbation=0.05)
+    a, b = MhdSolver(N), MhdSolver(N, precision="mixed")
+    for s in (a, b):
+        s.set_state(*state)
+        s.step()
+        s.step()
+        s.check_errors()
+    ref = _oracle_rk2(N, *state, 2)
+    for x, y, z in zip(a.state(), b.state(), ref[:4]):
+        assert _rel(x, z) <= 1e-12
+        assert _rel(y, x) <= 1e-5
+    assert np.allclose(a.dts.cpu().numpy(), ref[4][-1], rtol=1e-13)
+
+
+@pytest.mark.gpu
+@gpu
 def test_gpu_mhd_div_b_and_mixed():
     """Orszag-Tang at 32^3 for 10 steps: CT keeps max |div B| at round-off in both
     kernels; the mixed kernel's energy stays within 1e-4 (L1, relative) of FP64."""
