@@ -34,7 +34,8 @@ template<typename R>
 struct Mhd {
     __device__ static __forceinline__ R dot3(const R* a, const R* b)
     {
-        if constexpr (is_fp64<R>::value) return ((R(0) + a[0] * b[0]) + a[1] * b[1]) + a[2] * b[2];
+        // FP64: the reference's order, without its sum's leading zero
+        if constexpr (is_fp64<R>::value) return (a[0] * b[0] + a[1] * b[1]) + a[2] * b[2];
         else return fmaf(a[2], b[2], fmaf(a[1], b[1], a[0] * b[0]));
     }
 
@@ -48,7 +49,8 @@ struct Mhd {
         u[1] = d * v[0];
         u[2] = d * v[1];
         u[3] = d * v[2];
-        if constexpr (is_fp64<R>::value) u[4] = R(0.5) * d * dot3(v, v) + p[4] / (gamma - R(1)) + R(0.5) * dot3(b, b);
+        if constexpr (is_fp64<R>::value)
+            u[4] = R(0.5) * d * dot3(v, v) + Divisor<R>(gamma - R(1))(p[4]) + R(0.5) * dot3(b, b);
         else u[4] = fmaf(R(0.5) * d, dot3(v, v), fmaf(R(0.5), dot3(b, b), p[4] * frcp(gamma - R(1))));
     }
 
@@ -60,15 +62,18 @@ struct Mhd {
         const R* b = &p[5];
         constexpr int a = AXIS - 1;
         if constexpr (is_fp64<R>::value) {
-            R bn = R(0) + b[a];
-            R vn = R(0) + v[a];
+            // the reference's sums without the products with the zero
+            // components of the unit normal: the same values (a zero may
+            // differ in its sign) for every finite state, here and in the
+            // induction, the longitudinal field and the face electric field
+            // below
+            R bn = b[a];
+            R vn = v[a];
             R pt = p[4] + R(0.5) * dot3(b, b);
             R bv = dot3(b, v);
-            R n[3] = { R(AXIS == 1), R(AXIS == 2), R(AXIS == 3) };
-            f[0] = vn * u[0] + R(0) + R(0);
-            f[1] = vn * u[1] + pt * n[0] + -bn * b[0];
-            f[2] = vn * u[2] + pt * n[1] + -bn * b[1];
-            f[3] = vn * u[3] + pt * n[2] + -bn * b[2];
+            f[0] = vn * u[0];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) f[1 + k] = (k == a ? vn * u[1 + k] + pt : vn * u[1 + k]) + -bn * b[k];
             f[4] = vn * u[4] + pt * vn + -bn * bv;
         } else {
             R bn = b[a], vn = v[a];
@@ -88,22 +93,14 @@ struct Mhd {
     {
         const R* v = &p[1];
         const R* b = &p[5];
-        if constexpr (is_fp64<R>::value) {
-            R E[3] = { -(v[1] * b[2] - v[2] * b[1]), -(v[2] * b[0] - v[0] * b[2]), -(v[0] * b[1] - v[1] * b[0]) };
-            R n[3] = { R(AXIS == 1), R(AXIS == 2), R(AXIS == 3) };
-            out[0] = n[1] * E[2] - n[2] * E[1];
-            out[1] = n[2] * E[0] - n[0] * E[2];
-            out[2] = n[0] * E[1] - n[1] * E[0];
-        } else {
-            // n is the unit vector of axis a: n x E has no a component and
-            // its other two are -E_c and E_b (b, c the next axes in cyclic
-            // order), without the general form's products with the zero
-            // components of n (the same values up to the sign of a zero)
-            constexpr int a = AXIS - 1, bx = (a + 1) % 3, c = (a + 2) % 3;
-            out[a] = R(0);
-            out[bx] = v[a] * b[bx] - v[bx] * b[a];
-            out[c] = -(v[c] * b[a] - v[a] * b[c]);
-        }
+        // n is the unit vector of axis a: n x E has no a component and its
+        // other two are -E_c and E_b (b, c the next axes in cyclic order),
+        // without the general form's products with the zero components of n
+        // (the same values up to the sign of a zero)
+        constexpr int a = AXIS - 1, bx = (a + 1) % 3, c = (a + 2) % 3;
+        out[a] = R(0);
+        out[bx] = v[a] * b[bx] - v[bx] * b[a];
+        out[c] = -(v[c] * b[a] - v[a] * b[c]);
     }
 
     // outer_wavespeeds :216-246
@@ -118,12 +115,12 @@ struct Mhd {
             // bn * bn for pow(bn, 2), and the Newton-refined reciprocal and
             // square roots (each within a few ulp of the reference's
             // divisions, pow and sqrt)
-            R vn = R(0) + p[1 + a];
+            R vn = p[1 + a];
             const R id = rcp_nr(d);
             R cs2 = gamma * p[4] * id;
             R ca2 = dot3(b, b) * id;
             R cf2 = cs2 + ca2;
-            R bn = R(0) + b[a];
+            R bn = b[a];
             R can2 = (bn * bn) * id;
             R cg2 = sqrt_nr(cf2 * cf2 - R(4) * cs2 * can2);
             R cf = sqrt_nr(R(0.5) * (cf2 + cg2));
@@ -148,19 +145,10 @@ struct Mhd {
     __device__ static __forceinline__ void riemann(R* pl, R* pr, R bl, R gamma, R* f, R* e)
     {
         constexpr int a = AXIS - 1;
-        // with_longitudinal_field :165-176: (b - (b.n) n) + bl n
-        if constexpr (is_fp64<R>::value) {
-            R bnl = R(0) + pl[5 + a], bnr = R(0) + pr[5 + a];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                R nk = R(k == a);
-                pl[5 + k] = (pl[5 + k] - bnl * nk) + bl * nk;
-                pr[5 + k] = (pr[5 + k] - bnr * nk) + bl * nk;
-            }
-        } else {
-            pl[5 + a] = bl;
-            pr[5 + a] = bl;
-        }
+        // with_longitudinal_field :165-176: (b - (b.n) n) + bl n is bl along
+        // the normal and b across it
+        pl[5 + a] = bl;
+        pr[5 + a] = bl;
         R ul[5], ur[5], fl[5], fr[5], il[3], ir[3], alm, alp, arm, arp;
         cons(pl, gamma, ul);
         cons(pr, gamma, ur);
@@ -172,36 +160,33 @@ struct Mhd {
         wavespeeds<AXIS>(pr, gamma, arm, arp);
         R ap = smax(R(0), smax(alp, arp));
         R am = smin(R(0), smin(alm, arm));
+        // -n x hll_induction takes the two transverse components only (b, c
+        // the next axes after a in cyclic order: e_b = hi_c, e_c = -hi_b,
+        // e_a = 0)
+        constexpr int bx = (a + 1) % 3, c = (a + 2) % 3;
         R hi[3];
         if constexpr (is_fp64<R>::value) {
-            const R inv = rcp_nr(ap - am);   // one reciprocal for the eight components
+            const R inv = rcp_nr(ap - am);   // one reciprocal for the seven components
 #pragma unroll
             for (int k = 0; k < 5; ++k) f[k] = (ap * fl[k] - am * fr[k] - (ul[k] - ur[k]) * ap * am) * inv;
 #pragma unroll
-            for (int k = 0; k < 3; ++k) hi[k] = (ap * il[k] - am * ir[k] - (pl[5 + k] - pr[5 + k]) * ap * am) * inv;
+            for (int k = 0; k < 3; ++k) {
+                if (k == a) continue;
+                hi[k] = (ap * il[k] - am * ir[k] - (pl[5 + k] - pr[5 + k]) * ap * am) * inv;
+            }
         } else {
             R inv = frcp(ap - am), apam = ap * am;
 #pragma unroll
             for (int k = 0; k < 5; ++k) f[k] = fmaf(ap, fl[k], fmaf(-am, fr[k], -(ul[k] - ur[k]) * apam)) * inv;
-            // -n x hll_induction takes the two transverse components only
-            // (b, c the next axes after a in cyclic order: e_b = hi_c,
-            // e_c = -hi_b, e_a = 0)
-            constexpr int bx = (a + 1) % 3, c = (a + 2) % 3;
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
                 if (k == a) continue;
                 hi[k] = fmaf(ap, il[k], fmaf(-am, ir[k], -(pl[5 + k] - pr[5 + k]) * apam)) * inv;
             }
-            e[a] = R(0);
-            e[bx] = hi[c];
-            e[c] = -hi[bx];
-            return;
         }
-        // -n x hll_induction
-        R n[3] = { R(AXIS == 1), R(AXIS == 2), R(AXIS == 3) };
-        e[0] = -(n[1] * hi[2] - n[2] * hi[1]);
-        e[1] = -(n[2] * hi[0] - n[0] * hi[2]);
-        e[2] = -(n[0] * hi[1] - n[1] * hi[0]);
+        e[a] = R(0);
+        e[bx] = hi[c];
+        e[c] = -hi[bx];
     }
 };
 
@@ -360,15 +345,6 @@ mhd_prim_kernel(MhdArgs a, typename MhdPrim<R>::V* P)
     if (threadIdx.x == 0) a.vmax[blockIdx.x] = fmax(fmax(part[0], part[1]), fmax(part[2], part[3]));
 }
 
-// Half the PLM slope of the middle value: the reference's 0.5 * plm_gradient
-// in FP64, the three-operand median form in FP32 (the same value).
-template<typename R>
-__device__ __forceinline__ R mhd_half_slope(R c0, R c1, R c2, R theta)
-{
-    if constexpr (is_fp64<R>::value) return R(0.5) * plm(c0, c1, c2, theta);
-    else return plm_half(c0, c1, c2, theta);
-}
-
 // The flux pass fused with the conserved
 // update, by column tiles.  A workgroup owns TJ x TK columns (j, k) and
 // marches along i over TI planes of one segment.  Each thread keeps a
@@ -460,8 +436,8 @@ mhd_tile_kernel(MhdArgs a, const typename MhdPrim<R>::V* P, R* E1, R* E2, R* E3,
     auto states = [&] (const R* c0, const R* c1, const R* c2, const R* c3, R* pl, R* pr) {
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-            pl[q] = c1[q] + mhd_half_slope(c0[q], c1[q], c2[q], theta);
-            pr[q] = c2[q] - mhd_half_slope(c1[q], c2[q], c3[q], theta);
+            pl[q] = c1[q] + plm_half(c0[q], c1[q], c2[q], theta);
+            pr[q] = c2[q] - plm_half(c1[q], c2[q], c3[q], theta);
         }
     };
 
@@ -477,8 +453,8 @@ mhd_tile_kernel(MhdArgs a, const typename MhdPrim<R>::V* P, R* E1, R* E2, R* E3,
         loadP(cell(i0 + 1, j, k), Pp);
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-            g0[q] = mhd_half_slope(Pm[q], P0[q], Pp[q], theta);
-            pl[q] = Pm[q] + mhd_half_slope(Pm2[q], Pm[q], P0[q], theta);
+            g0[q] = plm_half(Pm[q], P0[q], Pp[q], theta);
+            pl[q] = Pm[q] + plm_half(Pm2[q], Pm[q], P0[q], theta);
             pr[q] = P0[q] - g0[q];
         }
         const long f = ((long)i0 * N + jc) * N + kc;
@@ -590,7 +566,7 @@ mhd_tile_kernel(MhdArgs a, const typename MhdPrim<R>::V* P, R* E1, R* E2, R* E3,
             R pl[8], pr[8], e[3];
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
-                const R gp = mhd_half_slope(P0[q], Pp[q], Pn[q], theta);
+                const R gp = plm_half(P0[q], Pp[q], Pn[q], theta);
                 pl[q] = P0[q] + g0[q];
                 pr[q] = Pp[q] - gp;
                 g0[q] = gp;

@@ -30,12 +30,13 @@ struct Euler {
     {
         if constexpr (is_fp64<R>::value) {
             double D = u[0], S1 = u[1], S2 = u[2], S3 = u[3], E = u[4];
-            double ls = ((0.0 + S1 * S1) + S2 * S2) + S3 * S3;
-            double ke = 0.5 * ls / D;
+            double ls = (S1 * S1 + S2 * S2) + S3 * S3;
+            const Divisor<double> by_D(D);
+            double ke = by_D(0.5 * ls);
             p[0] = D;
-            p[1] = S1 / D;
-            p[2] = S2 / D;
-            p[3] = S3 / D;
+            p[1] = by_D(S1);
+            p[2] = by_D(S2);
+            p[3] = by_D(S3);
             p[4] = (E - ke) * (prm.gamma - 1.0);
             return !(D < 0.0);
         } else {
@@ -61,17 +62,21 @@ struct Euler {
     {
         R d = p[0], v1 = p[1], v2 = p[2], v3 = p[3], pg = p[4];
         if constexpr (is_fp64<R>::value) {
-            R ls = ((R(0) + v1 * v1) + v2 * v2) + v3 * v3;
+            // The reference's sums with the zeros of the unit normal and of
+            // an empty sum left out: the same values (a zero may differ in
+            // its sign) for every finite state
+            R ls = (v1 * v1 + v2 * v2) + v3 * v3;
             u[0] = d;
             u[1] = d * v1;
             u[2] = d * v2;
             u[3] = d * v3;
-            u[4] = d * ls * R(0.5) + pg / (gamma - R(1));
-            R vn = R(0) + p[AXIS];
-            f[0] = vn * u[0] + R(0);
-            f[1] = vn * u[1] + pg * R(AXIS == 1 ? 1 : 0);
-            f[2] = vn * u[2] + pg * R(AXIS == 2 ? 1 : 0);
-            f[3] = vn * u[3] + pg * R(AXIS == 3 ? 1 : 0);
+            u[4] = d * ls * R(0.5) + Divisor<R>(gamma - R(1))(pg);   // the reciprocal is loop invariant
+            R vn = p[AXIS];
+            f[0] = vn * u[0];
+            f[1] = vn * u[1];
+            f[2] = vn * u[2];
+            f[3] = vn * u[3];
+            f[AXIS] += pg;
             f[4] = vn * u[4] + pg * vn;
         } else {
             R ls = fmaf(v3, v3, fmaf(v2, v2, v1 * v1));
@@ -95,8 +100,8 @@ struct Euler {
     __device__ static __forceinline__ void speeds(const R* p, R gamma, R& am, R& ap)
     {
         if constexpr (is_fp64<R>::value) {
-            R vn = R(0) + p[AXIS];
-            R cs = sqrt(gamma * p[4] / p[0]);
+            R vn = p[AXIS];
+            R cs = sqrt_ieee(gamma * p[4] / p[0]);
             am = vn - cs;
             ap = vn + cs;
         } else {
@@ -126,9 +131,10 @@ struct Euler {
         R ap = smax(R(0), smax(alp, arp));
         R am = smin(R(0), smin(alm, arm));
         if constexpr (is_fp64<R>::value) {
+            const Divisor<R> by_width(ap - am);
 #pragma unroll
             for (int k = 0; k < NC; ++k)
-                f[k] = (ap * fl[k] - am * fr[k] - (ul[k] - ur[k]) * ap * am) / (ap - am);
+                f[k] = by_width(ap * fl[k] - am * fr[k] - (ul[k] - ur[k]) * ap * am);
         } else {
             // the wave-speed weights folded in: F = wp F_L + wm F_R + wpm (U_L - U_R)
             // with wp = a+ / (a+ - a-), wm = -a- / (a+ - a-), wpm = -a+ a- / (a+ - a-)
@@ -217,9 +223,10 @@ struct Iso2d {
     __device__ static __forceinline__ void recover(const double* u, R* p)
     {
         if constexpr (is_fp64<R>::value) {
+            const Divisor<double> by_sigma(u[0]);
             p[0] = u[0];
-            p[1] = u[1] / u[0];
-            p[2] = u[2] / u[0];
+            p[1] = by_sigma(u[1]);
+            p[2] = by_sigma(u[2]);
         } else {
             float s = float(u[0]);
             float is = __builtin_amdgcn_rcpf(s);
@@ -239,11 +246,13 @@ struct Iso2d {
         if constexpr (is_fp64<R>::value) {
             R ul[3] = { pl[0], pl[0] * pl[1], pl[0] * pl[2] };
             R ur[3] = { pr[0], pr[0] * pr[1], pr[0] * pr[2] };
-            R vnl = R(0) + pl[AXIS], vnr = R(0) + pr[AXIS];
-            R pgl = pl[0] * cs2, pgr = pr[0] * cs2;
-            R fl[3] = { vnl * ul[0] + R(0), vnl * ul[1] + pgl * R(AXIS == 1 ? 1 : 0), vnl * ul[2] + pgl * R(AXIS == 2 ? 1 : 0) };
-            R fr[3] = { vnr * ur[0] + R(0), vnr * ur[1] + pgr * R(AXIS == 1 ? 1 : 0), vnr * ur[2] + pgr * R(AXIS == 2 ? 1 : 0) };
-            R cs = RCP ? sqrt_nr(cs2) : sqrt(cs2);
+            // without the zeros of the unit normal (as Euler::cons_flux)
+            R vnl = pl[AXIS], vnr = pr[AXIS];
+            R fl[3] = { vnl * ul[0], vnl * ul[1], vnl * ul[2] };
+            R fr[3] = { vnr * ur[0], vnr * ur[1], vnr * ur[2] };
+            fl[AXIS] += pl[0] * cs2;
+            fr[AXIS] += pr[0] * cs2;
+            R cs = RCP ? sqrt_nr(cs2) : sqrt_ieee(cs2);
             R alm = vnl - cs, alp = vnl + cs;
             R arm = vnr - cs, arp = vnr + cs;
             R ap = smax(R(0), smax(alp, arp));
@@ -254,9 +263,10 @@ struct Iso2d {
                 for (int k = 0; k < 3; ++k)
                     f[k] = (ap * fl[k] - am * fr[k] - (ul[k] - ur[k]) * ap * am) * inv;
             } else {
+                const Divisor<R> by_width(ap - am);
 #pragma unroll
                 for (int k = 0; k < 3; ++k)
-                    f[k] = (ap * fl[k] - am * fr[k] - (ul[k] - ur[k]) * ap * am) / (ap - am);
+                    f[k] = by_width(ap * fl[k] - am * fr[k] - (ul[k] - ur[k]) * ap * am);
             }
         } else {
             // The same HLL flux with the wave-speed weights folded in:

@@ -69,8 +69,9 @@ struct EulerScheme {
                                                   double dt, double dl, double* out)
     {
         if constexpr (is_fp64<R>::value) {
+            const Divisor<double> by_dl(dl);
 #pragma unroll
-            for (int q = 0; q < NC; ++q) out[q] = u[q] - (dfx[q] + dfy[q]) * dt / dl;
+            for (int q = 0; q < NC; ++q) out[q] = u[q] - by_dl((dfx[q] + dfy[q]) * dt);
         } else {
             double dtdl = dt / dl;
 #pragma unroll
@@ -426,8 +427,9 @@ struct IsoTableScheme {
                                                   const double* dfx, const double* dfy,
                                                   double dt, double dl, double* out)
     {
+        const Divisor<double> by_dl(dl);
 #pragma unroll
-        for (int q = 0; q < NC; ++q) out[q] = u[q] - (dfx[q] + dfy[q]) * dt / dl;
+        for (int q = 0; q < NC; ++q) out[q] = u[q] - by_dl((dfx[q] + dfy[q]) * dt);
     }
 };
 

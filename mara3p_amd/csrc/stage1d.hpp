@@ -203,10 +203,11 @@ stage1d_kernel(EulerParams prm, Stage1DArgs a)
         const int z = c0 + t;
         double* o = a.out + (size_t)b * NC * n + z;
         double wv[NC];
+        const Divisor<double> by_dl(dl);
         for (int q = 0; q < NC; ++q) {
             double dfx = double(F[q][t + 1]) - double(F[q][t]);
             double res;
-            if constexpr (is_fp64<R>::value) res = uz[q] - dfx * dt / dl;
+            if constexpr (is_fp64<R>::value) res = uz[q] - by_dl(dfx * dt);
             else res = uz[q] - dfx * (dt / dl);
             if (a.u0) res = U0[q] * a.rk_b + res * (1.0 - a.rk_b);
             o[(size_t)q * n] = res;

@@ -23,10 +23,10 @@ namespace m3p {
 
 template<typename R>
 struct ViscousTerms {
-    // derivative from two full slopes: 0.5 (a + b) / dl
-    __device__ static __forceinline__ R mean_over(R a, R b, double dl, R idl)
+    // derivative from two full slopes: 0.5 (a + b) / dl (FP32: times 1 / dl)
+    __device__ static __forceinline__ R mean_over(R a, R b, const Divisor<double>& by_dl, R idl)
     {
-        if constexpr (is_fp64<R>::value) return R(0.5) * (a + b) / dl;
+        if constexpr (is_fp64<R>::value) return by_dl(R(0.5) * (a + b));
         else return R(0.5) * (a + b) * idl;
     }
     // Adds the stress of a face of axis AXIS to f.  pl, pr: the face states
@@ -34,13 +34,13 @@ struct ViscousTerms {
     // and upper cells, along (L) and across (T) the face normal.
     template<int AXIS>
     __device__ static __forceinline__ void add(R* f, const R* pl, const R* pr, const R* glL, const R* guL,
-                                               const R* glT, const R* guT, double nu, double dl, R idl)
+                                               const R* glT, const R* guT, double nu, const Divisor<double>& by_dl, R idl)
     {
         R mu = R(nu) * R(0.5) * (pr[0] + pl[0]);
-        R dL_vx = mean_over(glL[1], guL[1], dl, idl);
-        R dT_vx = mean_over(glT[1], guT[1], dl, idl);
-        R dL_vy = mean_over(glL[2], guL[2], dl, idl);
-        R dT_vy = mean_over(glT[2], guT[2], dl, idl);
+        R dL_vx = mean_over(glL[1], guL[1], by_dl, idl);
+        R dT_vx = mean_over(glT[1], guT[1], by_dl, idl);
+        R dL_vy = mean_over(glL[2], guL[2], by_dl, idl);
+        R dT_vy = mean_over(glT[2], guT[2], by_dl, idl);
         if constexpr (AXIS == 1) {          // L = x, T = y
             R tauxx = mu * (dL_vx - dT_vy);
             R tauxy = mu * (dL_vy + dT_vx);
@@ -80,6 +80,7 @@ iso_visc_stage_kernel(typename S::Params prm, Ld ld_arg, StageArgs a, double nu)
     S::setup_zone(td, prm, tc);
     const double dt = a.dt_dev ? *a.dt_dev : a.dt;
     const double dl = a.dl_blk ? a.dl_blk[b] : a.dl;
+    const Divisor<double> by_dl(dl);
     const R idl = R(1.0 / dl);
     const R theta = R(S::theta(prm));
     bool ok = true;
@@ -116,22 +117,22 @@ iso_visc_stage_kernel(typename S::Params prm, Ld ld_arg, StageArgs a, double nu)
 #pragma unroll
         for (int m = 0; m < NC; ++m) { pl[m] = P[1][2][m] + R(0.5) * gxm[m]; pr[m] = P[2][2][m] - R(0.5) * gx0[m]; }
         S::template face<1>(pl, pr, prm, td, tc, k, c, f[0]);
-        ViscousTerms<R>::template add<1>(f[0], pl, pr, gxm, gx0, gym, gy0, nu, dl, idl);
+        ViscousTerms<R>::template add<1>(f[0], pl, pr, gxm, gx0, gym, gy0, nu, by_dl, idl);
         // x face above: cells (0,0) | (1,0)
 #pragma unroll
         for (int m = 0; m < NC; ++m) { pl[m] = P[2][2][m] + R(0.5) * gx0[m]; pr[m] = P[3][2][m] - R(0.5) * gxp[m]; }
         S::template face<1>(pl, pr, prm, td, tc, k + 1, c, f[1]);
-        ViscousTerms<R>::template add<1>(f[1], pl, pr, gx0, gxp, gy0, gyp, nu, dl, idl);
+        ViscousTerms<R>::template add<1>(f[1], pl, pr, gx0, gxp, gy0, gyp, nu, by_dl, idl);
         // y face left: cells (0,-1) | (0,0)
 #pragma unroll
         for (int m = 0; m < NC; ++m) { pl[m] = P[2][1][m] + R(0.5) * gyl[m]; pr[m] = P[2][2][m] - R(0.5) * gy0[m]; }
         S::template face<2>(pl, pr, prm, td, tc, k, c, f[2]);
-        ViscousTerms<R>::template add<2>(f[2], pl, pr, gyl, gy0, gxl, gx0, nu, dl, idl);
+        ViscousTerms<R>::template add<2>(f[2], pl, pr, gyl, gy0, gxl, gx0, nu, by_dl, idl);
         // y face right: cells (0,0) | (0,1)
 #pragma unroll
         for (int m = 0; m < NC; ++m) { pl[m] = P[2][2][m] + R(0.5) * gy0[m]; pr[m] = P[2][3][m] - R(0.5) * gyr[m]; }
         S::template face<2>(pl, pr, prm, td, tc, k, c + 1, f[3]);
-        ViscousTerms<R>::template add<2>(f[3], pl, pr, gy0, gyr, gx0, gxr, nu, dl, idl);
+        ViscousTerms<R>::template add<2>(f[3], pl, pr, gy0, gyr, gx0, gxr, nu, by_dl, idl);
     }
     double dfx[NC], dfy[NC], uu[NC], res[NC];
 #pragma unroll

@@ -228,6 +228,40 @@ def test_every_tile_shape_gives_the_same_minidisk_step(precision):
         assert err <= 1e-12, err
 
 
+@pytest.mark.parametrize("lo, hi", [(-8, 8), (-900, 400), (-1032, -960)])
+def test_quotients_by_one_denominator(lo, hi):
+    """The FP64 recovery takes the reciprocal of the density once: its four
+    quotients equal IEEE division bit for bit, over ordinary and extreme
+    binary exponents lo..hi of the numerators and -1000..900 of the density,
+    with zeros of both signs, infinities, NaN and zero densities among them."""
+    from mara3p_amd import check, lib
+    rng = np.random.default_rng(17)
+    n = 200000
+
+    def values(a, b):
+        x = np.ldexp(1.0 + rng.random(n), rng.integers(a, b, n)) * rng.choice([-1.0, 1.0], n)
+        x[rng.integers(0, n, 2000)] = 0.0
+        x[rng.integers(0, n, 2000)] = -0.0
+        return x
+    D = np.abs(values(-1000, 900))
+    S = [values(lo, hi) for _ in range(3)]
+    E = values(lo, hi)
+    D[:3], S[0][3], S[0][4] = [np.inf, np.nan, 1.0], np.inf, np.nan
+    u = torch.as_tensor(np.stack([D, *S, E]), device="cuda")
+    p = torch.empty_like(u)
+    check(lib().m3p_euler_recover_primitive_array(u.data_ptr(), p.data_ptr(), n, 5.0 / 3.0, None))
+    got = p.cpu().numpy()
+    with np.errstate(all="ignore"):
+        ke = 0.5 * ((S[0] * S[0] + S[1] * S[1]) + S[2] * S[2]) / D
+        ref = [D, S[0] / D, S[1] / D, S[2] / D, (E - ke) * (5.0 / 3.0 - 1.0)]
+        over = np.isinf(ke) | np.any([np.isinf(b) & np.isfinite(a) & (D != 0) for a, b in zip(S, ref[1:4])], axis=0)
+    for a, b in zip(got, ref):
+        # subnormal quotients and zones where one overflows aside
+        usual = ((np.abs(b) >= 2.0 ** -1022) | (b == 0) | ~np.isfinite(b)) & (~over | (D == 0))
+        assert usual.mean() > 0.4
+        assert np.array_equal(a[usual], b[usual], equal_nan=True)
+
+
 @pytest.mark.parametrize("n, depth", [(16, 0), (16, 5), (32, 1), (32, 5), (48, 1), (64, 0), (64, 3), (64, 4), (64, 5),
                                       (96, 2), (128, 4), (192, 1), (192, 3)])
 def test_tile_of_each_mesh_size(n, depth):
