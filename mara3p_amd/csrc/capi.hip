@@ -223,11 +223,14 @@ bool tile_fits(TileShape v, int n) { return n % v.tj == 0 && n % v.h == 0 && v.h
 // that fills the device wants long ones.  The lines are from sweeps of both
 // stages on meshes of 64^2 to 4096^2 zones: two-row strips below 2048 waves
 // of four rows (FP64 Euler, 256^2 zones in 32^2 blocks: 24 us a step, 32 with
-// four rows, 92 with sixteen), four rows up to 2048 waves of eight, eight up
-// to 4096 waves of sixteen (1024^2 zones in 64^2 blocks: FP64 95 us against
-// 115 with sixteen rows, mixed 47 against 65).  Beyond that sixteen rows in
-// FP64 (2048^2: 325 us against 339 with eight), eight in mixed (153 against
-// 169) and on quad-trees (1408 leaves of 64^2, mixed: 223 against 233).
+// four rows, 92 with sixteen), four rows up to 2048 waves of eight, then eight
+// (1024^2 zones in 64^2 blocks: FP64 80 us against 100 with sixteen rows,
+// mixed 47 against 65).  Meshes of 4096 waves of sixteen rows or more take
+// the wide tiles where they fit (4096^2 in 256^2 blocks, FP64: 1026 us against
+// 1076 with 64 x 8), else stay at eight (2048^2 in 64^2 blocks, FP64: 266 us
+// against 312 with sixteen; quad-tree of 1408 leaves, mixed: 223 against
+// 233), but for the FP64 minidisk from 8192 waves on (4096^2 in 64^2 blocks:
+// 806 us with sixteen, 841 with eight).
 TileShape pick_tile(int kind, int precision, int n, int nblk)
 {
     const int chosen = g_tile[kind][precision].load(std::memory_order_relaxed);
@@ -239,8 +242,11 @@ TileShape pick_tile(int kind, int precision, int n, int nblk)
         if (tile_fits(kLargeTile[kind], n)) return kLargeTile[kind];
         if (precision == M3P_MIXED && n % 128 == 0) return {128, 32};     // 153 us against 163 (64 x 8) at 2048^2
     }
+    if (n % 64 == 0) {
+        const bool long_strips = precision == M3P_FP64 && kind == M3P_KIND_MINIDISK && waves(16) >= 8192;
+        return {64, rows == 16 && !long_strips ? 8 : rows};
+    }
     if (rows == 16 && (precision == M3P_MIXED || kind == M3P_KIND_AMR_EULER2D)) rows = 8;
-    if (n % 64 == 0) return {64, rows};
     if (n % 32 == 0) return {32, 2 * rows};                   // two strips a wave
     if (n % 16 == 0) return {16, 4 * std::min(rows, 4)};      // four
     return {0, 0};

@@ -45,7 +45,7 @@ int launch_stage2d_shape(TileShape ts, const typename S::Params& prm, const Ld& 
 {
     // A stage without a base state has its own kernels only where the scheme
     // fetches more rows ahead there (and the loader pipelines its rows).
-    if constexpr (S::kPrefetchRows > 1 && Ld::kPrefetch)
+    if constexpr (S::kFirstStage && Ld::kPrefetch)
         if (!a.u0) return launch_stage2d_variant<S, Ld, true>(ts, prm, ld, a, s);
     return launch_stage2d_variant<S, Ld, false>(ts, prm, ld, a, s);
 }

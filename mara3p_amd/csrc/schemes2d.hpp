@@ -23,13 +23,21 @@ struct TileCtx {
 template<typename R>
 struct EulerScheme {
     static constexpr int NC = 5;
-    static constexpr int kWavesPerEU = is_fp64<R>::value ? 2 : 3;   // occupancy floor (VGPR budget)
-    static constexpr bool kLateBase = false;  // RK base loaded at the top of a row (pipelined loader)
-    static constexpr int kMarchUnroll = 2;   // rows per march iteration with a pipelined loader
-    // rows a first stage fetches ahead (pipelined loader): two made stage 1
-    // 2 % faster for KH FP64 and the quad-tree mixed stage, 1 % slower for
-    // the quad-tree FP64 stage
-    static constexpr int kPrefetchRows = 2;
+    // The march's schedule, by the rows of a strip.  FP64 strips of eight rows
+    // or more run at three waves per SIMD (166 VGPRs, no spills), which takes
+    // the RK base at the update, one row of loads ahead and one row per
+    // iteration: 4096^2 Kelvin-Helmholtz 1.08 to 1.01 ms a step, 1408 leaves
+    // of 64^2 434 to 400 us.  Shorter strips, on meshes that do not fill the
+    // device, keep two waves, the base at the top of the row, two rows ahead
+    // and two per iteration (22.2 to 21.5 us at 256^2 in 32^2 blocks).  Mixed:
+    // three waves, two rows per iteration; two rows ahead made stage 1 2 %
+    // faster for the quad-tree.
+    static constexpr bool lean(int rows) { return is_fp64<R>::value && rows >= 8; }
+    static constexpr int waves_per_eu(int rows) { return is_fp64<R>::value && !lean(rows) ? 2 : 3; }   // VGPR budget
+    static constexpr bool late_base(int rows) { return lean(rows); }    // RK base loaded at the update
+    static constexpr int march_unroll(int rows) { return lean(rows) ? 1 : 2; }
+    static constexpr int prefetch_rows(int rows) { return lean(rows) ? 1 : 2; }   // a first stage's rows ahead
+    static constexpr bool kFirstStage = true;    // first stages have kernels of their own
     static constexpr bool kCfl = true;       // stage kernels can fuse the CFL reduction
     // the fused RK2 step (both stages' windows of five components) at two
     // waves per SIMD: 178 VGPRs, and its 61 KB of LDS fit two workgroups per CU
@@ -118,15 +126,16 @@ struct MinidiskScheme {
     static constexpr int NC = 3;
     // FP64 at three waves per SIMD (168 VGPRs): the first stage spills 3
     // and runs 13 % faster than at two; the second, with its RK base loaded
-    // at the update (kLateBase), spills none and runs 5 % faster
-    static constexpr int kWavesPerEU = is_fp64<R>::value ? 3 : 4;
-    static constexpr bool kLateBase = is_fp64<R>::value;
+    // at the update, spills none and runs 5 % faster
+    static constexpr int waves_per_eu(int) { return is_fp64<R>::value ? 3 : 4; }
+    static constexpr bool late_base(int) { return is_fp64<R>::value; }
     // three rows per iteration rotate the three-row window in registers; the
     // FP64 kernel runs faster at two (register pressure)
-    static constexpr int kMarchUnroll = is_fp64<R>::value ? 2 : 3;
+    static constexpr int march_unroll(int) { return is_fp64<R>::value ? 2 : 3; }
     // a first stage (no base state) keeps two rows of loads in flight: its
     // stage 1 runs 9 % (mixed) and 2 % (FP64) faster than with one
-    static constexpr int kPrefetchRows = 2;
+    static constexpr int prefetch_rows(int) { return 2; }
+    static constexpr bool kFirstStage = true;
     // the fused RK2 step (both stages' windows) at three waves per SIMD
     static constexpr int kFusedWavesPerEU = 3;
     static constexpr bool kCfl = false;
@@ -389,10 +398,11 @@ struct IsoTableParams {
 template<typename R>
 struct IsoTableScheme {
     static constexpr int NC = 3;
-    static constexpr int kWavesPerEU = 2;
-    static constexpr bool kLateBase = false;
-    static constexpr int kMarchUnroll = 2;
-    static constexpr int kPrefetchRows = 1;
+    static constexpr int waves_per_eu(int) { return 2; }
+    static constexpr bool late_base(int) { return false; }
+    static constexpr int march_unroll(int) { return 2; }
+    static constexpr int prefetch_rows(int) { return 1; }
+    static constexpr bool kFirstStage = false;
     static constexpr bool kCfl = false;
     using Real = R;
     using Params = IsoTableParams;

@@ -105,7 +105,7 @@ struct MeshLoader {
     // Split load for software pipelining: fetch the raw conserved state of a
     // row zone one iteration ahead, recover it when it is needed.
     static constexpr bool kPrefetch = true;
-    static constexpr bool kUnroll = true;    // march unrolled by the scheme's kMarchUnroll
+    static constexpr bool kUnroll = true;    // march unrolled by the scheme's march_unroll
     static constexpr bool kEdgeFluxes = false;   // no edge-flux register (uniform meshes)
     __device__ __forceinline__ void fetch_row(int b, int r, int c, double* raw) const { cons_row(b, r, c, raw); }
     __device__ __forceinline__ bool finish_row(int, int, int, const typename S::Params& prm, const double* raw,
@@ -304,7 +304,7 @@ __device__ __forceinline__ void store_edge_flux(double* reg, int b, int e, int n
 // its load to its update (no second read of the state); otherwise re-load it
 // at the update (fewer registers).  FIRST: a stage without a base state
 // (a.u0 == nullptr is then assumed); it has fewer loads in flight per row, so
-// a scheme may ask it to fetch more rows ahead (S::kPrefetchRows).
+// a scheme may ask it to fetch more rows ahead (S::prefetch_rows).
 //
 // G: a tile of H rows is marched as G strips of H / G rows, by G groups of TJ
 // lanes side by side.  A tile narrower than a wave (TJ = 16 or 32) takes
@@ -314,13 +314,14 @@ __device__ __forceinline__ void store_edge_flux(double* reg, int b, int e, int n
 constexpr int stage2d_waves(int waves, int strips) { return strips > 1 && waves > 2 ? waves - 1 : waves; }
 
 template<class S, class Ld, int H, int TJ, int G, bool KEEPU, bool FIRST = false>
-__global__ void __launch_bounds__(TJ * G) __attribute__((amdgpu_waves_per_eu(stage2d_waves(S::kWavesPerEU, G), 8)))
+__global__ void __launch_bounds__(TJ * G) __attribute__((amdgpu_waves_per_eu(stage2d_waves(S::waves_per_eu(H / G), G), 8)))
 stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
 {
     constexpr int NC = S::NC;
     constexpr int NT = TJ * G;                 // lanes of the workgroup
     constexpr int HS = H / G;                  // rows of a strip
     static_assert(H % G == 0, "whole strips");
+    constexpr bool kLateBase = S::late_base(HS);
     using R = typename S::Real;
     resolve_params(prm);
 
@@ -408,7 +409,7 @@ stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
     // support it are software-pipelined: the raw state of the row three
     // ahead and the RK base of the current row are fetched at the top of an
     // iteration, so their latency overlaps the iteration's arithmetic (a
-    // scheme with kLateBase loads the RK base at the update instead, holding
+    // scheme with late_base loads the RK base at the update instead, holding
     // fewer registers across the row).
     auto march = [&] (auto dir) {
         constexpr int D = decltype(dir)::value;
@@ -454,14 +455,14 @@ stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
 
         // Prefetched raw rows: Unx[i] = row k + (2 + i) D of the iteration
         // that follows, kAhead rows in flight.
-        constexpr int kAhead = FIRST ? S::kPrefetchRows : 1;
+        constexpr int kAhead = FIRST ? S::prefetch_rows(HS) : 1;
         static_assert(kAhead >= 1 && kAhead <= HS, "rows ahead within the strip");
         double Unx[kAhead][NC] = {};
         if constexpr (Ld::kPrefetch) {
 #pragma unroll
             for (int i = 0; i < kAhead; ++i) ld.fetch_row(b, kfirst + (2 + i) * D, c, Unx[i]);
         }
-        constexpr int kRowsPerIter = Ld::kUnroll ? S::kMarchUnroll : 1;
+        constexpr int kRowsPerIter = Ld::kUnroll ? S::march_unroll(HS) : 1;
 #pragma unroll kRowsPerIter
         for (int kk = 0; kk < HS; ++kk) {
             const int k = kfirst + D * kk;
@@ -478,7 +479,7 @@ stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
                     for (int m = 0; m < NC; ++m) Unx[i][m] = Unx[i + 1][m];
                 // the last row a strip reads is kfirst + (HS + 1) D
                 if (kk + kAhead < HS) ld.fetch_row(b, k + (2 + kAhead) * D, c, Unx[kAhead - 1]);
-                if constexpr (!S::kLateBase) {
+                if constexpr (!kLateBase) {
                     if (!FIRST && a.u0) {
                         const double* z0 = a.u0 + ((size_t)b * NC * n + k) * n + c;
 #pragma unroll
@@ -545,11 +546,11 @@ stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
             // pipeline) are issued before the barrier, which orders memory
             // and so would hold them after it, so that their latency overlaps
             // the wait (FP64 KH and Sedov steps 0.6 and 0.9 % faster).  A
-            // scheme with kLateBase keeps its RK base load at the update: held
+            // scheme with late_base keeps its RK base load at the update: held
             // across the barrier it spills 20 registers.
             double uu[NC];
             if constexpr (!KEEPU) ld.cons_row(b, k, c, uu);
-            if constexpr (!Ld::kPrefetch && !S::kLateBase) {
+            if constexpr (!Ld::kPrefetch && !kLateBase) {
                 if (!FIRST && a.u0) {
                     const double* z0 = a.u0 + ((size_t)b * NC * n + k) * n + c;
 #pragma unroll
@@ -576,7 +577,7 @@ stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
             double* o = a.out + ((size_t)b * NC * n + k) * n + c;
             double wv[NC];
             if (!FIRST && a.u0) {
-                if constexpr (S::kLateBase) {
+                if constexpr (kLateBase) {
                     const double* z0 = a.u0 + ((size_t)b * NC * n + k) * n + c;
 #pragma unroll
                     for (int m = 0; m < NC; ++m) U0[m] = __builtin_nontemporal_load(&z0[(size_t)m * n * n]);
