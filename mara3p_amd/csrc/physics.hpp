@@ -204,10 +204,10 @@ struct Euler {
     // reduction and the separate reduction evaluate the same expression.
     __device__ static __forceinline__ double max_speed(const double* u, const Params& prm)
     {
-        double D = u[0], iD = 1.0 / D;
+        double D = u[0], iD = Divisor<double>(D)(1.0);
         double v1 = u[1] * iD, v2 = u[2] * iD, v3 = u[3] * iD;
         double pg = (u[4] - 0.5 * ((v1 * u[1] + v2 * u[2]) + v3 * u[3])) * (prm.gamma - 1.0);
-        double cs = sqrt(prm.gamma * pg * iD);
+        double cs = sqrt_ieee(prm.gamma * pg * iD);
         return fmax(fabs(v1), fabs(v2)) + cs;
     }
 };

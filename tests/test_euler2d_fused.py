@@ -46,6 +46,18 @@ def test_fused_rk2_equals_two_stages(depth, n, hllc):
     assert np.array_equal(ua, ub), float(np.abs(ua - ub).max())
 
 
+@pytest.mark.parametrize("depth, n", [(3, 128), (4, 64), (2, 256), (5, 64), (4, 128)])
+def test_fused_rk2_rows_by_mesh_size(depth, n):
+    """Meshes on both sides of each line of the rows-by-size rule, in every
+    block size: one step, equal in every value to two stage launches."""
+    a, b = _pair(depth, n, True, seed=8)
+    dt = float(a.cfl_dt(0.4).item())
+    a.step(dt)
+    b.step_fused(dt)
+    b.check_errors()
+    assert torch.equal(a.u, b.u)
+
+
 def test_fused_rk2_equals_two_stages_full_size():
     """The Kelvin-Helmholtz configuration (16 x 16 blocks of 256^2, HLLC):
     two steps, equal in every value."""

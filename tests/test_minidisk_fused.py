@@ -46,6 +46,19 @@ def test_fused_rk2_equals_two_stages(n, depth):
     assert np.array_equal(ua, ub), float(np.abs(ua - ub).max())
 
 
+@pytest.mark.parametrize("n, depth", [(128, 3), (64, 4), (256, 2), (64, 5), (128, 4)])
+def test_fused_rk2_rows_by_mesh_size(n, depth):
+    """Meshes on both sides of each line of the rows-by-size rule, in every
+    block size: one step, equal in every value to two stage launches."""
+    from mara3p_amd import problems
+    data, _, a, b = _pair(n, depth, seed=8)
+    dt = problems.minidisk_dt(data, a.time)
+    a.step(dt)
+    b.step_fused(dt)
+    b.check_errors()
+    assert torch.equal(a.u, b.u)
+
+
 def test_fused_rk2_equals_two_stages_full_size():
     """The full minidisk configuration (16 x 16 blocks of 256^2, [-8, 8]^2,
     softening 0.05, Mach 10, sink radius 0.05): two steps, equal in every
