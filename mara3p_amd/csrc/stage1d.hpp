@@ -35,15 +35,29 @@ struct Stage1DArgs {
 // Persistent work-list form: the grid is sized to the device and each
 // workgroup walks the list of (block, tile) items with a fixed stride, so one
 // launch covers any number of blocks of any mix of problems.
-template<typename R, int TJ>
-__global__ void __launch_bounds__(TJ)
+//
+// SINGLE: every workgroup has one item (the list is shorter than the grid).
+// Such a launch is bound by one item's chain of loads, faces and barriers, so
+// further lanes (a second wave where the tile fills the first) take the guard
+// zones and the left face, which otherwise a pass of its own computes before
+// (FP64) or after (mixed) the other faces.  1024 zones in blocks of 64:
+// 4.4 us a launch against 6.4 in FP64, 4.0 against 4.1 mixed; 400 blocks of 64,
+// FP64: 5.1 against 7.1.
+constexpr int stage1d_lanes(int TJ, bool single) { return !single ? TJ : TJ + 5 <= 64 ? 64 : TJ + 64; }
+
+template<typename R, int TJ, bool SINGLE>
+__global__ void __launch_bounds__(stage1d_lanes(TJ, SINGLE))
 stage1d_kernel(EulerParams prm, Stage1DArgs a)
 {
     constexpr int NC = 5;
+    constexpr int NT = stage1d_lanes(TJ, SINGLE);
+    constexpr int GL = SINGLE ? TJ : 0;     // first of the four lanes that load guard zones
     const int n = a.n;
     const int tiles = n / TJ;
     const long items = (long)a.nblk * tiles;
     const int t = threadIdx.x;
+    const bool zone = !SINGLE || t < TJ;    // the lane has a zone of the item
+    const int g = t - GL;                   // 0 .. 3: the lane's guard zone
     const R theta = R(prm.theta);
     const double dt = a.dt_dev ? *a.dt_dev : a.dt;
 
@@ -51,10 +65,10 @@ stage1d_kernel(EulerParams prm, Stage1DArgs a)
     // one pass of all lanes; the mixed kernel (bound by memory latency) lets
     // lane 0 compute its item's left face from the LDS row, which needs no
     // further loads.
-    constexpr bool kGroupLeftFaces = is_fp64<R>::value;
+    constexpr bool kGroupLeftFaces = is_fp64<R>::value && !SINGLE;
     __shared__ R P[NC][TJ + 4];   // [i] = zone c0 - 2 + i
     __shared__ R F[NC][TJ + 1];   // [i] = face c0 + i (left face of zone c0 + i)
-    __shared__ R Fl[NC][TJ];      // left face of each item of the current group
+    __shared__ R Fl[NC][kGroupLeftFaces ? TJ : 1];   // left face of each item of the current group
 
     // The lane's own zone of the next item, and for lanes 0-3 the four guard
     // zones of that item (c0 - 2, c0 - 1, c0 + TJ, c0 + TJ + 1: neighbour
@@ -79,13 +93,15 @@ stage1d_kernel(EulerParams prm, Stage1DArgs a)
     auto fetch = [&] (long it, double* raw, double* graw) {
         it = slot(it);
         const int b = (int)(it / tiles), c0 = (int)(it % tiles) * TJ;
-        const double* src = a.u + (size_t)b * NC * n + c0 + t;
+        if (zone) {
+            const double* src = a.u + (size_t)b * NC * n + c0 + t;
 #pragma unroll
-        for (int q = 0; q < NC; ++q) raw[q] = src[(size_t)q * n];
-        if (!a.pe && t < 4) {
-            const double* g = guard_zone(b, t < 2 ? c0 - 2 + t : c0 + TJ + (t - 2));
+            for (int q = 0; q < NC; ++q) raw[q] = src[(size_t)q * n];
+        }
+        if (!a.pe && g >= 0 && g < 4) {
+            const double* src = guard_zone(b, g < 2 ? c0 - 2 + g : c0 + TJ + (g - 2));
 #pragma unroll
-            for (int q = 0; q < NC; ++q) graw[q] = g[(size_t)q * n];
+            for (int q = 0; q < NC; ++q) graw[q] = src[(size_t)q * n];
         }
     };
     double nxt[NC] = {}, gnxt[NC] = {};
@@ -154,47 +170,46 @@ stage1d_kernel(EulerParams prm, Stage1DArgs a)
 #pragma unroll
         for (int q = 0; q < NC; ++q) { uz[q] = nxt[q]; gz[q] = gnxt[q]; }
         if (item + gridDim.x < items) fetch(item + gridDim.x, nxt, gnxt);
-        if (a.u0) {
+        if (a.u0 && zone) {
 #pragma unroll
             for (int q = 0; q < NC; ++q) U0[q] = a.u0[(size_t)b * NC * n + (size_t)q * n + c0 + t];
         }
         R p[NC];
-        if (a.pe) load_pe(c0 + t, p);
-        else ok &= Euler<R>::recover(uz, prm, p);
-        for (int q = 0; q < NC; ++q) P[q][t + 2] = p[q];
-        if (t < 4) {
-            if (a.pe) load_pe(t < 2 ? c0 - 2 + t : c0 + TJ + (t - 2), p);
+        if (zone) {
+            if (a.pe) load_pe(c0 + t, p);
+            else ok &= Euler<R>::recover(uz, prm, p);
+            for (int q = 0; q < NC; ++q) P[q][t + 2] = p[q];
+        }
+        if (g >= 0 && g < 4) {
+            if (a.pe) load_pe(g < 2 ? c0 - 2 + g : c0 + TJ + (g - 2), p);
             else ok &= Euler<R>::recover(gz, prm, p);
-            int slot = t < 2 ? t : TJ + 2 + (t - 2);
+            int slot = g < 2 ? g : TJ + 2 + (g - 2);
             for (int q = 0; q < NC; ++q) P[q][slot] = p[q];
         }
         __syncthreads();
-        {
-            // the right face of zone c0 + t (face t + 1), from the half slopes
-            // at zones c0 + t and c0 + t + 1
+        // face i of the tile (the left face of zone c0 + i), from the half
+        // slopes at zones c0 + i - 1 and c0 + i
+        auto face = [&] (int i) {
             R pl[NC], pr[NC], f[NC];
 #pragma unroll
             for (int q = 0; q < NC; ++q) {
-                pl[q] = P[q][t + 2] + plm_half(P[q][t + 1], P[q][t + 2], P[q][t + 3], theta);
-                pr[q] = P[q][t + 3] - plm_half(P[q][t + 2], P[q][t + 3], P[q][t + 4], theta);
+                pl[q] = P[q][i + 1] + plm_half(P[q][i], P[q][i + 1], P[q][i + 2], theta);
+                pr[q] = P[q][i + 2] - plm_half(P[q][i + 1], P[q][i + 2], P[q][i + 3], theta);
             }
             Euler<R>::template riemann<1>(pl, pr, prm, f);
 #pragma unroll
-            for (int q = 0; q < NC; ++q) F[q][t + 1] = f[q];
+            for (int q = 0; q < NC; ++q) F[q][i] = f[q];
+        };
+        if constexpr (SINGLE) {
+            if (t <= TJ) face(t < TJ ? t + 1 : 0);
+        } else {
+            face(t + 1);                    // the right face of the lane's zone
             if (t == 0) {
                 if constexpr (kGroupLeftFaces) {
 #pragma unroll
                     for (int q = 0; q < NC; ++q) F[q][0] = Fl[q][gpos];
                 } else {
-                    // the left face from the LDS row (zones c0 - 2 .. c0 + 1)
-#pragma unroll
-                    for (int q = 0; q < NC; ++q) {
-                        pl[q] = P[q][1] + plm_half(P[q][0], P[q][1], P[q][2], theta);
-                        pr[q] = P[q][2] - plm_half(P[q][1], P[q][2], P[q][3], theta);
-                    }
-                    Euler<R>::template riemann<1>(pl, pr, prm, f);
-#pragma unroll
-                    for (int q = 0; q < NC; ++q) F[q][0] = f[q];
+                    face(0);
                 }
             }
         }
@@ -204,7 +219,7 @@ stage1d_kernel(EulerParams prm, Stage1DArgs a)
         double* o = a.out + (size_t)b * NC * n + z;
         double wv[NC];
         const Divisor<double> by_dl(dl);
-        for (int q = 0; q < NC; ++q) {
+        if (zone) for (int q = 0; q < NC; ++q) {
             double dfx = double(F[q][t + 1]) - double(F[q][t]);
             double res;
             if constexpr (is_fp64<R>::value) res = uz[q] - by_dl(dfx * dt);
@@ -213,13 +228,13 @@ stage1d_kernel(EulerParams prm, Stage1DArgs a)
             o[(size_t)q * n] = res;
             wv[q] = res;
         }
-        if (a.rate_slot) rate = fmax(rate, Euler<double>::max_speed(wv, prm) * idl);
+        if (a.rate_slot && zone) rate = fmax(rate, Euler<double>::max_speed(wv, prm) * idl);
         if (!ok) { report_error(a.err, 1, b, z); ok = true; }
         // No barrier here: the next item writes P and Fl only after this
         // item's flux barrier, which every read of them precedes, and F only
         // after its own first barrier, which follows this item's update.
     }
-    if (a.rate_slot) workgroup_atomic_max<TJ>(rate, a.rate_slot);
+    if (a.rate_slot) workgroup_atomic_max<NT>(rate, a.rate_slot);
 }
 
 } // namespace m3p

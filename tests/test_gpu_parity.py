@@ -360,6 +360,36 @@ def test_euler1d_mesh_every_block_size(n, nblk):
     assert err <= 1e-5, err
 
 
+@pytest.mark.parametrize("n,nblk", [(16, 512), (16, 700), (32, 530), (64, 513), (128, 520), (256, 530), (512, 300)])
+def test_euler1d_long_lists(n, nblk):
+    """Lists of items at and past two per CU, where workgroups of one item
+    each give way to the persistent list, in every tile width: FP64 equals the
+    oracle, mixed stays near it, and the CFL reduction of the second stage
+    equals the separate one."""
+    from mara3p_amd.mesh import EnsembleMesh1D
+    from mara3p_amd.solvers import Euler1DEnsembleSolver
+    x = (np.arange(n * nblk) + 0.5) / (n * nblk)
+    rho, v, p = 1 + 0.2 * np.sin(40 * x), 0.3 * np.cos(30 * x), 1 + 0.3 * np.sin(90 * x)
+    u = np.stack([rho, rho * v, 0 * x, 0 * x, 0.5 * rho * v * v + p / 0.4])
+    u0 = c(u.reshape(5, nblk, n).transpose(1, 0, 2))
+    dl = 1.0 / (n * nblk)
+    ref = c(u0.transpose(0, 2, 1))
+    orc().orc_euler1d_mesh_rk2(P(ref), nblk, n, 0.2 * dl, dl, 1.5, 1.4, 1, 1)
+    for precision in ("fp64", "mixed"):
+        s = Euler1DEnsembleSolver(EnsembleMesh1D([n * nblk], n), gamma=1.4, plm_theta=1.5, precision=precision)
+        s.set_state(u0)
+        dt_next = torch.zeros(1, dtype=torch.float64, device="cuda")
+        s.stage(s.u, None, s.u1, 0.2 * dl)
+        s.stage(s.u1, s.u, s.u2, 0.2 * dl, cfl=0.4, dt_next=dt_next)
+        s.u, s.u2 = s.u2, s.u
+        s.check_errors()
+        if precision == "fp64":
+            assert np.array_equal(s.state(), ref.transpose(0, 2, 1))
+        else:
+            assert rel_err(s.state(), ref.transpose(0, 2, 1)) <= 1e-5
+        assert float(dt_next.item()) == float(s.cfl_dt(0.4).item())
+
+
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 def test_sod_to_t_0_2(precision):
     """The Sod configuration (1024 zones, gamma 1.4, PLM 1.5, HLLE, RK2, CFL
