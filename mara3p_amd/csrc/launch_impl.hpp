@@ -53,8 +53,9 @@ int launch_stage2d_shape(TileShape ts, const typename S::Params& prm, const Ld& 
 template<class S, class Ld>
 int launch_visc(const typename S::Params& prm, const Ld& ld, const StageArgs& a, double nu, hipStream_t s)
 {
-    const long zones = (long)a.nblk * a.n * a.n;
-    hipLaunchKernelGGL((iso_visc_stage_kernel<S, Ld>), dim3((zones + 255) / 256), dim3(256), 0, s, prm, ld, a, nu);
+    const int tiles = (a.n + kViscTile - 1) / kViscTile;
+    hipLaunchKernelGGL((iso_visc_stage_kernel<S, Ld, kViscTile>), dim3(a.nblk * tiles * tiles),
+                       dim3(kViscTile * kViscTile), 0, s, prm, ld, a, nu);
     return launch_status("iso_visc_stage_kernel");
 }
 

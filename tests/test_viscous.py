@@ -111,6 +111,27 @@ def test_minidisk_mesh_viscous_rk2_fp64():
     assert err <= 1e-12, err
 
 
+@pytest.mark.parametrize("n, depth", [(4, 1), (10, 0), (20, 2), (48, 1)])
+def test_minidisk_mesh_viscous_ragged_tiles(n, depth):
+    """Blocks that the 16 x 16 tiles do not divide, smaller and larger than a
+    tile, against the oracle's mesh RK2 (FP64) and FP64 (mixed)."""
+    from mara3p_amd import MinidiskData, problems
+    from mara3p_amd.mesh import to_device_layout, to_reference_layout
+    from mara3p_amd.solvers import MinidiskSolver
+    data = MinidiskData.defaults(block_size=n, depth=depth, domain_radius=2.0, softening_length=0.05,
+                                 sink_radius=0.05, kinematic_viscosity=0.01)
+    _, u0 = problems.minidisk(data, seed=4, noise=0.05)
+    ref = to_reference_layout(u0).copy()
+    dt = problems.minidisk_dt(data, 0.0)
+    assert orc().orc_minidisk_mesh_rk2(P(ref), OrcMinidisk.from_data(data), 0.0, dt, 1, 8) == 0
+    for precision, bar in (("fp64", 1e-12), ("mixed", 1e-5)):
+        s = MinidiskSolver(data, precision)
+        s.set_state(u0)
+        s.step(dt)
+        s.check_errors()
+        assert rel_err(s.state(), to_device_layout(ref)) <= bar
+
+
 def test_minidisk_mesh_viscous_mixed_conserves_and_tracks_fp64():
     """Mixed viscous stages: with sinks and buffer off, mass is conserved to
     round-off; density stays within 1e-5 (L1, relative) of FP64 after 20 steps."""
