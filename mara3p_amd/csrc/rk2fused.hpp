@@ -87,14 +87,25 @@ rk2_fused_kernel(typename S::Params p1, typename S::Params p2, MeshLoader<S> ld,
     __shared__ R e2[6][NC][H];     // U1 primitives at the same columns, rows k0 .. k0 + H - 1
     __shared__ R f2e[NC][H];
     // a step's row of each stage: rowP [t + 2] = column t, [0] and [1] =
-    // columns -2 and -1, [TJ + 2] = column n (pre-pass); rowF [t] = y flux at
-    // face t, [TJ] = face n (pre-pass)
-    __shared__ R rowP1[NC][TJ + 3], rowF1[NC][TJ + 1];
-    __shared__ R rowP2[NC][TJ + 3], rowF2[NC][TJ + 1];
+    // columns -2 and -1, [TJ + 2] = column n (pre-pass)
+    __shared__ R rowP1[NC][TJ + 3], rowP2[NC][TJ + 3];
     // U1 of the last three first-stage rows (row j in slot s % 3), each lane
     // its own column: the second stage reads row j - 3 from the slot the
-    // first stage then overwrites, in program order within the lane
+    // first stage then overwrites, in program order within the lane.
+    // kQueue: the same for U0, which the first stage's update has just read:
+    // read again three rows later it had partly left the L2, and the launch
+    // fetched 1.05 GB for the 0.40 GB of U0 (minidisk, 4096^2: 314 to 303 us
+    // with the queue).  Its LDS must not cost a workgroup per CU: the y fluxes
+    // then pass between lanes by a wave shift instead of an LDS row.  Euler's
+    // five components fit too, but the step takes 217 registers and is 4 %
+    // slower (4096^2: 552 us against 530).
+    constexpr bool kQueue = S::kFusedQueue && TJ == 256 && H == 32;
     __shared__ double u1q[3][NC][TJ];
+    __shared__ double u0q[kQueue ? 3 : 1][NC][kQueue ? TJ : 1];
+    // y flux [t] at face t, [TJ] at face n (pre-pass); kQueue: at each wave's
+    // first column, and [NW] at face n
+    constexpr int NW = TJ / 64, NF = kQueue ? NW + 1 : TJ + 1;
+    __shared__ R rowF1[NC][NF], rowF2[NC][NF];
 
     S::setup_rows(td, p1, tc, bi_of(xm), bi_of(xp));
     const R theta = R(S::theta(p1));
@@ -236,6 +247,29 @@ rk2_fused_kernel(typename S::Params p1, typename S::Params p2, MeshLoader<S> ld,
     double UN[3][NC];
     const double wb = 1.0 - a.rk_b;
 
+    // y fluxes of a row: each lane's own into F (kQueue: the first lane of each
+    // wave's), and after the barrier the flux above the lane's column
+    auto put_flux = [&] (const R* Fy, R (&F)[NC][NF], auto& face_n, int r) {
+        if (!kQueue || (t & 63) == 0) {
+#pragma unroll
+            for (int m = 0; m < NC; ++m) F[m][kQueue ? t / 64 : t] = Fy[m];
+        }
+        if (t == TJ - 1) {
+#pragma unroll
+            for (int m = 0; m < NC; ++m) F[m][NF - 1] = face_n[m][r];
+        }
+    };
+    auto flux_above = [&] (R own, const R (&F)[NC][NF], int m) -> R {
+        if constexpr (kQueue) {
+            // wave_shl:1, the last lane of the wave keeps the first operand
+            static_assert(sizeof(R) == 4, "one register");
+            return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(F[m][t / 64 + 1]), __float_as_int(own),
+                                                              0x130, 0xf, 0xf, false));
+        } else {
+            return F[m][t + 1];
+        }
+    };
+
     auto step = [&] (auto do1_c, auto do2_c, auto rot_c, auto fetch_c, int s) {
         constexpr bool DO1 = decltype(do1_c)::value, DO2 = decltype(do2_c)::value;
         constexpr bool FETCH = decltype(fetch_c)::value;
@@ -291,7 +325,7 @@ rk2_fused_kernel(typename S::Params p1, typename S::Params p2, MeshLoader<S> ld,
         }
         __syncthreads();
         if constexpr (DO1) cons_of(ld.row(b, j) + c, U0j);
-        if constexpr (DO2) cons_of(ld.row(b, k) + c, U0k);
+        if constexpr (DO2 && !kQueue) cons_of(ld.row(b, k) + c, U0k);
         // phase B: y half slopes (own column and the left neighbour's), y
         // fluxes at the lower face of each column
         if constexpr (DO1) {
@@ -304,12 +338,7 @@ rk2_fused_kernel(typename S::Params p1, typename S::Params p2, MeshLoader<S> ld,
                 pr[m] = P1[A][m] - gy1[m];
             }
             S::template face<2>(pl, pr, p1, td, tc, j, c, Fy1);
-#pragma unroll
-            for (int m = 0; m < NC; ++m) rowF1[m][t] = Fy1[m];
-            if (t == TJ - 1) {
-#pragma unroll
-                for (int m = 0; m < NC; ++m) rowF1[m][TJ] = f1e[m][s];
-            }
+            put_flux(Fy1, rowF1, f1e, s);
         }
         if constexpr (DO2) {
             R pl[NC], pr[NC];
@@ -321,12 +350,7 @@ rk2_fused_kernel(typename S::Params p1, typename S::Params p2, MeshLoader<S> ld,
                 pr[m] = P2[A][m] - gy2[m];
             }
             S::template face<2>(pl, pr, p2, td, tc, k, c, Fy2);
-#pragma unroll
-            for (int m = 0; m < NC; ++m) rowF2[m][t] = Fy2[m];
-            if (t == TJ - 1) {
-#pragma unroll
-                for (int m = 0; m < NC; ++m) rowF2[m][TJ] = f2e[m][kl];
-            }
+            put_flux(Fy2, rowF2, f2e, kl);
         }
         __syncthreads();
         // phase C: updates; the second stage reads row k's U1 from the queue
@@ -336,8 +360,9 @@ rk2_fused_kernel(typename S::Params p1, typename S::Params p2, MeshLoader<S> ld,
 #pragma unroll
             for (int m = 0; m < NC; ++m) {
                 dfx[m] = double(F2[B][m]) - double(F2[A][m]);
-                dfy[m] = double(rowF2[m][t + 1]) - double(Fy2[m]);
+                dfy[m] = double(flux_above(Fy2[m], rowF2, m)) - double(Fy2[m]);
                 u1k[m] = u1q[slot][m][t];
+                if constexpr (kQueue) U0k[m] = u0q[slot][m][t];
             }
             S::update(p2, td, tc, k, c, u1k, P2[A], dfx, dfy, dt, dl, res);
             double* o = a.out + ((size_t)b * NC * n + k) * n + c;
@@ -357,12 +382,15 @@ rk2_fused_kernel(typename S::Params p1, typename S::Params p2, MeshLoader<S> ld,
 #pragma unroll
             for (int m = 0; m < NC; ++m) {
                 dfx[m] = double(F1[B][m]) - double(F1[A][m]);
-                dfy[m] = double(rowF1[m][t + 1]) - double(Fy1[m]);
+                dfy[m] = double(flux_above(Fy1[m], rowF1, m)) - double(Fy1[m]);
             }
             S::update(p1, td, tc, j, c, U0j, P1[A], dfx, dfy, dt, dl, u1);
             ok &= S::recover(u1, p2, P2[A]);
 #pragma unroll
-            for (int m = 0; m < NC; ++m) u1q[slot][m][t] = u1[m];
+            for (int m = 0; m < NC; ++m) {
+                u1q[slot][m][t] = u1[m];
+                if constexpr (kQueue) u0q[slot][m][t] = U0j[m];
+            }
         }
     };
     using T_ = std::true_type;

@@ -42,6 +42,7 @@ struct EulerScheme {
     // the fused RK2 step (both stages' windows of five components) at two
     // waves per SIMD: 178 VGPRs, and its 61 KB of LDS fit two workgroups per CU
     static constexpr int kFusedWavesPerEU = 2;
+    static constexpr bool kFusedQueue = false;
     using Real = R;
     using Params = EulerParams;
     __device__ static __forceinline__ double cfl_speed(const double* u, const Params& prm)
@@ -136,17 +137,24 @@ struct MinidiskScheme {
     // stage 1 runs 9 % (mixed) and 2 % (FP64) faster than with one
     static constexpr int prefetch_rows(int) { return 2; }
     static constexpr bool kFirstStage = true;
-    // the fused RK2 step (both stages' windows) at three waves per SIMD
+    // the fused RK2 step (both stages' windows) at three waves per SIMD, with
+    // room in LDS for a queue of U0 rows (rk2fused.hpp)
     static constexpr int kFusedWavesPerEU = 3;
+    static constexpr bool kFusedQueue = true;
     static constexpr bool kCfl = false;
     __device__ static __forceinline__ double cfl_speed(const double*, const MinidiskParams&) { return 0.0; }
     using Real = R;
     using Params = MinidiskParams;
-    // Vertex coordinates of the tile's rows/columns in FP64 (reference formula),
-    // plus FP32 vertex and centre copies for the mixed kernel.
+    // Vertex coordinates of the tile's rows/columns (reference formula), FP64;
+    // the mixed kernels keep FP32 copies of the vertices and centres instead.
     template<int H, int TJ> struct TileData {
-        double xv[H + 1]; double yv[TJ + 1];
-        float xvf[H + 1]; float xcf[H]; float yvf[TJ + 1]; float ycf[TJ];
+        static constexpr bool kD = is_fp64<R>::value;
+        double xv[kD ? H + 1 : 1], yv[kD ? TJ + 1 : 1];
+        float xvf[kD ? 1 : H + 1], xcf[kD ? 1 : H], yvf[kD ? 1 : TJ + 1], ycf[kD ? 1 : TJ];
+        __device__ __forceinline__ void put_x(int t, double v) { if constexpr (kD) xv[t] = v; else xvf[t] = float(v); }
+        __device__ __forceinline__ void put_y(int t, double v) { if constexpr (kD) yv[t] = v; else yvf[t] = float(v); }
+        __device__ __forceinline__ void put_xc(int t, double v) { if constexpr (!kD) xcf[t] = float(v); }
+        __device__ __forceinline__ void put_yc(int t, double v) { if constexpr (!kD) ycf[t] = float(v); }
     };
 
     // theta = 2 is hard-coded by the reference (problems/minidisk_scheme.cpp:313-314)
@@ -180,15 +188,13 @@ struct MinidiskScheme {
     {
         for (int t = threadIdx.x; t <= H; t += blockDim.x) {
             double v = vertex(prm.R, tc.n, prm.level, tc.bi, tc.k0 + t);
-            td.xv[t] = v;
-            td.xvf[t] = float(v);
-            if (t < H) td.xcf[t] = float(0.5 * (v + vertex(prm.R, tc.n, prm.level, tc.bi, tc.k0 + t + 1)));
+            td.put_x(t, v);
+            if (t < H) td.put_xc(t, 0.5 * (v + vertex(prm.R, tc.n, prm.level, tc.bi, tc.k0 + t + 1)));
         }
         for (int t = threadIdx.x; t <= TJ; t += blockDim.x) {
             double v = vertex(prm.R, tc.n, prm.level, tc.bj, tc.c0 + t);
-            td.yv[t] = v;
-            td.yvf[t] = float(v);
-            if (t < TJ) td.ycf[t] = float(0.5 * (v + vertex(prm.R, tc.n, prm.level, tc.bj, tc.c0 + t + 1)));
+            td.put_y(t, v);
+            if (t < TJ) td.put_yc(t, 0.5 * (v + vertex(prm.R, tc.n, prm.level, tc.bj, tc.c0 + t + 1)));
         }
     }
 
@@ -207,36 +213,31 @@ struct MinidiskScheme {
             const int ob = v < 0 ? bi_m : (v > n ? bi_p : tc.bi);
             const int vl = v < 0 ? v + n : (v > n ? v - n : v);
             const double x = vertex(prm.R, n, prm.level, ob, vl);
-            td.xv[t] = x;
-            td.xvf[t] = float(x);
+            td.put_x(t, x);
             if (t < H) {
                 const int rb = v < 0 ? bi_m : (v >= n ? bi_p : tc.bi);
                 const int rl = v < 0 ? v + n : (v >= n ? v - n : v);
-                td.xcf[t] = float(0.5 * (vertex(prm.R, n, prm.level, rb, rl) + vertex(prm.R, n, prm.level, rb, rl + 1)));
+                td.put_xc(t, 0.5 * (vertex(prm.R, n, prm.level, rb, rl) + vertex(prm.R, n, prm.level, rb, rl + 1)));
             }
         }
         for (int t = threadIdx.x; t <= TJ; t += blockDim.x) {
             double v = vertex(prm.R, tc.n, prm.level, tc.bj, tc.c0 + t);
-            td.yv[t] = v;
-            td.yvf[t] = float(v);
-            if (t < TJ) td.ycf[t] = float(0.5 * (v + vertex(prm.R, tc.n, prm.level, tc.bj, tc.c0 + t + 1)));
+            td.put_y(t, v);
+            if (t < TJ) td.put_yc(t, 0.5 * (v + vertex(prm.R, tc.n, prm.level, tc.bj, tc.c0 + t + 1)));
         }
     }
 
     // One zone's TileData (k0 = row, c0 = column): the per-zone kernels.
     __device__ static __forceinline__ void setup_zone(TileData<1, 1>& td, const Params& prm, const TileCtx& tc)
     {
-#pragma unroll
-        for (int t = 0; t <= 1; ++t) {
-            double v = vertex(prm.R, tc.n, prm.level, tc.bi, tc.k0 + t);
-            td.xv[t] = v;
-            td.xvf[t] = float(v);
-            double w = vertex(prm.R, tc.n, prm.level, tc.bj, tc.c0 + t);
-            td.yv[t] = w;
-            td.yvf[t] = float(w);
-        }
-        td.xcf[0] = float(0.5 * (td.xv[0] + td.xv[1]));
-        td.ycf[0] = float(0.5 * (td.yv[0] + td.yv[1]));
+        const double x0 = vertex(prm.R, tc.n, prm.level, tc.bi, tc.k0), x1 = vertex(prm.R, tc.n, prm.level, tc.bi, tc.k0 + 1);
+        const double y0 = vertex(prm.R, tc.n, prm.level, tc.bj, tc.c0), y1 = vertex(prm.R, tc.n, prm.level, tc.bj, tc.c0 + 1);
+        td.put_x(0, x0);
+        td.put_x(1, x1);
+        td.put_y(0, y0);
+        td.put_y(1, y1);
+        td.put_xc(0, 0.5 * (x0 + x1));
+        td.put_yc(0, 0.5 * (y0 + y1));
     }
 
     // sound_speed_squared :127-132 at face_coordinates :134-151
@@ -348,38 +349,43 @@ struct MinidiskScheme {
             float sig = pc[0];
             float ax = fmaf(g1, dx1, fmaf(g2, dx2, fmaf(om * om, xf, 2.0f * om * pc[2])));
             float ay = fmaf(g1, dy1, fmaf(g2, dy2, fmaf(om * om, yf, -2.0f * om * pc[1])));
-            // Sink and buffer terms are evaluated only where they are not
-            // negligible (skipped wave-uniformly elsewhere): the sink
+            // Sink and buffer terms are evaluated and applied only where they
+            // are not negligible (skipped wave-uniformly elsewhere): the sink
             // exp(-q^3 / r_sink^6) is below 1e-45 once its argument passes
             // 104, and the buffer rate is below 4e-18 of its maximum once
             // (r - R) / scale < -20.  The initial state U_init enters only the
             // buffer term.
-            float sr = 0.0f;
-            if (fminf(q1, q2) < float(prm.q_sink_cut)) {
-                float is6 = float(prm.inv_s6);
-                float t1 = q1 * q1 * q1 * is6, t2 = q2 * q2 * q2 * is6;
-                sr = float(prm.sink_rate) * (__expf(-t1) + __expf(-t2));
-            }
             float q0 = fmaf(xf, xf, yf * yf);
             float ir0 = __builtin_amdgcn_rsqf(q0);
             float rr = q0 * ir0;
             float yb = (rr - float(prm.R)) * float(prm.inv_buffer_scale);
-            float br = 0.0f, ui[3] = { 1.0f, 0.0f, 0.0f };
-            if (yb > -20.0f) {
-                // 0.5 * rate * (1 + tanh(y)) = rate / (1 + exp(-2y))
-                br = float(prm.buffer_rate) * __builtin_amdgcn_rcpf(1.0f + __expf(-2.0f * yb));
-                float ph = __builtin_amdgcn_rsqf(q0 + s2);
-                float vp = __builtin_amdgcn_sqrtf(ph) - om * rr;
-                ui[1] = vp * (-yf * ir0);
-                ui[2] = vp * (xf * ir0);
-            }
-            float sa[3] = { 0.0f, sig * ax, sig * ay };
+            const bool sink = fminf(q1, q2) < float(prm.q_sink_cut);
+            float src[3] = { 0.0f, sig * ax, sig * ay };
             double dtdl = dt / dl;
 #pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                float src = sa[q] - float(u[q]) * sr - float(u[q] - double(ui[q])) * br;
-                out[q] = fma(double(src), dt, fma(-(dfx[q] + dfy[q]), dtdl, u[q]));
+            for (int q = 0; q < 3; ++q) out[q] = fma(-(dfx[q] + dfy[q]), dtdl, u[q]);
+            if (sink || yb > -20.0f) {
+                float sr = 0.0f, br = 0.0f, ui[3] = { 1.0f, 0.0f, 0.0f };
+                if (sink) {
+                    float is6 = float(prm.inv_s6);
+                    float t1 = q1 * q1 * q1 * is6, t2 = q2 * q2 * q2 * is6;
+                    sr = float(prm.sink_rate) * (__expf(-t1) + __expf(-t2));
+                }
+                if (yb > -20.0f) {
+                    // 0.5 * rate * (1 + tanh(y)) = rate / (1 + exp(-2y))
+                    br = float(prm.buffer_rate) * __builtin_amdgcn_rcpf(1.0f + __expf(-2.0f * yb));
+                    float ph = __builtin_amdgcn_rsqf(q0 + s2);
+                    float vp = __builtin_amdgcn_sqrtf(ph) - om * rr;
+                    ui[1] = vp * (-yf * ir0);
+                    ui[2] = vp * (xf * ir0);
+                }
+#pragma unroll
+                for (int q = 0; q < 3; ++q)
+                    src[q] = src[q] - float(u[q]) * sr - float(u[q] - double(ui[q])) * br;
+                out[0] = fma(double(src[0]), dt, out[0]);
             }
+#pragma unroll
+            for (int q = 1; q < 3; ++q) out[q] = fma(double(src[q]), dt, out[q]);
         }
     }
 };

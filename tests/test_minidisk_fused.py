@@ -46,7 +46,7 @@ def test_fused_rk2_equals_two_stages(n, depth):
     assert np.array_equal(ua, ub), float(np.abs(ua - ub).max())
 
 
-@pytest.mark.parametrize("n, depth", [(128, 3), (64, 4), (256, 2), (64, 5), (128, 4)])
+@pytest.mark.parametrize("n, depth", [(128, 3), (64, 4), (256, 2), (256, 3), (64, 5), (128, 4)])
 def test_fused_rk2_rows_by_mesh_size(n, depth):
     """Meshes on both sides of each line of the rows-by-size rule, in every
     block size: one step, equal in every value to two stage launches."""
