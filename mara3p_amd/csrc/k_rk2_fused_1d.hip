@@ -8,25 +8,14 @@ namespace m3p {
 int launch_rk2_fused_1d(const EulerParams& prm, const Stage1DArgs& a, hipStream_t s)
 {
     const int n = a.n;
-    // one workgroup per (block, tile) item; the kernel is small (about 5 KB
-    // of LDS at TJ = 64), so many workgroups share a CU and hide each
-    // other's load latency
-    auto go = [&] (auto kern, int TJ) {
-        const long items = (long)a.nblk * (n / TJ);
-        if (items > INT_MAX) return fail(M3P_ERR_BAD_SHAPE, "m3p: too many 1D blocks for one launch");
-        hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(TJ), 0, s, prm, a);
-        return launch_status("rk2_fused_1d_kernel");
-    };
-    switch (n) {
-        case 16:  return go(rk2_fused_1d_kernel<16>, 16);
-        case 32:  return go(rk2_fused_1d_kernel<32>, 32);
-        case 64:  return go(rk2_fused_1d_kernel<64>, 64);
-        case 128: return go(rk2_fused_1d_kernel<128>, 128);
-        default:
-            if (n >= 256 && n % 256 == 0) return go(rk2_fused_1d_kernel<256>, 256);
-    }
-    return fail(M3P_ERR_BAD_SHAPE, "m3p: 1D block size must be 16, 32, 64, 128 or a multiple of 256 (got " +
-                                   std::to_string(n) + ")");
+    if (n != 16 && n != 32 && n != 64 && n != 128 && (n < 256 || n % 256 != 0))
+        return fail(M3P_ERR_BAD_SHAPE, "m3p: 1D block size must be 16, 32, 64, 128 or a multiple of 256 (got " +
+                                       std::to_string(n) + ")");
+    constexpr long zones = (long)kWindow1D * kWindowGroup;
+    const long groups = ((long)a.nblk * n + zones - 1) / zones;
+    if (groups > INT_MAX) return fail(M3P_ERR_BAD_SHAPE, "m3p: too many 1D blocks for one launch");
+    hipLaunchKernelGGL(rk2_fused_1d_kernel, dim3((unsigned)groups), dim3(64 * kWindowGroup), 0, s, prm, a);
+    return launch_status("rk2_fused_1d_kernel");
 }
 
 } // namespace m3p

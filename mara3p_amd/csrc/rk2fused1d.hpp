@@ -4,187 +4,179 @@
 // The two-stage form (stage1d_kernel twice) writes U1 = L(U0) for every block
 // and reads it back, with its guard zones, for U = b U0 + (1 - b) L(U1)
 // (modules::euler1d::updated_conserved, src/module_euler.cpp:107-135, per
-// stage; outflow ends, src/mara.cpp:123-143).  Here a workgroup of TJ lanes
-// owns TJ zones c0 .. c0 + TJ - 1 of one block.  It loads U0 on zones
-// c0 - 4 .. c0 + TJ + 3, computes the first stage on zones c0 - 2 ..
-// c0 + TJ + 1 (its own zones and the two on each side that the second stage
-// reads), keeps U1's primitives in LDS and its own zones' U1 in registers,
-// then computes the second stage and the RK combine of its own zones.
+// stage; outflow ends, src/mara.cpp:123-143).  Here a wave owns 56 zones,
+// consecutive in storage, and holds them in its lanes 4 .. 59 with the four
+// zones before and after: each lane takes one half slope and one face flux
+// (the left face of its zone) and one update per stage, and gets its
+// neighbours' values by wave shifts.  Each stage leaves two lanes less at each
+// end with the right values, so after two stages lanes 4 .. 59 have theirs.
+// Nothing passes through LDS and nothing waits at a barrier.
 //
-// Every U1 value is the one the two-stage path computes: a zone of the
-// neighbouring block is updated with that block's cell spacing from the same
-// operands (the neighbour's guard zones are this block's zones, which needs
-// the prev/next links to be mutual: block pb = prev(b) has next(pb) = b, and
-// likewise for next, as in every chain and ring; a table where they are not
-// is reported through the error latch with code M3P_ERR_BAD_SHAPE).  At an
-// outflow end the second stage's guard zones copy U1 of the edge zone, as the
-// two-stage guard fill copies it, instead of being updated.  So the step
-// equals two stage1d launches value for value; HBM sees U0 (and eight guard
-// zones per TJ zones) and U once, instead of U0, U1, U1, U0 and U.
+// A workgroup per 64-zone block, a lane per zone, needed 69 and 65 faces of 64
+// lanes in the two stages, two nearly empty passes out of four, took two
+// slopes per face and met four barriers.  512 problems of 512 to 8192 zones in
+// blocks of 64: 55 to 47 us a step (553 VALU instructions per 56 zones, 965 per
+// 64 before; 190 MB, 4.0 TB/s), with the CFL reduction at half that size 52 to
+// 36, 300 problems in blocks of 16 16.7 to 8.9.  One-wave workgroups: 48 us,
+// with the CFL reduction 48.
+//
+// Zones of a window are one chain where every block boundary in it joins
+// blocks that are linked and consecutive in storage (nearly always).  Else the
+// window is done in pieces, each piece's lanes finding their zones along the
+// prev/next links from the piece's first zone: a neighbour stored elsewhere,
+// or, past an outflow end, a copy of the edge zone, whose lanes take the edge
+// zone's U1 in the second stage as the two-stage guard fill does.
+//
+// Every U1 value is the one the two-stage path computes: a zone of another
+// block is updated with that block's cell spacing from the same operands (its
+// guard zones are this chain's zones, which needs the prev/next links to be
+// mutual: block pb = prev(b) has next(pb) = b, and likewise for next, as in
+// every chain and ring; a table where they are not is reported through the
+// error latch with code M3P_ERR_BAD_SHAPE, and such an end is treated as
+// outflow).  So the step equals two stage1d launches value for value; HBM sees
+// U0 and U once, instead of U0, U1, U1, U0 and U.
 #pragma once
 #include "stage1d.hpp"
 
 namespace m3p {
 
-template<int TJ>
-__global__ void __launch_bounds__(TJ)
+constexpr int kWindow1D = 56;          // zones a wave updates
+constexpr int kWindowGroup = 4;        // waves of a workgroup
+
+// the value of the lane before / after (the first / last lane keeps its own)
+__device__ __forceinline__ float lane_before(float x)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(x), __float_as_int(x), 0x138 /* wave_shr:1 */,
+                                                      0xf, 0xf, false));
+}
+__device__ __forceinline__ float lane_after(float x)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(x), __float_as_int(x), 0x130 /* wave_shl:1 */,
+                                                      0xf, 0xf, false));
+}
+
+static __global__ void __launch_bounds__(64 * kWindowGroup)
 rk2_fused_1d_kernel(EulerParams prm, Stage1DArgs a)
 {
     using R = float;
     constexpr int NC = 5;
-    static_assert(TJ >= 8, "eight guard lanes");
     const int n = a.n;
-    const int tiles = n / TJ;
-    const int b = (int)(blockIdx.x / tiles);
-    const int c0 = (int)(blockIdx.x % tiles) * TJ;
-    const int t = threadIdx.x;
+    const int i = threadIdx.x & 63;
+    const long total = (long)a.nblk * n;
+    const long first = ((long)blockIdx.x * kWindowGroup + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * kWindow1D;
+    const long end = first + kWindow1D < total ? first + kWindow1D : total;
     const R theta = R(prm.theta);
     const double dt = a.dt_dev ? *a.dt_dev : a.dt;
-    const int pb = a.nbr[2 * b], nb = a.nbr[2 * b + 1];
-    const bool lo_edge = c0 == 0, hi_edge = c0 + TJ == n;
-    const bool lo_out = lo_edge && pb < 0, hi_out = hi_edge && nb < 0;
-    if ((lo_edge && pb >= 0 && a.nbr[2 * pb + 1] != b) || (hi_edge && nb >= 0 && a.nbr[2 * nb] != b)) {
-        if (t == 0) report_error(a.err, 4, b, lo_edge && pb >= 0 && a.nbr[2 * pb + 1] != b ? -1 : n);
-        return;
-    }
-    const double dl = a.dl_blk ? a.dl_blk[b] : a.dl;
-    // the cell spacing of the neighbours whose edge zones this tile updates
-    // in the first stage, loaded here rather than after a barrier, where
-    // its latency held up the workgroup (launch 2 % faster)
-    const double dl_lo = lo_edge && pb >= 0 && a.dl_blk ? a.dl_blk[pb] : dl;
-    const double dl_hi = hi_edge && nb >= 0 && a.dl_blk ? a.dl_blk[nb] : dl;
+    double rate = 0.0;                      // fused CFL reduction
 
-    __shared__ R P0[NC][TJ + 8];   // [i] = zone c0 - 4 + i: U0 primitives
-    __shared__ R F1[NC][TJ + 5];   // [i] = face c0 - 2 + i (the left face of zone c0 - 2 + i): first stage
-    __shared__ R P1[NC][TJ + 4];   // [i] = zone c0 - 2 + i: U1 primitives
-    __shared__ R F2[NC][TJ + 1];   // [i] = face c0 + i: second stage
-
-    // zone i in [-4, 0) or [n, n + 4) of block b: the neighbour's zone, or
-    // the edge zone at an outflow end (the stage kernel's guard fill)
-    auto zone_ptr = [&] (int i) {
-        int bb = b, z = i;
-        if (i < 0)       { if (pb < 0) z = 0;     else { bb = pb; z = i + n; } }
-        else if (i >= n) { if (nb < 0) z = n - 1; else { bb = nb; z = i - n; } }
-        return a.u + (size_t)bb * NC * n + z;
-    };
-    // guard lane g (t < 8): zone c0 - 4 + g, or c0 + TJ + g - 4
-    const int gz_zone = t < 4 ? c0 - 4 + t : c0 + TJ + (t - 4);
-    const int gz_slot = t < 4 ? t : TJ + 4 + (t - 4);
-
-    bool ok = true;
-    double u0[NC], gu0[NC];
-    {
-        const double* src = a.u + (size_t)b * NC * n + c0 + t;
+    for (long lo = first; lo < end;) {
+        // block and zone of lo, then of each lane along the storage order
+        const int b0 = total < (1l << 31) ? (int)((unsigned)lo / (unsigned)n) : (int)(lo / n);
+        const int p0 = (int)(lo - (long)b0 * n) + i - 4;      // the lane's zone counted from block b0's first
+        int b = b0, z = p0;
+        while (z >= n) { ++b; z -= n; }
+        if (z < 0) { --b; z += n; }
+        const bool inside = lo >= 4 && lo + 60 <= total;
+        int prev = b - 1, next = b;                           // the links across the boundary before the lane's zone
+        if (inside && i > 0 && z == 0) { prev = a.nbr[2 * b]; next = a.nbr[2 * (b - 1) + 1]; }
+        // the state is fetched before the links are known (the latencies
+        // overlap), and again by the pieces that do not follow the storage
+        double u0[NC];
+        auto fetch = [&] () {
+            const double* src = a.u + (size_t)b * NC * n + z;
 #pragma unroll
-        for (int q = 0; q < NC; ++q) u0[q] = src[(size_t)q * n];
-        if (t < 8) {
-            const double* g = zone_ptr(gz_zone);
-#pragma unroll
-            for (int q = 0; q < NC; ++q) gu0[q] = g[(size_t)q * n];
+            for (int q = 0; q < NC; ++q) u0[q] = src[(size_t)q * n];
+        };
+        double dl = a.dl;
+        if (inside) {
+            fetch();
+            if (a.dl_blk) dl = a.dl_blk[b];
         }
-        R p[NC];
-        ok &= Euler<R>::recover(u0, prm, p);
-#pragma unroll
-        for (int q = 0; q < NC; ++q) P0[q][t + 4] = p[q];
-        if (t < 8) {
-            ok &= Euler<R>::recover(gu0, prm, p);
-#pragma unroll
-            for (int q = 0; q < NC; ++q) P0[q][gz_slot] = p[q];
+        int count = (int)(end - lo);                          // zones this piece updates
+        unsigned long long low = 0, high = 0;                 // lanes past an outflow end
+        if (__builtin_expect(__ballot(inside && prev == b - 1 && next == b) != ~0ull, 0)) {
+            b = b0;
+            z = p0;
+            bool out_lo = false, out_hi = false;
+            if (z < 0) {
+                const int pb = a.nbr[2 * b];
+                const bool mutual = pb < 0 || a.nbr[2 * pb + 1] == b;
+                if (!mutual) report_error(a.err, 4, b, -1);
+                if (pb >= 0 && mutual) { b = pb; z += n; }
+                else { z = 0; out_lo = true; }
+            }
+            while (z >= n) {
+                const int nb = a.nbr[2 * b + 1];
+                const bool mutual = nb < 0 || a.nbr[2 * nb] == b;
+                if (!mutual) report_error(a.err, 4, b, n);
+                if (nb >= 0 && mutual) { b = nb; z -= n; }
+                else { z = n - 1; out_hi = true; }
+            }
+            low = __ballot(out_lo);
+            high = __ballot(out_hi);
+            // the piece ends at the first lane whose zone is not the storage's
+            const unsigned long long other = __ballot(i >= 4 && (out_hi || (long)b * n + z != lo + (i - 4)));
+            if (other) count = min(count, __builtin_ctzll(other) - 4);
+            fetch();
+            if (a.dl_blk) dl = a.dl_blk[b];
         }
-    }
-    __syncthreads();
+        const bool mine = i >= 4 && i < 4 + min(count, kWindow1D);
+        const double dtdl = dt / dl;
+        double u1[NC];
+        R p[NC], f[NC];
 
-    // first stage, faces c0 - 2 .. c0 + TJ + 2: face i from zones i .. i + 3
-    // of the P0 row, with the operands and order of stage1d_kernel's faces
-    auto face1 = [&] (int i) {
-        R pl[NC], pr[NC], f[NC];
+        // the left face of the lane's zone, from the half slopes of this zone
+        // and the one before, with the operands and order of stage1d_kernel
+        auto face = [&] () {
+            R pl[NC], pr[NC];
 #pragma unroll
-        for (int q = 0; q < NC; ++q) {
-            pl[q] = P0[q][i + 1] + plm_half(P0[q][i], P0[q][i + 1], P0[q][i + 2], theta);
-            pr[q] = P0[q][i + 2] - plm_half(P0[q][i + 1], P0[q][i + 2], P0[q][i + 3], theta);
-        }
-        Euler<R>::template riemann<1>(pl, pr, prm, f);
-#pragma unroll
-        for (int q = 0; q < NC; ++q) F1[q][i] = f[q];
-    };
-    face1(t);
-    if (t < 5) face1(TJ + t);
-    __syncthreads();
+            for (int q = 0; q < NC; ++q) {
+                const R g = plm_half(lane_before(p[q]), p[q], lane_after(p[q]), theta);
+                pl[q] = lane_before(p[q] + g);
+                pr[q] = p[q] - g;
+            }
+            Euler<R>::template riemann<1>(pl, pr, prm, f);
+        };
+        auto flux_difference = [&] (int q) { return double(lane_after(f[q])) - double(f[q]); };
 
-    // first-stage update of zone c0 - 2 + j with the cell spacing of its block
-    auto update1 = [&] (int j, const double* uz, double dlz, double* u1) {
+        bool ok = Euler<R>::recover(u0, prm, p);
+        face();
 #pragma unroll
-        for (int q = 0; q < NC; ++q) {
-            const double dfx = double(F1[q][j + 1]) - double(F1[q][j]);
-            u1[q] = uz[q] - dfx * (dt / dlz);
-        }
-    };
-    double u1[NC];
-    {
-        update1(t + 2, u0, dl, u1);
-        R p[NC];
+        for (int q = 0; q < NC; ++q) u1[q] = u0[q] - flux_difference(q) * dtdl;
         ok &= Euler<R>::recover(u1, prm, p);
+        if (low) {          // the lanes below take the edge zone's, the first lane of the chain
+            const int e = 64 - __builtin_clzll(low);
 #pragma unroll
-        for (int q = 0; q < NC; ++q) P1[q][t + 2] = p[q];
-        // outflow ends: the second stage's guard zones copy the edge zone
-        if (t == 0 && lo_out) {
-#pragma unroll
-            for (int q = 0; q < NC; ++q) { P1[q][0] = p[q]; P1[q][1] = p[q]; }
+            for (int q = 0; q < NC; ++q) {
+                const R v = __shfl(p[q], e, 64);
+                if (i < e) p[q] = v;
+            }
         }
-        if (t == TJ - 1 && hi_out) {
+        if (high) {         // and those above the last lane's
+            const int e = __builtin_ctzll(high) - 1;
 #pragma unroll
-            for (int q = 0; q < NC; ++q) { P1[q][TJ + 2] = p[q]; P1[q][TJ + 3] = p[q]; }
+            for (int q = 0; q < NC; ++q) {
+                const R v = __shfl(p[q], e, 64);
+                if (i > e) p[q] = v;
+            }
         }
-        // lanes 2, 3 (zones c0 - 2, c0 - 1) and 4, 5 (zones c0 + TJ, c0 + TJ + 1)
-        // update the guard zones they loaded, unless at an outflow end
-        const bool lo_x = (t == 2 || t == 3) && !lo_out;
-        const bool hi_x = (t == 4 || t == 5) && !hi_out;
-        if (lo_x || hi_x) {
-            const int j = lo_x ? t - 2 : TJ + (t - 2);
-            const double dlz = lo_x ? dl_lo : dl_hi;
-            double g1[NC];
-            update1(j, gu0, dlz, g1);
-            ok &= Euler<R>::recover(g1, prm, p);
-#pragma unroll
-            for (int q = 0; q < NC; ++q) P1[q][j] = p[q];
-        }
-    }
-    __syncthreads();
-
-    // second stage, faces c0 .. c0 + TJ: lane t the right face of its zone
-    // (P1 zones t + 1 .. t + 4), lane 0 also the left face of the tile
-    auto face2 = [&] (int i) {
-        R pl[NC], pr[NC], f[NC];
+        face();
+        double wv[NC];
 #pragma unroll
         for (int q = 0; q < NC; ++q) {
-            pl[q] = P1[q][i + 1] + plm_half(P1[q][i], P1[q][i + 1], P1[q][i + 2], theta);
-            pr[q] = P1[q][i + 2] - plm_half(P1[q][i + 1], P1[q][i + 2], P1[q][i + 3], theta);
+            const double res = u1[q] - flux_difference(q) * dtdl;
+            wv[q] = u0[q] * a.rk_b + res * (1.0 - a.rk_b);
         }
-        Euler<R>::template riemann<1>(pl, pr, prm, f);
+        if (mine) {
+            double* o = a.out + (size_t)b * NC * n + z;
 #pragma unroll
-        for (int q = 0; q < NC; ++q) F2[q][i] = f[q];
-    };
-    face2(t + 1);
-    if (t == 0) face2(0);
-    __syncthreads();
-
-    // second-stage update and the RK combine (stage1d_kernel's arithmetic)
-    const int z = c0 + t;
-    double* o = a.out + (size_t)b * NC * n + z;
-    double wv[NC];
-#pragma unroll
-    for (int q = 0; q < NC; ++q) {
-        const double dfx = double(F2[q][t + 1]) - double(F2[q][t]);
-        double res = u1[q] - dfx * (dt / dl);
-        res = u0[q] * a.rk_b + res * (1.0 - a.rk_b);
-        o[(size_t)q * n] = res;
-        wv[q] = res;
+            for (int q = 0; q < NC; ++q) o[(size_t)q * n] = wv[q];
+            if (!ok) report_error(a.err, 1, b, z);
+            if (a.rate_slot) rate = fmax(rate, Euler<double>::max_speed(wv, prm) * (1.0 / dl));
+        }
+        lo += count;
     }
-    if (!ok) report_error(a.err, 1, b, z);
-    if (a.rate_slot) {
-        const double idl = 1.0 / dl;
-        workgroup_atomic_max<TJ>(Euler<double>::max_speed(wv, prm) * idl, a.rate_slot);
-    }
+    if (a.rate_slot) workgroup_atomic_max<64 * kWindowGroup>(rate, a.rate_slot);
 }
 
 } // namespace m3p

@@ -114,6 +114,51 @@ def test_fused_rk2_cfl_graph_replays_match_eager_separate():
     del g
 
 
+@pytest.mark.parametrize("n", [16, 32, 64, 128, 256])
+@pytest.mark.parametrize("order", ["storage", "reversed", "shuffled"])
+def test_fused_rk2_windows_follow_the_links(n, order):
+    """Windows of 56 zones over tables whose links leave the storage order:
+    chains of two to nine blocks (shorter and longer than a window), rings of
+    one and three blocks, their blocks stored in order, backwards and shuffled,
+    each with its own cell spacing.  Equal in every value to two stage
+    launches, and the CFL form to the separate reduction."""
+    from mara3p_amd.mesh import EnsembleMesh1D
+    from mara3p_amd.solvers import Euler1DEnsembleSolver
+    rng = np.random.default_rng(n)
+    chains, rings = [2, 9, 3, 2, 5], [1, 3]
+    total = sum(chains) + sum(rings)
+    where = {"storage": np.arange(total), "reversed": np.arange(total)[::-1], "shuffled": rng.permutation(total)}[order]
+    nbr, dl, first = np.full((total, 2), -1, np.int32), np.empty(total), 0
+    for m, ring in [(m, False) for m in chains] + [(m, True) for m in rings]:
+        for k in range(m):
+            b = where[first + k]
+            if k > 0 or ring:
+                nbr[b, 0] = where[first + (k - 1) % m]
+            if k < m - 1 or ring:
+                nbr[b, 1] = where[first + (k + 1) % m]
+            dl[b] = 1.0 / (m * n)
+        first += m
+    s = Euler1DEnsembleSolver(EnsembleMesh1D([total * n], n), precision="mixed")
+    s.nbr.copy_(torch.as_tensor(nbr))
+    s.dl.copy_(torch.as_tensor(dl))
+    rho, v, p = 1.0 + rng.random((total, n)), 0.5 * rng.standard_normal((total, n)), 0.5 + rng.random((total, n))
+    u0 = np.stack([rho, rho * v, 0 * v, 0.1 * rho, 0.5 * rho * (v * v + 0.01) + p / 0.4], axis=1)
+    s.set_state(u0)
+    dt = 0.02 / (9 * n)
+    s.stage(s.u, None, s.u1, dt)
+    s.stage(s.u1, s.u, s.u2, dt)
+    out = torch.empty_like(s.u)
+    dt_next = torch.zeros(1, dtype=torch.float64, device="cuda")
+    s.rk2_step(s.u, out, dt)
+    assert torch.equal(out, s.u2)
+    out.zero_()
+    s.rk2_step(s.u, out, dt, cfl=0.4, dt_next=dt_next)
+    s.check_errors()
+    assert torch.equal(out, s.u2)
+    s.u = out
+    assert float(dt_next.item()) == float(s.cfl_dt(0.4).item())
+
+
 def test_fused_rk2_refuses_what_it_does_not_compute():
     """FP64, a block size outside the list and aliasing are refused before
     any launch; a one-block problem (prev outflow, next itself: links that
