@@ -226,11 +226,13 @@ bool tile_fits(TileShape v, int n) { return n % v.tj == 0 && n % v.h == 0 && v.h
 // four rows, 92 with sixteen), four rows up to 2048 waves of eight, then eight
 // (1024^2 zones in 64^2 blocks: FP64 80 us against 100 with sixteen rows,
 // mixed 47 against 65).  Meshes of 4096 waves of sixteen rows or more take
-// the wide tiles where they fit (4096^2 in 256^2 blocks, FP64: 1026 us against
-// 1076 with 64 x 8), else stay at eight (2048^2 in 64^2 blocks, FP64: 266 us
-// against 312 with sixteen; quad-tree of 1408 leaves, mixed: 223 against
-// 233), but for the FP64 minidisk from 8192 waves on (4096^2 in 64^2 blocks:
-// 806 us with sixteen, 841 with eight).
+// the wide tiles where they fit, in FP64 from 8192 waves on (256^2 blocks,
+// FP64 HLLC, 4096^2: 993 us against 1055 with 64 x 8, 2048^2: 274 against 264;
+// minidisk, 2048^2: 198 against 187; mixed HLLC, 4096^2: 655 against 690), else
+// stay at eight (2048^2 in 64^2 blocks, FP64: 266 us against 312 with sixteen;
+// quad-tree of 1408 leaves, mixed: 223 against 233), but for the FP64 minidisk
+// from 8192 waves on (4096^2 in 64^2 blocks: 806 us with sixteen, 841 with
+// eight).
 TileShape pick_tile(int kind, int precision, int n, int nblk)
 {
     const int chosen = g_tile[kind][precision].load(std::memory_order_relaxed);
@@ -239,7 +241,7 @@ TileShape pick_tile(int kind, int precision, int n, int nblk)
     auto waves = [&] (int rows) { return zones / (64.0 * rows); };
     int rows = waves(16) >= 4096 ? 16 : waves(8) >= 2048 ? 8 : waves(4) >= 2048 ? 4 : 2;
     if (rows == 16 && kind != M3P_KIND_AMR_EULER2D) {
-        if (tile_fits(kLargeTile[kind], n)) return kLargeTile[kind];
+        if (tile_fits(kLargeTile[kind], n) && (precision == M3P_MIXED || waves(16) >= 8192)) return kLargeTile[kind];
         if (precision == M3P_MIXED && n % 128 == 0) return {128, 32};     // 153 us against 163 (64 x 8) at 2048^2
     }
     if (n % 64 == 0) {

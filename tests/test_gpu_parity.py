@@ -263,7 +263,7 @@ def test_quotients_by_one_denominator(lo, hi):
 
 
 @pytest.mark.parametrize("n, depth", [(16, 0), (16, 5), (32, 1), (32, 5), (48, 1), (64, 0), (64, 3), (64, 4), (64, 5),
-                                      (96, 2), (128, 4), (192, 1), (192, 3)])
+                                      (96, 2), (128, 4), (192, 1), (192, 3), (256, 3)])
 def test_tile_of_each_mesh_size(n, depth):
     """The tile that the library picks by the size of the mesh (block sizes of
     each width, meshes on both sides of each line of the rule): FP64 equals
