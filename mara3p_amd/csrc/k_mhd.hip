@@ -13,8 +13,16 @@ long mhd_workspace_bytes(int N, int precision)
     return (8 * N3 + 3 * 2 * nf) * rs + 8 * kMhdPrimGroups + 8 + 2 * 256;
 }
 
-template<typename R>
-int mhd_advance(MhdArgs a, char* work, hipStream_t s)
+// The three states of an RK2 step (64 B a cell each) are larger than the
+// 256 MB memory-side cache.  Non-temporal accesses then, for what a pass
+// touches once: a step of 256^3 mixed 2625 us to 2470 (FP64 3995 to 3930),
+// 160^3 664 to 616, 128^3 343 to 301 (553 to 530), 112^3 245 to 242 (407 to
+// 394); below the line the next pass would find them in cache, and 100^3 took
+// 201 us instead of 191 (332 instead of 313), 96^3 160 instead of 154.
+static bool mhd_streams(int N) { return 3 * 64 * (long)N * N * N > 256l << 20; }
+
+template<typename R, bool NT>
+static int mhd_advance_as(MhdArgs a, char* work, hipStream_t s)
 {
     const int N = a.N;
     const long N3 = (long)N * N * N, nf = (long)(N + 1) * N * N;
@@ -27,7 +35,7 @@ int mhd_advance(MhdArgs a, char* work, hipStream_t s)
     if (!a.dt) a.dt = a.vmax + kMhdPrimGroups;
     const int gc = (int)((N3 + 255) / 256);
     a.nvmax = std::min(gc, kMhdPrimGroups);
-    hipLaunchKernelGGL(mhd_prim_kernel<R>, dim3(a.nvmax), dim3(256), 0, s, a, P);
+    hipLaunchKernelGGL((mhd_prim_kernel<R, NT>), dim3(a.nvmax), dim3(256), 0, s, a, P);
     FaceE<R> fe{ E1, E2, E3, N, nf };
     // Column tiles of 8 x 32 columns: fluxes and the conserved update in one
     // pass (16 x 16 tiles 0 to 10 % slower at 64 to 256, 8 x 8 tiles 20 to
@@ -44,8 +52,8 @@ int mhd_advance(MhdArgs a, char* work, hipStream_t s)
         hipLaunchKernelGGL(kern, dim3(cols * ((N + TI - 1) / TI)), dim3(256), 0, s, a,
                            (const typename MhdPrim<R>::V*)P, E1, E2, E3, TI);
     };
-    if (N % 32 == 0) tiles(mhd_tile_kernel<R, 8, 32, false>);
-    else             tiles(mhd_tile_kernel<R, 8, 32, true>);
+    if (N % 32 == 0) tiles(mhd_tile_kernel<R, 8, 32, false, NT>);
+    else             tiles(mhd_tile_kernel<R, 8, 32, true, NT>);
     if (int st = launch_status("mhd_tile_kernel")) return st;
     // The face fields: FP64 by bricks of 4 x 4 x 32 cells where they divide
     // the cube (the step 4.41 ms at 256^3 against 4.71 per cell, 626 us
@@ -54,13 +62,19 @@ int mhd_advance(MhdArgs a, char* work, hipStream_t s)
     // the four faces of an edge re-read come from cache (bricks 0.5 % slower).
     if constexpr (is_fp64<R>::value) {
         if (N % 32 == 0) {
-            hipLaunchKernelGGL((mhd_face_b_brick_kernel<R, 4, 4, 32>), dim3((N / 4) * (N / 4) * (N / 32)), dim3(512),
+            hipLaunchKernelGGL((mhd_face_b_brick_kernel<R, 4, 4, 32, NT>), dim3((N / 4) * (N / 4) * (N / 32)), dim3(512),
                                0, s, a, fe);
             return launch_status("m3p_mhd_advance_ct");
         }
     }
-    hipLaunchKernelGGL(mhd_face_b_kernel<R>, dim3(gc), dim3(256), 0, s, a, fe);
+    hipLaunchKernelGGL((mhd_face_b_kernel<R, NT>), dim3(gc), dim3(256), 0, s, a, fe);
     return launch_status("m3p_mhd_advance_ct");
+}
+
+template<typename R>
+int mhd_advance(MhdArgs a, char* work, hipStream_t s)
+{
+    return mhd_streams(a.N) ? mhd_advance_as<R, true>(a, work, s) : mhd_advance_as<R, false>(a, work, s);
 }
 
 template int mhd_advance<double>(MhdArgs, char*, hipStream_t);

@@ -255,6 +255,24 @@ __device__ __forceinline__ void cell_index(long c, int N, int& i, int& j, int& k
     }
 }
 
+// Conserved values and face fields that a pass touches once.  Where the arrays
+// of a step are far larger than the memory-side cache (NT, mhd_streams) they
+// are loaded and stored non-temporally, which leaves the cache to what the
+// next pass reads back: the primitives, the electric fields and the fields
+// that neighbouring cells share.
+template<bool NT>
+__device__ __forceinline__ double get_once(const double* p)
+{
+    if constexpr (NT) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+template<bool NT>
+__device__ __forceinline__ void put_once(double x, double* p)
+{
+    if constexpr (NT) __builtin_nontemporal_store(x, p);
+    else *p = x;
+}
+
 // 256-cell workgroups of about one plane, a multiple of 8 (xcd_remap_chunk)
 __device__ __forceinline__ int mhd_plane_groups(int N)
 {
@@ -294,7 +312,7 @@ struct MhdPrim {
 // reduces for itself (no slots to clear, no launch for the time step).
 constexpr int kMhdPrimGroups = 2048;
 
-template<typename R>
+template<typename R, bool NT>
 __global__ void __launch_bounds__(256)
 mhd_prim_kernel(MhdArgs a, typename MhdPrim<R>::V* P)
 {
@@ -311,7 +329,7 @@ mhd_prim_kernel(MhdArgs a, typename MhdPrim<R>::V* P)
                         0.5 * (a.b3[((long)i * N + j) * (N + 1) + k] + a.b3[((long)i * N + j) * (N + 1) + k + 1]) };
         double u[5], p[8];
 #pragma unroll
-        for (int q = 0; q < 5; ++q) u[q] = a.uc[q * N3 + c];
+        for (int q = 0; q < 5; ++q) u[q] = get_once<NT>(&a.uc[q * N3 + c]);
         if constexpr (is_fp64<R>::value) {
             int st = mhd_recover<true>(u, b, a.gamma, p);
             if (st) report_error(a.err, st == 1 ? 1 : 2, 0, (int)c);
@@ -371,11 +389,11 @@ mhd_prim_kernel(MhdArgs a, typename MhdPrim<R>::V* P)
 // association order.
 template<typename R> struct MhdTileWaves { static constexpr int value = is_fp64<R>::value ? 2 : 4; };
 
-template<typename R, int TJ, int TK, bool RAGGED>
+template<typename R, int TJ, int TK, bool RAGGED, bool NT>
 __global__ void __launch_bounds__(TJ * TK) __attribute__((amdgpu_waves_per_eu(MhdTileWaves<R>::value, 8)))
 mhd_tile_kernel(MhdArgs a, const typename MhdPrim<R>::V* P, R* E1, R* E2, R* E3, int TI)
 {
-    constexpr int NT = TJ * TK;
+    constexpr int LANES = TJ * TK;
     constexpr int EJ = TJ + 4, EK = TK + 4;
     using Vec = typename MhdPrim<R>::V;
     constexpr int NV = MhdPrim<R>::NV;
@@ -402,10 +420,10 @@ mhd_tile_kernel(MhdArgs a, const typename MhdPrim<R>::V* P, R* E1, R* E2, R* E3,
     __shared__ R F2s[5][TJ + 1][TK];  // y-face fluxes of plane i, faces j0 .. j0 + TJ
     __shared__ R F3s[5][TJ][TK + 1];  // z-face fluxes of plane i, faces k0 .. k0 + TK
 
-    __shared__ double vpart[NT / 64];  // fastest speed, by wave
+    __shared__ double vpart[LANES / 64];  // fastest speed, by wave
     {
         double v = 0.0;
-        for (int r = t; r < a.nvmax; r += NT) v = fmax(v, a.vmax[r]);
+        for (int r = t; r < a.nvmax; r += LANES) v = fmax(v, a.vmax[r]);
         v = wave_max(v);
         if ((t & 63) == 0) vpart[t >> 6] = v;
     }
@@ -464,7 +482,7 @@ mhd_tile_kernel(MhdArgs a, const typename MhdPrim<R>::V* P, R* E1, R* E2, R* E3,
     __syncthreads();
     double vmax = vpart[0];
 #pragma unroll
-    for (int r = 1; r < NT / 64; ++r) vmax = fmax(vmax, vpart[r]);
+    for (int r = 1; r < LANES / 64; ++r) vmax = fmax(vmax, vpart[r]);
     const double dt = a.cfl * a.dl / vmax;
     if (blockIdx.x == 0 && t == 0) *a.dt = dt;
     const double dtdl = dt / a.dl;
@@ -484,7 +502,7 @@ mhd_tile_kernel(MhdArgs a, const typename MhdPrim<R>::V* P, R* E1, R* E2, R* E3,
     // Where every ring cell has a thread of its own (the 8 x 32 tiles): the
     // ring of the next plane is fetched while this plane computes (its load
     // latency off the plane's critical path; 127 VGPRs mixed, 254 FP64).
-    constexpr bool kRingAhead = NH <= NT;
+    constexpr bool kRingAhead = NH <= LANES;
     int hj = 0, hk = 0;
     R Hn[8];
     if constexpr (kRingAhead) {
@@ -507,7 +525,7 @@ mhd_tile_kernel(MhdArgs a, const typename MhdPrim<R>::V* P, R* E1, R* E2, R* E3,
                 if (il + 1 < ni) loadP(cell(i + 1, j0 - 2 + hj, k0 - 2 + hk), Hn);
             }
         } else {
-            for (int r = t; r < NH; r += NT) {
+            for (int r = t; r < NH; r += LANES) {
                 int rj, rk;
                 ring(r, rj, rk);
                 R h[8];
@@ -583,10 +601,10 @@ mhd_tile_kernel(MhdArgs a, const typename MhdPrim<R>::V* P, R* E1, R* E2, R* E3,
         {
             const long c = ((long)i * N + jc) * N + kc;
 #pragma unroll
-            for (int q = 0; q < 5; ++q) ucv[q] = a.uc[q * N3 + c];
+            for (int q = 0; q < 5; ++q) ucv[q] = get_once<NT>(&a.uc[q * N3 + c]);
             if (a.u0) {
 #pragma unroll
-                for (int q = 0; q < 5; ++q) u0v[q] = a.u0[q * N3 + c];
+                for (int q = 0; q < 5; ++q) u0v[q] = get_once<NT>(&a.u0[q * N3 + c]);
             }
         }
         __syncthreads();
@@ -607,7 +625,7 @@ mhd_tile_kernel(MhdArgs a, const typename MhdPrim<R>::V* P, R* E1, R* E2, R* E3,
                     r = fma(-(d1 + d2 + d3), dtdl, ucv[q]);
                     if (a.u0) r = fma(u0v[q], a.rk_b, r * (1.0 - a.rk_b));
                 }
-                a.uo[q * N3 + c] = r;
+                put_once<NT>(r, &a.uo[q * N3 + c]);
             }
         }
         // No third barrier: the next plane writes Pl before its first
@@ -664,7 +682,7 @@ struct FaceE {
     }
 };
 
-template<typename R, int A>
+template<bool NT, typename R, int A>
 __device__ __forceinline__ void mhd_update_face(const MhdArgs& a, const FaceE<R>& fe, double dt, int i, int j, int k)
 {
     const int N = a.N;
@@ -674,27 +692,27 @@ __device__ __forceinline__ void mhd_update_face(const MhdArgs& a, const FaceE<R>
         f = ((long)i * N + j) * N + k;
         cf = (fe.ee3(i, j + 1, k) - fe.ee3(i, j, k)) - (fe.ee2(i, j, k + 1) - fe.ee2(i, j, k));
         b = a.b1[f];
-        if (a.u0) b0 = a.b01[f];
+        if (a.u0) b0 = get_once<NT>(&a.b01[f]);
     } else if (A == 2) {
         f = ((long)i * (N + 1) + j) * N + k;
         cf = (fe.ee1(i, j, k + 1) - fe.ee1(i, j, k)) - (fe.ee3(i + 1, j, k) - fe.ee3(i, j, k));
         b = a.b2[f];
-        if (a.u0) b0 = a.b02[f];
+        if (a.u0) b0 = get_once<NT>(&a.b02[f]);
     } else {
         f = ((long)i * N + j) * (N + 1) + k;
         cf = (fe.ee2(i + 1, j, k) - fe.ee2(i, j, k)) - (fe.ee1(i, j + 1, k) - fe.ee1(i, j, k));
         b = a.b3[f];
-        if (a.u0) b0 = a.b03[f];
+        if (a.u0) b0 = get_once<NT>(&a.b03[f]);
     }
     double r = b - cf * (dt / a.dl);
     if (a.u0) r = b0 * a.rk_b + r * (1.0 - a.rk_b);
     double* out = A == 1 ? a.bo1 : (A == 2 ? a.bo2 : a.bo3);
-    out[f] = r;
+    put_once<NT>(r, &out[f]);
 }
 
 // The face-field update per cell: the three faces below it (and the faces at
 // N on the last planes).
-template<typename R>
+template<typename R, bool NT>
 __global__ void __launch_bounds__(256)
 mhd_face_b_kernel(MhdArgs a, FaceE<R> fe)
 {
@@ -706,12 +724,12 @@ mhd_face_b_kernel(MhdArgs a, FaceE<R> fe)
     int i, j, k;
     cell_index(c, N, i, j, k);
     const double dt = *a.dt;
-    mhd_update_face<R, 1>(a, fe, dt, i, j, k);
-    mhd_update_face<R, 2>(a, fe, dt, i, j, k);
-    mhd_update_face<R, 3>(a, fe, dt, i, j, k);
-    if (i == N - 1) mhd_update_face<R, 1>(a, fe, dt, N, j, k);
-    if (j == N - 1) mhd_update_face<R, 2>(a, fe, dt, i, N, k);
-    if (k == N - 1) mhd_update_face<R, 3>(a, fe, dt, i, j, N);
+    mhd_update_face<NT, R, 1>(a, fe, dt, i, j, k);
+    mhd_update_face<NT, R, 2>(a, fe, dt, i, j, k);
+    mhd_update_face<NT, R, 3>(a, fe, dt, i, j, k);
+    if (i == N - 1) mhd_update_face<NT, R, 1>(a, fe, dt, N, j, k);
+    if (j == N - 1) mhd_update_face<NT, R, 2>(a, fe, dt, i, N, k);
+    if (k == N - 1) mhd_update_face<NT, R, 3>(a, fe, dt, i, j, N);
 }
 
 // The face-field update by bricks, for cubes the column-tile pass covers: a
@@ -724,11 +742,11 @@ mhd_face_b_kernel(MhdArgs a, FaceE<R> fe)
 // N on the last planes, with the operands and arithmetic of
 // mhd_update_face.  A thread's face fields and RK base are loaded before the
 // edges, so their latency overlaps the edge loads.
-template<typename R, int BI, int BJ, int BK>
+template<typename R, int BI, int BJ, int BK, bool NT>
 __global__ void __launch_bounds__(BI * BJ * BK)
 mhd_face_b_brick_kernel(MhdArgs a, FaceE<R> fe)
 {
-    constexpr int NT = BI * BJ * BK;
+    constexpr int LANES = BI * BJ * BK;
     constexpr int N1 = BI * (BJ + 1) * (BK + 1);        // x edges
     constexpr int N2 = (BI + 1) * BJ * (BK + 1);        // y edges
     constexpr int N3 = (BI + 1) * (BJ + 1) * BK;        // z edges
@@ -749,9 +767,9 @@ mhd_face_b_brick_kernel(MhdArgs a, FaceE<R> fe)
     const long fz = ((long)i * N + j) * (N + 1) + k;
     const double bx = a.b1[fx], by = a.b2[fy], bz = a.b3[fz];
     double b0x = 0.0, b0y = 0.0, b0z = 0.0;
-    if (a.u0) { b0x = a.b01[fx]; b0y = a.b02[fy]; b0z = a.b03[fz]; }
+    if (a.u0) { b0x = get_once<NT>(&a.b01[fx]); b0y = get_once<NT>(&a.b02[fy]); b0z = get_once<NT>(&a.b03[fz]); }
 
-    for (int e = t; e < N1 + N2 + N3; e += NT) {
+    for (int e = t; e < N1 + N2 + N3; e += LANES) {
         if (e < N1) {
             const int c = e % (BK + 1), r = e / (BK + 1) % (BJ + 1), p = e / ((BK + 1) * (BJ + 1));
             X1[p][r][c] = fe.ee1(i0 + p, j0 + r, k0 + c);
@@ -772,7 +790,7 @@ mhd_face_b_brick_kernel(MhdArgs a, FaceE<R> fe)
     auto put = [&] (double b, double b0, double* out, long f, double cf) {
         double r = b - cf * dtdl;
         if (a.u0) r = b0 * a.rk_b + r * (1.0 - a.rk_b);
-        out[f] = r;
+        put_once<NT>(r, &out[f]);
     };
     put(bx, b0x, a.bo1, fx, (Z3[il][jl + 1][kl] - Z3[il][jl][kl]) - (Y2[il][jl][kl + 1] - Y2[il][jl][kl]));
     put(by, b0y, a.bo2, fy, (X1[il][jl][kl + 1] - X1[il][jl][kl]) - (Z3[il + 1][jl][kl] - Z3[il][jl][kl]));
