@@ -207,9 +207,8 @@ constexpr int tile_index(int tj, int h)
         if (kTileVariants[i].tj == tj && kTileVariants[i].h == h) return i;
     return -1;
 }
-// [kind][precision]: the shape of meshes that fill the device, from sweeps of
-// the benchmark meshes (the tree kind runs 64^2 leaves); g_tile holds a
-// caller's choice, or -1.
+// What m3p_get_stage2d_tile reports while no caller has chosen a shape; g_tile
+// ([kind][precision]) holds a caller's choice, or -1.
 constexpr TileShape kLargeTile[kNumKinds] = { {256, 16}, {256, 16}, {64, 16} };
 std::atomic<int> g_tile[kNumKinds][2] = { { -1, -1 }, { -1, -1 }, { -1, -1 } };
 
@@ -220,19 +219,22 @@ bool tile_fits(TileShape v, int n) { return n % v.tj == 0 && n % v.h == 0 && v.h
 // its strip in series (2 to 3 us a row for FP64 Euler), so a mesh of few
 // zones is bound by that chain and wants short strips; every strip also
 // recovers four extra rows and computes one extra row of x fluxes, so a mesh
-// that fills the device wants long ones.  The lines are from sweeps of both
-// stages on meshes of 64^2 to 4096^2 zones: two-row strips below 2048 waves
-// of four rows (FP64 Euler, 256^2 zones in 32^2 blocks: 24 us a step, 32 with
-// four rows, 92 with sixteen), four rows up to 2048 waves of eight, then eight
-// (1024^2 zones in 64^2 blocks: FP64 80 us against 100 with sixteen rows,
-// mixed 47 against 65).  Meshes of 4096 waves of sixteen rows or more take
-// the wide tiles where they fit, in FP64 from 8192 waves on (256^2 blocks,
-// FP64 HLLC, 4096^2: 993 us against 1055 with 64 x 8, 2048^2: 274 against 264;
-// minidisk, 2048^2: 198 against 187; mixed HLLC, 4096^2: 655 against 690), else
-// stay at eight (2048^2 in 64^2 blocks, FP64: 266 us against 312 with sixteen;
-// quad-tree of 1408 leaves, mixed: 223 against 233), but for the FP64 minidisk
-// from 8192 waves on (4096^2 in 64^2 blocks: 806 us with sixteen, 841 with
-// eight).
+// that fills the device wants long ones.  Tiles of one wave exchange columns
+// by wave shifts (stage2d.hpp), so wide blocks are cut into them.  The lines
+// are from sweeps of both stages on meshes of 64^2 to 4096^2 zones: two-row
+// strips below 2048 waves of four rows (FP64 Euler, 256^2 zones in 32^2 blocks:
+// 20 us a step, 28 with four rows, 90 with sixteen), four rows up to 2048 waves
+// of eight, then eight (1024^2 zones in 64^2 blocks: FP64 75 us against 84 with
+// four rows and 88 with sixteen, mixed 44 against 47 and 53); sixteen for FP64
+// from 8192 waves of sixteen rows on (4096^2 in 256^2 blocks: HLLC 1017 us
+// against 1030 with eight rows and 1059 with 256 x 16 tiles, HLLE 968, 1020 and
+// 1034, minidisk 674, 708 and 720; 2048^2 in 64^2 blocks: HLLC 272 with sixteen,
+// 264 with eight), the quad-tree's leaves and mixed precision staying at eight
+// (tree of 1408 leaves: mixed 214 us, 236 with sixteen; FP64 362 and 376; mixed
+// HLLC, 4096^2: 677 us, 692 with sixteen, 685 with 256 x 16 tiles), but for the
+// mixed minidisk, whose wide tiles read fewer halos (4096^2: 399 us, 405 with 64
+// x 8).  Blocks of 32^2 take sixteen rows from 4096 waves on in FP64 (2048^2:
+// HLLC 304 us, 314 with eight).
 TileShape pick_tile(int kind, int precision, int n, int nblk)
 {
     const int chosen = g_tile[kind][precision].load(std::memory_order_relaxed);
@@ -240,12 +242,9 @@ TileShape pick_tile(int kind, int precision, int n, int nblk)
     const double zones = (double)nblk * n * n;
     auto waves = [&] (int rows) { return zones / (64.0 * rows); };
     int rows = waves(16) >= 4096 ? 16 : waves(8) >= 2048 ? 8 : waves(4) >= 2048 ? 4 : 2;
-    if (rows == 16 && kind != M3P_KIND_AMR_EULER2D) {
-        if (tile_fits(kLargeTile[kind], n) && (precision == M3P_MIXED || waves(16) >= 8192)) return kLargeTile[kind];
-        if (precision == M3P_MIXED && n % 128 == 0) return {128, 32};     // 153 us against 163 (64 x 8) at 2048^2
-    }
+    if (rows == 16 && kind == M3P_KIND_MINIDISK && precision == M3P_MIXED && n % 256 == 0) return {256, 16};
     if (n % 64 == 0) {
-        const bool long_strips = precision == M3P_FP64 && kind == M3P_KIND_MINIDISK && waves(16) >= 8192;
+        const bool long_strips = precision == M3P_FP64 && kind != M3P_KIND_AMR_EULER2D && waves(16) >= 8192;
         return {64, rows == 16 && !long_strips ? 8 : rows};
     }
     if (rows == 16 && (precision == M3P_MIXED || kind == M3P_KIND_AMR_EULER2D)) rows = 8;

@@ -238,6 +238,29 @@ __device__ __forceinline__ double wave_sum(double v)
     return v;
 }
 
+// The value of the lane before / after in the wave; the first / last lane
+// takes `edge`.  Every lane must be active.
+__device__ __forceinline__ float lane_before(float x, float edge)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(edge), __float_as_int(x), 0x138 /* wave_shr:1 */,
+                                                      0xf, 0xf, false));
+}
+__device__ __forceinline__ float lane_after(float x, float edge)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(edge), __float_as_int(x), 0x130 /* wave_shl:1 */,
+                                                      0xf, 0xf, false));
+}
+__device__ __forceinline__ double lane_before(double x, double edge)
+{
+    return __hiloint2double(__builtin_amdgcn_update_dpp(__double2hiint(edge), __double2hiint(x), 0x138, 0xf, 0xf, false),
+                            __builtin_amdgcn_update_dpp(__double2loint(edge), __double2loint(x), 0x138, 0xf, 0xf, false));
+}
+__device__ __forceinline__ double lane_after(double x, double edge)
+{
+    return __hiloint2double(__builtin_amdgcn_update_dpp(__double2hiint(edge), __double2hiint(x), 0x130, 0xf, 0xf, false),
+                            __builtin_amdgcn_update_dpp(__double2loint(edge), __double2loint(x), 0x130, 0xf, 0xf, false));
+}
+
 // XCD-aware workgroup remap.  Workgroups are dispatched round-robin over the
 // 8 XCDs (each with its own L2); give each XCD a contiguous range of logical
 // tiles so that tiles sharing halo rows share an L2.

@@ -261,10 +261,7 @@ rk2_fused_kernel(typename S::Params p1, typename S::Params p2, MeshLoader<S> ld,
     };
     auto flux_above = [&] (R own, const R (&F)[NC][NF], int m) -> R {
         if constexpr (kQueue) {
-            // wave_shl:1, the last lane of the wave keeps the first operand
-            static_assert(sizeof(R) == 4, "one register");
-            return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(F[m][t / 64 + 1]), __float_as_int(own),
-                                                              0x130, 0xf, 0xf, false));
+            return lane_after(own, F[m][t / 64 + 1]);
         } else {
             return F[m][t + 1];
         }

@@ -43,17 +43,9 @@ namespace m3p {
 constexpr int kWindow1D = 56;          // zones a wave updates
 constexpr int kWindowGroup = 4;        // waves of a workgroup
 
-// the value of the lane before / after (the first / last lane keeps its own)
-__device__ __forceinline__ float lane_before(float x)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(x), __float_as_int(x), 0x138 /* wave_shr:1 */,
-                                                      0xf, 0xf, false));
-}
-__device__ __forceinline__ float lane_after(float x)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(x), __float_as_int(x), 0x130 /* wave_shl:1 */,
-                                                      0xf, 0xf, false));
-}
+// (the first / last lane of the wave keeps its own)
+__device__ __forceinline__ float lane_before(float x) { return lane_before(x, x); }
+__device__ __forceinline__ float lane_after(float x) { return lane_after(x, x); }
 
 static __global__ void __launch_bounds__(64 * kWindowGroup)
 rk2_fused_1d_kernel(EulerParams prm, Stage1DArgs a)

@@ -5,10 +5,16 @@
 // adjacent columns (the contiguous axis) of one block and marches down H
 // rows.  Each thread keeps a three-row register window of primitives for the
 // x (row-axis) stencil, so every x face flux is computed once and carried to
-// the next row.  The y (column-axis) stencil goes through three LDS rows
-// (primitives, slopes, fluxes); the two halo columns on each side and the
-// tile's right-edge y flux for all H rows are computed once, up front, by a
-// halo pre-pass, so no lane does redundant per-row work.
+// the next row.  The two halo columns on each side and the tile's right-edge y
+// flux for all H rows are computed once, up front, by a halo pre-pass, so no
+// lane does redundant per-row work.  For the y (column-axis) stencil the lanes
+// of a one-wave tile take their neighbours' values by wave shifts, the edge
+// lanes theirs from one LDS row of the pre-pass (five 16-byte reads in mixed
+// precision); a wider tile exchanges whole rows through LDS (primitives,
+// slopes, fluxes: some 80 LDS instructions and three waits a row, which a
+// one-wave tile also paid before).  A step of 1408 quad-tree leaves, mixed: 252
+// to 234 us; FP64 2048^2 zones in 64^2 blocks: Euler HLLE 279 to 259; minidisk,
+// 1024^2: 63 to 57.5.
 //
 // Guard zones are never materialised: a zone outside the block is read
 // directly from the neighbouring block through the neighbour table (the
@@ -321,6 +327,8 @@ stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
     constexpr int NT = TJ * G;                 // lanes of the workgroup
     constexpr int HS = H / G;                  // rows of a strip
     static_assert(H % G == 0, "whole strips");
+    constexpr bool kShift = NT == 64;          // one wave: neighbours by wave shifts
+    static_assert(kShift || G == 1, "strips share a wave");
     constexpr bool kLateBase = S::late_base(HS);
     using R = typename S::Real;
     resolve_params(prm);
@@ -359,12 +367,14 @@ stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
     __shared__ R hraw[7][NC][H];     // pre-pass primitives at 7 edge columns
     __shared__ R hG[NC][H];          // y half slope at column c0-1
     __shared__ R hF[NC][H];          // y flux at face c0+TJ
-    __shared__ R rowPs[G][NC][TJ + 2];   // [t+1] = column c0+t; [0], [TJ+1] from hraw
-    __shared__ R rowGs[G][NC][TJ + 1];   // [t+1] = half slope at column c0+t; [0] from hG
-    __shared__ R rowFs[G][NC][TJ + 1];   // [t] = y flux at face c0+t; [TJ] from hF
-    R (&rowP)[NC][TJ + 2] = rowPs[g];
-    R (&rowG)[NC][TJ + 1] = rowGs[g];
-    R (&rowF)[NC][TJ + 1] = rowFs[g];
+    // one wave (kShift): what the edge lanes of a row take from beyond the
+    // tile, the primitives at column c0-1, their sum with the half slope
+    // there, the primitives at column c0+TJ and the flux at face c0+TJ
+    __shared__ alignas(16) R edge[kShift ? H : 1][kShift ? 4 : 1][NC];
+    // several waves: rows of LDS
+    __shared__ R rowP[NC][kShift ? 1 : TJ + 2];   // [t+1] = column c0+t; [0], [TJ+1] from hraw
+    __shared__ R rowG[NC][kShift ? 1 : TJ + 1];   // [t+1] = half slope at column c0+t; [0] from hG
+    __shared__ R rowF[NC][kShift ? 1 : TJ + 1];   // [t] = y flux at face c0+t; [TJ] from hF
 
     S::setup(td, prm, tc);
     bool ok = true;
@@ -392,7 +402,15 @@ stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
         }
         S::template face<2>(pl, pr, prm, td, tc, tc.k0 + r, tc.c0 + TJ, f);
 #pragma unroll
-        for (int m = 0; m < NC; ++m) hF[m][r] = f[m];
+        for (int m = 0; m < NC; ++m) {
+            hF[m][r] = f[m];
+            if constexpr (kShift) {
+                edge[r][0][m] = hraw[1][m][r];
+                edge[r][1][m] = hraw[1][m][r] + hG[m][r];
+                edge[r][2][m] = hraw[5][m][r];
+                edge[r][3][m] = f[m];
+            }
+        }
         if (Ld::kEdgeFluxes && a.flux_reg && tc.c0 + TJ == n) store_edge_flux<NC>(a.flux_reg, b, 3, n, tc.k0 + r, f);
     }
 
@@ -404,13 +422,14 @@ stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
     // is computed from the same operands in the same order in both
     // directions, so the results do not depend on the direction.
     //
-    // Edge lanes read their out-of-tile neighbours from the pre-pass arrays
-    // through a selected address (no divergent branch).  Loaders that
-    // support it are software-pipelined: the raw state of the row three
-    // ahead and the RK base of the current row are fetched at the top of an
-    // iteration, so their latency overlaps the iteration's arithmetic (a
-    // scheme with late_base loads the RK base at the update instead, holding
-    // fewer registers across the row).
+    // Edge lanes take their out-of-tile neighbours from the pre-pass without a
+    // divergent branch.  Loaders that support it are software-pipelined: the
+    // raw state of the row three ahead and the RK base of the current row are
+    // fetched at the top of an iteration, so their latency overlaps the
+    // iteration's arithmetic (a scheme with late_base loads the RK base at the
+    // update instead, holding fewer registers across the row).
+    auto before = [&] (R x, R e) { const R y = lane_before(x, e); return G > 1 && t == 0 ? e : y; };
+    auto after = [&] (R x, R e) { const R y = lane_after(x, e); return G > 1 && t == TJ - 1 ? e : y; };
     auto march = [&] (auto dir) {
         constexpr int D = decltype(dir)::value;
         const int kfirst = D > 0 ? tc.k0 + g * HS : tc.k0 + g * HS + HS - 1;
@@ -508,38 +527,59 @@ stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
             S::template face<1>(pl, pr, prm, td, tc, fk, c, Fa);
             if (Ld::kEdgeFluxes && a.flux_reg && (fk == 0 || fk == n)) store_edge_flux<NC>(a.flux_reg, b, fk == 0 ? 0 : 1, n, c, Fa);
 
-            // The two edge lanes also store the out-of-tile neighbours of this
-            // row (from the pre-pass) at the ends of the LDS rows, so every
-            // lane reads its neighbours at the same offsets, with no select.
+            // the primitives of the columns on each side: y slope and left state
+            R eF[NC];
+            if constexpr (kShift) {
+                R el[NC], es[NC], er[NC];
 #pragma unroll
-            for (int m = 0; m < NC; ++m) rowP[m][t + 1] = Pa[m];
-            if (t == 0) {
+                for (int m = 0; m < NC; ++m) {
+                    el[m] = edge[kl][0][m];
+                    es[m] = edge[kl][1][m];
+                    er[m] = edge[kl][2][m];
+                    eF[m] = edge[kl][3][m];
+                }
 #pragma unroll
-                for (int m = 0; m < NC; ++m) { rowP[m][0] = hraw[1][m][kl]; rowG[m][0] = hG[m][kl]; }
-            }
-            if (t == TJ - 1) {
+                for (int m = 0; m < NC; ++m) {
+                    gy[m] = plm_half(before(Pa[m], el[m]), Pa[m], after(Pa[m], er[m]), theta);
+                    pl[m] = before(Pa[m] + gy[m], es[m]);
+                    pr[m] = Pa[m] - gy[m];
+                }
+            } else {
+                // The two edge lanes also store the out-of-tile neighbours of this
+                // row (from the pre-pass) at the ends of the LDS rows, so every
+                // lane reads its neighbours at the same offsets, with no select.
 #pragma unroll
-                for (int m = 0; m < NC; ++m) rowP[m][TJ + 1] = hraw[5][m][kl];
-            }
-            __syncthreads();
+                for (int m = 0; m < NC; ++m) rowP[m][t + 1] = Pa[m];
+                if (t == 0) {
 #pragma unroll
-            for (int m = 0; m < NC; ++m) {
-                gy[m] = plm_half(rowP[m][t], Pa[m], rowP[m][t + 2], theta);
-                rowG[m][t + 1] = gy[m];
-            }
-            __syncthreads();
+                    for (int m = 0; m < NC; ++m) { rowP[m][0] = hraw[1][m][kl]; rowG[m][0] = hG[m][kl]; }
+                }
+                if (t == TJ - 1) {
 #pragma unroll
-            for (int m = 0; m < NC; ++m) {
-                pl[m] = rowP[m][t] + rowG[m][t];
-                pr[m] = Pa[m] - gy[m];
+                    for (int m = 0; m < NC; ++m) rowP[m][TJ + 1] = hraw[5][m][kl];
+                }
+                __syncthreads();
+#pragma unroll
+                for (int m = 0; m < NC; ++m) {
+                    gy[m] = plm_half(rowP[m][t], Pa[m], rowP[m][t + 2], theta);
+                    rowG[m][t + 1] = gy[m];
+                }
+                __syncthreads();
+#pragma unroll
+                for (int m = 0; m < NC; ++m) {
+                    pl[m] = rowP[m][t] + rowG[m][t];
+                    pr[m] = Pa[m] - gy[m];
+                }
             }
             S::template face<2>(pl, pr, prm, td, tc, k, c, Fy);
-#pragma unroll
-            for (int m = 0; m < NC; ++m) rowF[m][t] = Fy[m];
             if (Ld::kEdgeFluxes && a.flux_reg && c == 0) store_edge_flux<NC>(a.flux_reg, b, 2, n, k, Fy);
-            if (t == TJ - 1) {
+            if constexpr (!kShift) {
 #pragma unroll
-                for (int m = 0; m < NC; ++m) rowF[m][TJ] = hF[m][kl];
+                for (int m = 0; m < NC; ++m) rowF[m][t] = Fy[m];
+                if (t == TJ - 1) {
+#pragma unroll
+                    for (int m = 0; m < NC; ++m) rowF[m][TJ] = hF[m][kl];
+                }
             }
             // The update's loads (the zone's state where the kernel does not
             // keep it in registers, the RK base where the loader has no
@@ -557,14 +597,15 @@ stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
                     for (int m = 0; m < NC; ++m) U0[m] = __builtin_nontemporal_load(&z0[(size_t)m * n * n]);
                 }
             }
-            __syncthreads();
+            if constexpr (!kShift) __syncthreads();
 
             double dfx[NC], dfy[NC], res[NC], fa[NC];
 #pragma unroll
             for (int m = 0; m < NC; ++m) {
                 fa[m] = double(Fa[m]);
                 dfx[m] = D > 0 ? fa[m] - Fb[m] : Fb[m] - fa[m];
-                dfy[m] = double(rowF[m][t + 1]) - double(Fy[m]);
+                if constexpr (kShift) dfy[m] = double(after(Fy[m], eF[m])) - double(Fy[m]);
+                else                  dfy[m] = double(rowF[m][t + 1]) - double(Fy[m]);
             }
             if constexpr (KEEPU) {
 #pragma unroll
