@@ -45,15 +45,17 @@ static int mhd_advance_as(MhdArgs a, char* work, hipStream_t s)
     // workgroups as it can give (FP64 64^3: 98 us a step with 2 planes, 236
     // with 16; mixed 100^3: 190 us with 8, 233 with 16).  Mixed keeps to 8
     // planes (1.37 ms at 200^3 against 1.42 with 16, equal at 256^3).
-    auto tiles = [&] (auto kern) {
-        const int cols = ((N + 7) / 8) * ((N + 31) / 32);
-        const int groups = is_fp64<R>::value ? 640 : 768, cap = is_fp64<R>::value ? 16 : 8;
-        const int TI = (int)std::max(2l, std::min((long)cap, (long)N * cols / groups));
-        hipLaunchKernelGGL(kern, dim3(cols * ((N + TI - 1) / TI)), dim3(256), 0, s, a,
-                           (const typename MhdPrim<R>::V*)P, E1, E2, E3, TI);
-    };
-    if (N % 32 == 0) tiles(mhd_tile_kernel<R, 8, 32, false, NT>);
-    else             tiles(mhd_tile_kernel<R, 8, 32, true, NT>);
+    const bool ragged = N % 32 != 0;
+    const MhdTile tile = ragged && !NT ? mhd_ragged_tile(N) : kMhdWideTile;
+    auto kern = ragged ? mhd_tile_kernel<R, true, false, NT> : mhd_tile_kernel<R, false, false, NT>;
+    if constexpr (!NT) {
+        if (tile.tj != kMhdWideTile.tj || tile.tk != kMhdWideTile.tk) kern = mhd_tile_kernel<R, true, true, NT>;
+    }
+    const int cols = ((N + tile.tj - 1) / tile.tj) * ((N + tile.tk - 1) / tile.tk);
+    const int groups = is_fp64<R>::value ? 640 : 768, cap = is_fp64<R>::value ? 16 : 8;
+    const int TI = (int)std::max(2l, std::min((long)cap, (long)N * cols / groups));
+    hipLaunchKernelGGL(kern, dim3(cols * ((N + TI - 1) / TI)), dim3(kMhdTileLanes), 0, s, a,
+                       (const typename MhdPrim<R>::V*)P, E1, E2, E3, TI, tile);
     if (int st = launch_status("mhd_tile_kernel")) return st;
     // The face fields: FP64 by bricks of 4 x 4 x 32 cells where they divide
     // the cube (the step 4.41 ms at 256^3 against 4.71 per cell, 626 us

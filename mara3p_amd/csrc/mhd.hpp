@@ -26,6 +26,7 @@
 // and the tile pass gives an XCD whole rows of tiles (2.48 GB a stage, was
 // 2.67 with an XCD per strip of 32 cells along k; the RK2 step 2.76 to 2.62 ms).
 #pragma once
+#include <algorithm>
 #include "device_common.hpp"
 
 namespace m3p {
@@ -379,9 +380,8 @@ mhd_prim_kernel(MhdArgs a, typename MhdPrim<R>::V* P)
 // fluxes never leave the workgroup; the transverse face electric fields go to
 // the E arrays for the face update.  Every face is computed from the same
 // operands in the same order wherever it is computed, so a face shared by two
-// tiles or segments has one value.  RAGGED: the tiles do not divide the cube
-// (100^3 mixed: 200 us a step, 278 through passes per cell that wrote and
-// re-read every face flux).
+// tiles or segments has one value.  RAGGED: a cube that 8 x 32 tiles do not
+// divide.
 // Mixed: four waves per SIMD, where the register allocator fits the kernel
 // in 128 VGPRs without spills (150 when unconstrained, three waves) and the
 // extra wave hides load latency (11 % faster per RK2 step at 256^3).  FP64:
@@ -389,12 +389,50 @@ mhd_prim_kernel(MhdArgs a, typename MhdPrim<R>::V* P)
 // association order.
 template<typename R> struct MhdTileWaves { static constexpr int value = is_fp64<R>::value ? 2 : 4; };
 
-template<typename R, int TJ, int TK, bool RAGGED, bool NT>
-__global__ void __launch_bounds__(TJ * TK) __attribute__((amdgpu_waves_per_eu(MhdTileWaves<R>::value, 8)))
-mhd_tile_kernel(MhdArgs a, const typename MhdPrim<R>::V* P, R* E1, R* E2, R* E3, int TI)
+constexpr int kMhdTileLanes = 256;
+constexpr int kMhdTileHalo = 448, kMhdTileF2 = 296, kMhdTileF3 = 272;   // LDS of a ragged tile
+
+// The shape of a ragged tile (SHAPED, given at run time): of those whose columns
+// fit the lanes, whose halo ring has a lane for each cell and whose planes fit
+// the LDS above, the one that covers the N x N columns with the fewest tiles,
+// and of these the one with the smallest halo (100: 10 x 25 columns, 40 tiles of
+// 250 cells, where 8 x 32 takes 52 that reach past the cube).  It is taken where
+// that is at most 5/6 of the tiles, for cubes that the cache holds, whose pass
+// is bound by its arithmetic, and that give the device more than a few
+// workgroups: RK2 step of 100^3 mixed 192 to 173 us, FP64 322 to 283; 80^3 106
+// to 98 and 180 to 162; 65^3 78 to 75 and 129 to 118; 45^3 53 to 51 and 74 to 62.
+// With every ragged cube so, 110^3 mixed 234 to 239, 25^3 FP64 49 to 51, and,
+// bound by memory, where rows of partial cache lines cost more, 250^3 mixed
+// 2684 to 3265.
+struct MhdTile { int tj, tk; };
+constexpr MhdTile kMhdWideTile{ 8, 32 };
+inline MhdTile mhd_ragged_tile(int N)
 {
-    constexpr int LANES = TJ * TK;
-    constexpr int EJ = TJ + 4, EK = TK + 4;
+    MhdTile best = kMhdWideTile;
+    long tiles = 0, halo = 0;
+    for (int nk = (N + 39) / 40; nk <= N; ++nk) {
+        const int tk = (N + nk - 1) / nk;
+        if (tk < 8 && N >= 8) break;
+        const int most = std::min(16, std::min(kMhdTileLanes / tk, kMhdTileHalo / (tk + 4) - 4));
+        const int nj = (N + most - 1) / most, tj = (N + nj - 1) / nj;
+        const long t = (long)nk * nj, h = (long)(tj + 4) * (tk + 4);
+        if (tiles == 0 || t < tiles || (t == tiles && h < halo)) { best = { tj, tk }; tiles = t; halo = h; }
+    }
+    const long wide = (long)((N + 7) / 8) * ((N + 31) / 32);
+    return N > 32 && 6 * tiles <= 5 * wide ? best : kMhdWideTile;
+}
+
+template<typename R, bool RAGGED, bool SHAPED, bool NT>
+__global__ void __launch_bounds__(kMhdTileLanes) __attribute__((amdgpu_waves_per_eu(MhdTileWaves<R>::value, 8)))
+mhd_tile_kernel(MhdArgs a, const typename MhdPrim<R>::V* P, R* E1, R* E2, R* E3, int TI, MhdTile tile)
+{
+    constexpr int LANES = kMhdTileLanes;
+    static_assert(RAGGED || !SHAPED);
+    const int TJ = SHAPED ? tile.tj : 8, TK = SHAPED ? tile.tk : 32;
+    const int EK = TK + 4;
+    // the most of any tile (MhdTile), or those of 8 x 32
+    constexpr int NP = SHAPED ? kMhdTileHalo : 12 * 36;
+    constexpr int NF2 = SHAPED ? kMhdTileF2 : 9 * 32, NF3 = SHAPED ? kMhdTileF3 : 8 * 33;
     using Vec = typename MhdPrim<R>::V;
     constexpr int NV = MhdPrim<R>::NV;
     const int N = a.N;
@@ -407,18 +445,19 @@ mhd_tile_kernel(MhdArgs a, const typename MhdPrim<R>::V* P, R* E1, R* E2, R* E3,
     // planes last, so they are the likeliest to still be cached
     const int i0 = ((N + TI - 1) / TI - 1 - w) * TI;
     const int ni = min(TI, N - i0);
-    const int t = threadIdx.x, jl = t / TK, kl = t % TK;
+    // lanes past a tile of fewer cells repeat the last one's work, storing nothing
+    const int t = threadIdx.x, tt = SHAPED ? min(t, TJ * TK - 1) : t, jl = tt / TK, kl = tt % TK;
     const int j = j0 + jl, k = k0 + kl;
     // A ragged tile reaches past the cube: its lanes there load from the
     // nearest index inside (jc, kc for cells, clamped face indices below) and
     // store nothing; the first row and column of them compute the upper
     // boundary faces, which are the cube's.
     const int jc = RAGGED ? min(j, N - 1) : j, kc = RAGGED ? min(k, N - 1) : k;
-    const bool in_j = !RAGGED || j < N, in_k = !RAGGED || k < N;
+    const bool in_j = !RAGGED || (j < N && t == tt), in_k = !RAGGED || k < N;
 
-    __shared__ Vec Pl[NV][EJ][EK];    // primitives of plane i, (j0 - 2 .. j0 + TJ + 1) x (k0 - 2 .. k0 + TK + 1)
-    __shared__ R F2s[5][TJ + 1][TK];  // y-face fluxes of plane i, faces j0 .. j0 + TJ
-    __shared__ R F3s[5][TJ][TK + 1];  // z-face fluxes of plane i, faces k0 .. k0 + TK
+    __shared__ Vec Pl[NV][NP];   // primitives of plane i, (j0 - 2 .. j0 + TJ + 1) x (k0 - 2 .. k0 + TK + 1)
+    __shared__ R F2s[5][NF2];    // y-face fluxes of plane i, faces j0 .. j0 + TJ, [TJ + 1][TK]
+    __shared__ R F3s[5][NF3];    // z-face fluxes of plane i, faces k0 .. k0 + TK, [TJ][TK + 1]
 
     __shared__ double vpart[LANES / 64];  // fastest speed, by wave
     {
@@ -428,26 +467,29 @@ mhd_tile_kernel(MhdArgs a, const typename MhdPrim<R>::V* P, R* E1, R* E2, R* E3,
         if ((t & 63) == 0) vpart[t >> 6] = v;
     }
     const R theta = R(a.theta), gamma = R(a.gamma);
-    auto cell = [&] (int ii, int jj, int kk) {
+    // place of a column in its plane, and of a cell of it
+    auto column = [&] (int jj, int kk) {
         if (RAGGED) { jj = min(jj, N + 1); kk = min(kk, N + 1); }
-        return ((long)wrapi(ii, N) * N + wrapi(jj, N)) * N + wrapi(kk, N);
+        return wrapi(jj, N) * N + wrapi(kk, N);
     };
+    auto cell = [&] (int ii, int col) { return (long)wrapi(ii, N) * N * N + col; };
+    const int own_col = column(j, k);
     auto loadP = [&] (long c, R* p) {
         Vec x[NV];
 #pragma unroll
         for (int v = 0; v < NV; ++v) x[v] = P[v * N3 + c];
         MhdPrim<R>::unpack(x, p);
     };
-    auto putP = [&] (int rj, int rk, const R* p) {
+    auto putP = [&] (int at, const R* p) {
         Vec x[NV];
         MhdPrim<R>::pack(p, x);
 #pragma unroll
-        for (int v = 0; v < NV; ++v) Pl[v][rj][rk] = x[v];
+        for (int v = 0; v < NV; ++v) Pl[v][at] = x[v];
     };
-    auto getP = [&] (int rj, int rk, R* p) {
+    auto getP = [&] (int at, R* p) {
         Vec x[NV];
 #pragma unroll
-        for (int v = 0; v < NV; ++v) x[v] = Pl[v][rj][rk];
+        for (int v = 0; v < NV; ++v) x[v] = Pl[v][at];
         MhdPrim<R>::unpack(x, p);
     };
     // face states from four cells along the face normal (lower two, upper two)
@@ -465,10 +507,10 @@ mhd_tile_kernel(MhdArgs a, const typename MhdPrim<R>::V* P, R* E1, R* E2, R* E3,
     R Pm[8], P0[8], Pp[8], g0[8], Fx_lo[5];
     {
         R Pm2[8], pl[8], pr[8], e[3];
-        loadP(cell(i0 - 2, j, k), Pm2);
-        loadP(cell(i0 - 1, j, k), Pm);
-        loadP(cell(i0, j, k), P0);
-        loadP(cell(i0 + 1, j, k), Pp);
+        loadP(cell(i0 - 2, own_col), Pm2);
+        loadP(cell(i0 - 1, own_col), Pm);
+        loadP(cell(i0, own_col), P0);
+        loadP(cell(i0 + 1, own_col), Pp);
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
             g0[q] = plm_half(Pm[q], P0[q], Pp[q], theta);
@@ -488,7 +530,7 @@ mhd_tile_kernel(MhdArgs a, const typename MhdPrim<R>::V* P, R* E1, R* E2, R* E3,
     const double dtdl = dt / a.dl;
 
     // The plane's two-cell halo ring (NH cells): position of ring cell r.
-    constexpr int NH = 4 * EK + 4 * TJ;
+    const int NH = 4 * EK + 4 * TJ;
     auto ring = [&] (int r, int& rj, int& rk) {
         if (r < 2 * EK)      { rj = r / EK; rk = r % EK; }
         else if (r < 4 * EK) { rj = TJ + 2 + (r - 2 * EK) / EK; rk = (r - 2 * EK) % EK; }
@@ -499,39 +541,30 @@ mhd_tile_kernel(MhdArgs a, const typename MhdPrim<R>::V* P, R* E1, R* E2, R* E3,
             rk = side < 2 ? side : TK + side;
         }
     };
-    // Where every ring cell has a thread of its own (the 8 x 32 tiles): the
-    // ring of the next plane is fetched while this plane computes (its load
-    // latency off the plane's critical path; 127 VGPRs mixed, 254 FP64).
-    constexpr bool kRingAhead = NH <= LANES;
-    int hj = 0, hk = 0;
+    // Every ring cell has a thread of its own: the ring of the next plane is
+    // fetched while this plane computes (its load latency off the plane's
+    // critical path).
+    const int here = (jl + 2) * EK + kl + 2;            // the cell's place in the plane
+    int h_at = 0, h_col = 0;
     R Hn[8];
-    if constexpr (kRingAhead) {
-        if (t < NH) {
-            ring(t, hj, hk);
-            loadP(cell(i0, j0 - 2 + hj, k0 - 2 + hk), Hn);
-        }
+    if (t < NH) {
+        int hj, hk;
+        ring(t, hj, hk);
+        h_at = hj * EK + hk;
+        h_col = column(j0 - 2 + hj, k0 - 2 + hk);
+        loadP(cell(i0, h_col), Hn);
     }
 
     for (int il = 0; il < ni; ++il) {
         const int i = i0 + il;
         R Pn[8];
-        loadP(cell(i + 2, j, k), Pn);
+        loadP(cell(i + 2, own_col), Pn);
 
         // LDS plane i: interior from the window, halo ring from memory
-        putP(jl + 2, kl + 2, P0);
-        if constexpr (kRingAhead) {
-            if (t < NH) {
-                putP(hj, hk, Hn);
-                if (il + 1 < ni) loadP(cell(i + 1, j0 - 2 + hj, k0 - 2 + hk), Hn);
-            }
-        } else {
-            for (int r = t; r < NH; r += LANES) {
-                int rj, rk;
-                ring(r, rj, rk);
-                R h[8];
-                loadP(cell(i, j0 - 2 + rj, k0 - 2 + rk), h);
-                putP(rj, rk, h);
-            }
+        putP(here, P0);
+        if (t < NH) {
+            putP(h_at, Hn);
+            if (il + 1 < ni) loadP(cell(i + 1, h_col), Hn);
         }
         // FP64: the longitudinal fields of the cell's own y and z faces are
         // loaded before the barrier, their latency off the faces' path (the
@@ -551,14 +584,15 @@ mhd_tile_kernel(MhdArgs a, const typename MhdPrim<R>::V* P, R* E1, R* E2, R* E3,
         // y face below the cell (face j), and the tile's upper y face by the last row
         auto yface = [&] (int jf /* local face row 0..TJ */, bool own) {
             R c0[8], c1[8], c2[8], c3[8], pl[8], pr[8], f[5], e[3];
-            getP(jf, kl + 2, c0); getP(jf + 1, kl + 2, c1);
-            getP(jf + 2, kl + 2, c2); getP(jf + 3, kl + 2, c3);
+            const int at = own ? here : here + EK;      // the face's upper cell
+            getP(at - 2 * EK, c0); getP(at - EK, c1);
+            getP(at, c2); getP(at + EK, c3);
             states(c0, c1, c2, c3, pl, pr);
             const long fi = ((long)i * (N + 1) + (RAGGED ? min(j0 + jf, N) : j0 + jf)) * N + kc;
             Mhd<R>::template riemann<2>(pl, pr, kPreB && own ? bly : R(a.b2[fi]), gamma, f, e);
 #pragma unroll
-            for (int q = 0; q < 5; ++q) F2s[q][jf][kl] = f[q];
-            if ((jf < TJ || j0 + jf == N) && in_k && (!RAGGED || j0 + jf <= N)) { E2[fi] = e[0]; E2[nf + fi] = e[2]; }
+            for (int q = 0; q < 5; ++q) F2s[q][jf * TK + kl] = f[q];
+            if ((jf < TJ || j0 + jf == N) && in_k && (!RAGGED || (j0 + jf <= N && t == tt))) { E2[fi] = e[0]; E2[nf + fi] = e[2]; }
         };
         yface(jl, true);
         if (jl == TJ - 1) yface(TJ, false);
@@ -566,15 +600,16 @@ mhd_tile_kernel(MhdArgs a, const typename MhdPrim<R>::V* P, R* E1, R* E2, R* E3,
         // z face below the cell (face k), and the tile's upper z faces by threads 0 .. TJ-1
         auto zface = [&] (int row, int kf /* local face column 0..TK */, bool own) {
             R c0[8], c1[8], c2[8], c3[8], pl[8], pr[8], f[5], e[3];
-            getP(row + 2, kf, c0); getP(row + 2, kf + 1, c1);
-            getP(row + 2, kf + 2, c2); getP(row + 2, kf + 3, c3);
+            const int at = own ? here : (row + 2) * EK + kf + 2;
+            getP(at - 2, c0); getP(at - 1, c1);
+            getP(at, c2); getP(at + 1, c3);
             states(c0, c1, c2, c3, pl, pr);
             const long fi = ((long)i * N + (RAGGED ? min(j0 + row, N - 1) : j0 + row)) * (N + 1)
                           + (RAGGED ? min(k0 + kf, N) : k0 + kf);
             Mhd<R>::template riemann<3>(pl, pr, kPreB && own ? blz : R(a.b3[fi]), gamma, f, e);
 #pragma unroll
-            for (int q = 0; q < 5; ++q) F3s[q][row][kf] = f[q];
-            if ((kf < TK || k0 + kf == N) && (!RAGGED || (j0 + row < N && k0 + kf <= N))) { E3[fi] = e[0]; E3[nf + fi] = e[1]; }
+            for (int q = 0; q < 5; ++q) F3s[q][row * (TK + 1) + kf] = f[q];
+            if ((kf < TK || k0 + kf == N) && (!RAGGED || (j0 + row < N && k0 + kf <= N && t == tt))) { E3[fi] = e[0]; E3[nf + fi] = e[1]; }
         };
         zface(jl, kl, true);
         if (t < TJ) zface(t, TK, false);
@@ -615,8 +650,8 @@ mhd_tile_kernel(MhdArgs a, const typename MhdPrim<R>::V* P, R* E1, R* E2, R* E3,
 #pragma unroll
             for (int q = 0; q < 5; ++q) {
                 double d1 = double(Fx_hi[q]) - double(Fx_lo[q]);
-                double d2 = double(F2s[q][jl + 1][kl]) - double(F2s[q][jl][kl]);
-                double d3 = double(F3s[q][jl][kl + 1]) - double(F3s[q][jl][kl]);
+                double d2 = double(F2s[q][(jl + 1) * TK + kl]) - double(F2s[q][jl * TK + kl]);
+                double d3 = double(F3s[q][jl * (TK + 1) + kl + 1]) - double(F3s[q][jl * (TK + 1) + kl]);
                 double r;
                 if constexpr (is_fp64<R>::value) {
                     r = ucv[q] - (d1 + d2 + d3) * dtdl;

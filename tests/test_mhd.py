@@ -135,10 +135,12 @@ def test_gpu_mhd_advance_ct_fp64_matches_oracle(N):
 
 @pytest.mark.gpu
 @gpu
-@pytest.mark.parametrize("N", [2, 3, 7, 9, 31, 33, 50, 65, 111, 112, 128])
+@pytest.mark.parametrize("N", [2, 3, 7, 9, 31, 33, 50, 65, 81, 111, 112, 128])
 def test_gpu_mhd_ragged_tiles(N):
     """Cubes that the 8 x 32 column tiles do not divide: smaller than a tile,
-    one cell more or less than whole tiles, and a short last segment; and the
+    one cell more or less than whole tiles, and a short last segment (33, 50,
+    65 and 81 take tiles of 7 x 33, 10 x 25, 11 x 22 and 9 x 27 columns, so 231
+    to 250 of 256 lanes); and the
     sizes around the one from which the passes bypass the cache (112, and 128
     whole tiles).  FP64 against the oracle at the bar of the other sizes; mixed against FP64 at
     the bar of test_gpu_mhd_mixed_tracks_fp64."""
