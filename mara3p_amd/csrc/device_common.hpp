@@ -261,6 +261,28 @@ __device__ __forceinline__ double lane_after(double x, double edge)
                             __builtin_amdgcn_update_dpp(__double2loint(edge), __double2loint(x), 0x130, 0xf, 0xf, false));
 }
 
+// The same where the first / last lane's value is of no use (it is 0): the
+// compiler can make the shift part of the instruction that takes the value
+// (fused 1D step: 20 of 50 shifts, 3 to 4 % of the step).
+__device__ __forceinline__ float lane_before(float x)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float lane_after(float x)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x130, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double lane_before(double x)
+{
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x138, 0xf, 0xf, true),
+                            __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double lane_after(double x)
+{
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x130, 0xf, 0xf, true),
+                            __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x130, 0xf, 0xf, true));
+}
+
 // XCD-aware workgroup remap.  Workgroups are dispatched round-robin over the
 // 8 XCDs (each with its own L2); give each XCD a contiguous range of logical
 // tiles so that tiles sharing halo rows share an L2.

@@ -15,8 +15,8 @@
 // A workgroup per 64-zone block, a lane per zone, needed 69 and 65 faces of 64
 // lanes in the two stages, two nearly empty passes out of four, took two
 // slopes per face and met four barriers.  512 problems of 512 to 8192 zones in
-// blocks of 64: 55 to 47 us a step (553 VALU instructions per 56 zones, 965 per
-// 64 before; 190 MB, 4.0 TB/s), with the CFL reduction at half that size 52 to
+// blocks of 64: 55 to 45 us a step (some 530 VALU instructions per 56 zones, 965
+// per 64 before; 201 MB, 4.5 TB/s), with the CFL reduction at half that size 52 to
 // 36, 300 problems in blocks of 16 16.7 to 8.9.  One-wave workgroups: 48 us,
 // with the CFL reduction 48.
 //
@@ -42,10 +42,6 @@ namespace m3p {
 
 constexpr int kWindow1D = 56;          // zones a wave updates
 constexpr int kWindowGroup = 4;        // waves of a workgroup
-
-// (the first / last lane of the wave keeps its own)
-__device__ __forceinline__ float lane_before(float x) { return lane_before(x, x); }
-__device__ __forceinline__ float lane_after(float x) { return lane_after(x, x); }
 
 static __global__ void __launch_bounds__(64 * kWindowGroup)
 rk2_fused_1d_kernel(EulerParams prm, Stage1DArgs a)

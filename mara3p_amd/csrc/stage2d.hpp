@@ -428,8 +428,16 @@ stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
     // fetched at the top of an iteration, so their latency overlaps the
     // iteration's arithmetic (a scheme with late_base loads the RK base at the
     // update instead, holding fewer registers across the row).
-    auto before = [&] (R x, R e) { const R y = lane_before(x, e); return G > 1 && t == 0 ? e : y; };
-    auto after = [&] (R x, R e) { const R y = lane_after(x, e); return G > 1 && t == TJ - 1 ? e : y; };
+    auto before = [&] (R x, R e) {
+        if constexpr (G == 1) return lane_before(x, e);
+        const R y = lane_before(x);
+        return t == 0 ? e : y;
+    };
+    auto after = [&] (R x, R e) {
+        if constexpr (G == 1) return lane_after(x, e);
+        const R y = lane_after(x);
+        return t == TJ - 1 ? e : y;
+    };
     auto march = [&] (auto dir) {
         constexpr int D = decltype(dir)::value;
         const int kfirst = D > 0 ? tc.k0 + g * HS : tc.k0 + g * HS + HS - 1;
