@@ -63,11 +63,9 @@ constexpr int kSlotCflRate = 3008;           // kRateSlots words
 struct StreamState {
     int* err = nullptr;                  // int[4]: code, block, zone
     unsigned long long* red = nullptr;   // kRedWords words
-    int cus = 0;                         // compute units of the device
 };
 
 struct DeviceState {
-    int cus = 0;
     std::unordered_map<hipStream_t, StreamState> streams;
     std::vector<int*> free_latches;
 };
@@ -91,14 +89,6 @@ int new_latch(int** out)
     return hip_check(hipMemcpy(*out, zero, sizeof(zero), hipMemcpyHostToDevice), "hipMemcpy(error latch)");
 }
 
-int device_cus(DeviceState& d, int dev)
-{
-    if (d.cus == 0)
-        if (int st = hip_check(hipDeviceGetAttribute(&d.cus, hipDeviceAttributeMultiprocessorCount, dev),
-                               "hipDeviceGetAttribute")) return st;
-    return M3P_OK;
-}
-
 // The state of (current device, stream), created on first use.  Creating it
 // allocates, which a stream under graph capture must not do: the first call
 // on a stream has to come before its capture begins (m3p_graph_begin does it).
@@ -115,9 +105,7 @@ int stream_state(void* stream, StreamState** out)
     if (s && hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone)
         return fail(M3P_ERR_BAD_ARGUMENT, "m3p: the first call on a stream must come before its graph capture "
                                           "(begin captures with m3p_graph_begin)");
-    if (int st = device_cus(d, dev)) return st;
     StreamState ss;
-    ss.cus = d.cus;
     if (int st = new_latch(&ss.err)) return st;
     if (int st = hip_check(hipMalloc(&ss.red, kRedWords * sizeof(unsigned long long)), "hipMalloc(reduction)")) {
         (void)hipFree(ss.err);
@@ -131,7 +119,6 @@ int stream_state(void* stream, StreamState** out)
 // the call's kernels have finished, cleared if set, and given back.
 struct Lease {
     int* latch = nullptr;
-    int cus = 0;
     int dev = -1;
     bool pending = false;      // kernels may still write the latch
     hipStream_t stream = nullptr;
@@ -143,8 +130,6 @@ struct Lease {
         {
             std::lock_guard<std::mutex> lock(g_mutex);
             DeviceState& d = g_dev[dev];
-            if (int st = device_cus(d, dev)) return st;
-            cus = d.cus;
             if (!d.free_latches.empty()) {
                 latch = d.free_latches.back();
                 d.free_latches.pop_back();
@@ -518,7 +503,7 @@ int m3p_euler1d_updated_conserved(const double* uc, const double* pe, double* ou
     a.u = uc; a.out = out; a.dt = dt; a.dl = dl; a.rk_b = 0.5; a.n = n; a.nblk = 1; a.err = lease.latch;
     a.pe = pe; a.outflow_lower = outflow_lower; a.outflow_upper = outflow_upper;
     hipStream_t s = (hipStream_t)stream;
-    int st = precision == M3P_FP64 ? launch_stage1d<double>(prm, a, s, lease.cus) : launch_stage1d<float>(prm, a, s, lease.cus);
+    int st = precision == M3P_FP64 ? launch_stage1d<double>(prm, a, s) : launch_stage1d<float>(prm, a, s);
     if (st) return st;
     return lease.finish();
 }
@@ -719,7 +704,7 @@ int m3p_euler1d_stage(const double* u, const double* u0, double* out, const int*
     a.u = u; a.u0 = u0; a.out = out; a.nbr = nbr; a.dt = dt; a.dl = dl; a.rk_b = rk_b;
     a.n = n; a.nblk = nblk; a.err = ds->err;
     hipStream_t s = (hipStream_t)stream;
-    return precision == M3P_FP64 ? launch_stage1d<double>(prm, a, s, ds->cus) : launch_stage1d<float>(prm, a, s, ds->cus);
+    return precision == M3P_FP64 ? launch_stage1d<double>(prm, a, s) : launch_stage1d<float>(prm, a, s);
 }
 
 int m3p_euler_cfl_dt(const double* u, int nblk, long zones_per_block, double gamma_law_index,
@@ -932,7 +917,7 @@ static int euler1d_stage_blocks(const double* u, const double* u0, double* out, 
     a.u = u; a.u0 = u0; a.out = out; a.nbr = nbr; a.dt = dt; a.dt_dev = dt_dev; a.dl_blk = dl_blk; a.rk_b = rk_b;
     a.n = n; a.nblk = nblk; a.err = ds->err; a.rate_slot = rate_slot;
     hipStream_t s = (hipStream_t)stream;
-    return precision == M3P_FP64 ? launch_stage1d<double>(prm, a, s, ds->cus) : launch_stage1d<float>(prm, a, s, ds->cus);
+    return precision == M3P_FP64 ? launch_stage1d<double>(prm, a, s) : launch_stage1d<float>(prm, a, s);
 }
 
 int m3p_euler1d_stage_blocks(const double* u, const double* u0, double* out, const int* nbr, const double* dl_blk,

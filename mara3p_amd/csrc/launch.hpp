@@ -40,9 +40,9 @@ template<class S>
 int launch_rk2_fused(const typename S::Params& p1, const typename S::Params& p2, const MeshLoader<S>& ld,
                      const StageArgs& a, hipStream_t s);
 
-// One 1D work-list stage; cus = compute units of the device (grid sizing).
+// One 1D work-list stage; blocks of 16, 32, 64, 128 or a multiple of 256 zones.
 template<typename R>
-int launch_stage1d(const EulerParams& prm, const Stage1DArgs& a, hipStream_t s, int cus);
+int launch_stage1d(const EulerParams& prm, const Stage1DArgs& a, hipStream_t s);
 
 // One fused RK2 step (both stages in one launch, mixed precision) over the
 // 1D work-list: a.u the state, a.out the result, a.rk_b the RK weight of the

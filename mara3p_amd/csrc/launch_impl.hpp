@@ -1,7 +1,7 @@
 // Definitions of the stage launchers declared in launch.hpp, included only by
 // the k_*.hip units that instantiate them (M3P_INSTANTIATE_* below).
 #pragma once
-#include <algorithm>
+#include <climits>
 #include "launch.hpp"
 #include "viscous2d.hpp"
 
@@ -60,37 +60,16 @@ int launch_visc(const typename S::Params& prm, const Ld& ld, const StageArgs& a,
 }
 
 template<typename R>
-int launch_stage1d(const EulerParams& prm, const Stage1DArgs& a, hipStream_t s, int cus)
+int launch_stage1d(const EulerParams& prm, const Stage1DArgs& a, hipStream_t s)
 {
     const int n = a.n;
-    // persistent grid: 16 (FP64) or 32 (mixed) waves per CU, somewhat above
-    // what is resident at once (about 160 and 100 VGPRs: 12 and 20 waves);
-    // the excess workgroups start as others finish.  A grid of exactly the
-    // resident workgroups (the runtime's occupancy query) measured 1.5 %
-    // faster in FP64 and 3 % slower in the mixed second stage.
-    const int waves_per_cu = is_fp64<R>::value ? 16 : 32;
-    // a list of at most two items per CU: one item a workgroup, with lanes of
-    // their own for its guard zones and left face
-    auto go = [&] (auto kern, auto single, int TJ) {
-        const long items = (long)a.nblk * (n / TJ);
-        if (items <= 2l * cus) {
-            hipLaunchKernelGGL(single, dim3((int)items), dim3(stage1d_lanes(TJ, true)), 0, s, prm, a);
-            return launch_status("stage1d_kernel");
-        }
-        const int wgs_per_cu = std::max(1, waves_per_cu / std::max(1, TJ / 64));
-        const int grid = (int)std::min<long>(items, (long)std::max(cus, 1) * wgs_per_cu);
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(TJ), 0, s, prm, a);
-        return launch_status("stage1d_kernel");
-    };
-    switch (n) {
-        case 16:  return go(stage1d_kernel<R, 16, false>, stage1d_kernel<R, 16, true>, 16);
-        case 32:  return go(stage1d_kernel<R, 32, false>, stage1d_kernel<R, 32, true>, 32);
-        case 64:  return go(stage1d_kernel<R, 64, false>, stage1d_kernel<R, 64, true>, 64);
-        case 128: return go(stage1d_kernel<R, 128, false>, stage1d_kernel<R, 128, true>, 128);
-        default:
-            if (n >= 256 && n % 256 == 0) return go(stage1d_kernel<R, 256, false>, stage1d_kernel<R, 256, true>, 256);
-    }
-    return fail(M3P_ERR_BAD_SHAPE, "m3p: 1D block size must be 16, 32, 64, 128 or a multiple of 256 (got " + std::to_string(n) + ")");
+    if (n != 16 && n != 32 && n != 64 && n != 128 && (n < 256 || n % 256 != 0))
+        return fail(M3P_ERR_BAD_SHAPE, "m3p: 1D block size must be 16, 32, 64, 128 or a multiple of 256 (got " + std::to_string(n) + ")");
+    constexpr long zones = (long)kWindowStage1D * kWindowGroup;
+    const long groups = ((long)a.nblk * n + zones - 1) / zones;
+    if (groups > INT_MAX) return fail(M3P_ERR_BAD_SHAPE, "m3p: too many 1D blocks for one launch");
+    hipLaunchKernelGGL(stage1d_kernel<R>, dim3((unsigned)groups), dim3(64 * kWindowGroup), 0, s, prm, a);
+    return launch_status("stage1d_kernel");
 }
 
 } // namespace m3p

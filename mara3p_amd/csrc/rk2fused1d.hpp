@@ -41,7 +41,6 @@
 namespace m3p {
 
 constexpr int kWindow1D = 56;          // zones a wave updates
-constexpr int kWindowGroup = 4;        // waves of a workgroup
 
 static __global__ void __launch_bounds__(64 * kWindowGroup)
 rk2_fused_1d_kernel(EulerParams prm, Stage1DArgs a)

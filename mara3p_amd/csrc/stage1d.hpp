@@ -3,12 +3,25 @@
 //   modules::euler1d::updated_conserved, src/module_euler.cpp:107-135
 //   outflow boundary condition,           src/mara.cpp:123-143
 //
-// A workgroup of TJ threads owns TJ zones of one block.  Primitives of the TJ
-// zones and four guard zones go to LDS; each lane computes the right face of
-// its zone (from the half slopes at its zone and the next, the latter also
-// computed by the next lane, from the same operands), and the left faces of
-// TJ items at a time come from one pass of all lanes.  Every face flux is
-// computed once.
+// A wave owns 60 zones, consecutive in storage, and holds them in its lanes 2 ..
+// 61 with the two zones before and after: each lane recovers its zone and takes
+// one half slope, one face flux (the left face of its zone) and one update, with
+// its neighbours' values by wave shifts.  Every face flux is computed once in a
+// window; nothing passes through LDS and nothing waits at a barrier.
+//
+// A workgroup per block with LDS rows took both slopes of every face, met two
+// barriers and needed a pass of its own for the left faces; it was bound by its
+// arithmetic.  512 problems of 512 to 8192 zones in blocks of 64, both stages,
+// FP64: 149 to 100 us (445 MB, 4.5 TB/s: bound by memory); 64 problems in blocks
+// of 128, 22.6 to 18.1; 1688 blocks of 32, 17.9 to 10.2; 1024 zones, a launch
+// 4.5 to 4.1.
+//
+// Zones of a window are one chain where every block boundary in it joins blocks
+// that are linked and consecutive in storage (nearly always).  Else the window is
+// done in pieces, each piece's lanes finding their zones from the piece's first
+// zone along the prev/next links: a neighbour stored elsewhere, or a copy of the
+// edge zone past an outflow end.  A piece ends where the next block's own prev
+// link does not lead back (its guard zones are not this chain's).
 #pragma once
 #include "physics.hpp"
 
@@ -32,209 +45,118 @@ struct Stage1DArgs {
     unsigned long long* rate_slot;
 };
 
-// Persistent work-list form: the grid is sized to the device and each
-// workgroup walks the list of (block, tile) items with a fixed stride, so one
-// launch covers any number of blocks of any mix of problems.
-//
-// SINGLE: every workgroup has one item (the list is shorter than the grid).
-// Such a launch is bound by one item's chain of loads, faces and barriers, so
-// further lanes (a second wave where the tile fills the first) take the guard
-// zones and the left face, which otherwise a pass of its own computes before
-// (FP64) or after (mixed) the other faces.  1024 zones in blocks of 64:
-// 4.4 us a launch against 6.4 in FP64, 4.0 against 4.1 mixed; 400 blocks of 64,
-// FP64: 5.1 against 7.1.
-constexpr int stage1d_lanes(int TJ, bool single) { return !single ? TJ : TJ + 5 <= 64 ? 64 : TJ + 64; }
+constexpr int kWindowStage1D = 60;     // zones a wave updates
+constexpr int kWindowGroup = 4;        // waves of a workgroup
 
-template<typename R, int TJ, bool SINGLE>
-__global__ void __launch_bounds__(stage1d_lanes(TJ, SINGLE))
+template<typename R>
+__global__ void __launch_bounds__(64 * kWindowGroup)
 stage1d_kernel(EulerParams prm, Stage1DArgs a)
 {
     constexpr int NC = 5;
-    constexpr int NT = stage1d_lanes(TJ, SINGLE);
-    constexpr int GL = SINGLE ? TJ : 0;     // first of the four lanes that load guard zones
     const int n = a.n;
-    const int tiles = n / TJ;
-    const long items = (long)a.nblk * tiles;
-    const int t = threadIdx.x;
-    const bool zone = !SINGLE || t < TJ;    // the lane has a zone of the item
-    const int g = t - GL;                   // 0 .. 3: the lane's guard zone
+    const int i = threadIdx.x & 63;
+    const long total = (long)a.nblk * n;
+    // The second RK stage (u0 given) walks the list backwards: its first reads
+    // are what the first stage wrote last (likeliest to be cached).
+    const long group = a.u0 ? (long)gridDim.x - 1 - blockIdx.x : blockIdx.x;
+    const long first = (group * kWindowGroup + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * kWindowStage1D;
+    const long end = first + kWindowStage1D < total ? first + kWindowStage1D : total;
     const R theta = R(prm.theta);
     const double dt = a.dt_dev ? *a.dt_dev : a.dt;
+    double rate = 0.0;                      // fused CFL reduction
 
-    // FP64 (bound by its arithmetic) computes the left faces of TJ items in
-    // one pass of all lanes; the mixed kernel (bound by memory latency) lets
-    // lane 0 compute its item's left face from the LDS row, which needs no
-    // further loads.
-    constexpr bool kGroupLeftFaces = is_fp64<R>::value && !SINGLE;
-    __shared__ R P[NC][TJ + 4];   // [i] = zone c0 - 2 + i
-    __shared__ R F[NC][TJ + 1];   // [i] = face c0 + i (left face of zone c0 + i)
-    __shared__ R Fl[NC][kGroupLeftFaces ? TJ : 1];   // left face of each item of the current group
-
-    // The lane's own zone of the next item, and for lanes 0-3 the four guard
-    // zones of that item (c0 - 2, c0 - 1, c0 + TJ, c0 + TJ + 1: neighbour
-    // block, or the edge zone at an outflow boundary), are fetched while the
-    // current item is computed (software pipelining across the work list).
-    // The second RK stage (u0 given) walks the list backwards: its first
-    // reads are what the first stage wrote last (likeliest to be cached).
-    const bool rev = a.u0 != nullptr;
-    auto slot = [&] (long it) { return rev ? items - 1 - it : it; };
-    auto guard_zone = [&] (int b, int i) {
-        // zone index i in [-2, 0) or [n, n+2) of block b
-        int bb = b, z = i;
-        if (i < 0) {
-            int pb = a.nbr[2 * b];
-            if (pb < 0) z = 0; else { bb = pb; z = i + n; }
-        } else if (i >= n) {
-            int nb = a.nbr[2 * b + 1];
-            if (nb < 0) z = n - 1; else { bb = nb; z = i - n; }
-        }
-        return a.u + (size_t)bb * NC * n + z;
-    };
-    auto fetch = [&] (long it, double* raw, double* graw) {
-        it = slot(it);
-        const int b = (int)(it / tiles), c0 = (int)(it % tiles) * TJ;
-        if (zone) {
-            const double* src = a.u + (size_t)b * NC * n + c0 + t;
+    for (long lo = first; lo < end;) {
+        // block and zone of lo, then of each lane along the storage order
+        const int b0 = total < (1l << 31) ? (int)((unsigned)lo / (unsigned)n) : (int)(lo / n);
+        const int p0 = (int)(lo - (long)b0 * n) + i - 2;      // the lane's zone counted from block b0's first
+        int b = b0, z = p0;
+        while (z >= n) { ++b; z -= n; }
+        if (z < 0) { --b; z += n; }
+        const bool inside = !a.pe && lo >= 2 && lo + 62 <= total;
+        int prev = b - 1, next = b;                           // the links across the boundary before the lane's zone
+        if (inside && i > 0 && z == 0) { prev = a.nbr[2 * b]; next = a.nbr[2 * (b - 1) + 1]; }
+        // the state is fetched before the links are known (the latencies
+        // overlap), and again by the pieces that do not follow the storage
+        double u[NC], u0[NC] = {};
+        double dl = a.dl;
+        auto fetch = [&] () {
+            const size_t at = (size_t)b * NC * n + z;
 #pragma unroll
-            for (int q = 0; q < NC; ++q) raw[q] = src[(size_t)q * n];
-        }
-        if (!a.pe && g >= 0 && g < 4) {
-            const double* src = guard_zone(b, g < 2 ? c0 - 2 + g : c0 + TJ + (g - 2));
+            for (int q = 0; q < NC; ++q) u[q] = a.u[at + (size_t)q * n];
+            if (a.u0) {
 #pragma unroll
-            for (int q = 0; q < NC; ++q) graw[q] = src[(size_t)q * n];
-        }
-    };
-    double nxt[NC] = {}, gnxt[NC] = {};
-    if (blockIdx.x < items) fetch(blockIdx.x, nxt, gnxt);
-
-    // extended-array mode (per-block compatibility): zone index i in
-    // [-2, n+2) of the caller's primitive array
-    auto load_pe = [&] (int i, R* p) {
-        int e = i;
-        if (a.outflow_lower && i < 0) e = 0;
-        else if (!a.outflow_lower && a.outflow_upper && i >= n) e = n - 1;
-        for (int q = 0; q < NC; ++q) p[q] = R(a.pe[(size_t)q * (n + 4) + e + 2]);
-    };
-    // The left face of item `it` (zones c0 - 2 .. c0 + 1), with the operands
-    // and arithmetic of every other face.  A tile of TJ zones has TJ + 1
-    // faces; each lane computes the right face of its zone, and the left
-    // faces of a group of TJ items come from one pass of all lanes, so no
-    // item needs a second, nearly idle flux pass.  Recovery errors in these
-    // zones are reported by the items that own them.
-    auto left_face = [&] (long it, R* f) {
-        const int b = (int)(it / tiles), c0 = (int)(it % tiles) * TJ;
-        R pz[4][NC];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int i = c0 - 2 + r;
-            if (a.pe) {
-                load_pe(i, pz[r]);
-            } else {
-                const double* src = i < 0 ? guard_zone(b, i) : a.u + (size_t)b * NC * n + i;
-                double uu[NC];
-#pragma unroll
-                for (int q = 0; q < NC; ++q) uu[q] = src[(size_t)q * n];
-                (void)Euler<R>::recover(uu, prm, pz[r]);
+                for (int q = 0; q < NC; ++q) u0[q] = a.u0[at + (size_t)q * n];
             }
-        }
-        R pl[NC], pr[NC];
-#pragma unroll
-        for (int q = 0; q < NC; ++q) {
-            pl[q] = pz[1][q] + plm_half(pz[0][q], pz[1][q], pz[2][q], theta);
-            pr[q] = pz[2][q] - plm_half(pz[1][q], pz[2][q], pz[3][q], theta);
-        }
-        Euler<R>::template riemann<1>(pl, pr, prm, f);
-    };
-
-    bool ok = true;
-    double rate = 0.0;                  // fused CFL reduction
-    for (long item = blockIdx.x; item < items; item += gridDim.x) {
-        // position of this item in its group of TJ consecutive items of this
-        // workgroup; the group's left faces are computed at its first item
-        const int gpos = (int)(((item - blockIdx.x) / gridDim.x) % TJ);
-        if (kGroupLeftFaces && gpos == 0) {
-            const long li = item + (long)t * gridDim.x;
-            if (li < items) {
-                R f[NC];
-                left_face(slot(li), f);
-#pragma unroll
-                for (int q = 0; q < NC; ++q) Fl[q][t] = f[q];
-            }
-        }
-        const long it = slot(item);
-        const int b = (int)(it / tiles);
-        const int c0 = (int)(it % tiles) * TJ;
-        const double dl = a.dl_blk ? a.dl_blk[b] : a.dl;
-        const double idl = a.rate_slot ? 1.0 / dl : 0.0;
-        double uz[NC], gz[NC], U0[NC];
-#pragma unroll
-        for (int q = 0; q < NC; ++q) { uz[q] = nxt[q]; gz[q] = gnxt[q]; }
-        if (item + gridDim.x < items) fetch(item + gridDim.x, nxt, gnxt);
-        if (a.u0 && zone) {
-#pragma unroll
-            for (int q = 0; q < NC; ++q) U0[q] = a.u0[(size_t)b * NC * n + (size_t)q * n + c0 + t];
-        }
-        R p[NC];
-        if (zone) {
-            if (a.pe) load_pe(c0 + t, p);
-            else ok &= Euler<R>::recover(uz, prm, p);
-            for (int q = 0; q < NC; ++q) P[q][t + 2] = p[q];
-        }
-        if (g >= 0 && g < 4) {
-            if (a.pe) load_pe(g < 2 ? c0 - 2 + g : c0 + TJ + (g - 2), p);
-            else ok &= Euler<R>::recover(gz, prm, p);
-            int slot = g < 2 ? g : TJ + 2 + (g - 2);
-            for (int q = 0; q < NC; ++q) P[q][slot] = p[q];
-        }
-        __syncthreads();
-        // face i of the tile (the left face of zone c0 + i), from the half
-        // slopes at zones c0 + i - 1 and c0 + i
-        auto face = [&] (int i) {
-            R pl[NC], pr[NC], f[NC];
-#pragma unroll
-            for (int q = 0; q < NC; ++q) {
-                pl[q] = P[q][i + 1] + plm_half(P[q][i], P[q][i + 1], P[q][i + 2], theta);
-                pr[q] = P[q][i + 2] - plm_half(P[q][i + 1], P[q][i + 2], P[q][i + 3], theta);
-            }
-            Euler<R>::template riemann<1>(pl, pr, prm, f);
-#pragma unroll
-            for (int q = 0; q < NC; ++q) F[q][i] = f[q];
+            if (a.dl_blk) dl = a.dl_blk[b];
         };
-        if constexpr (SINGLE) {
-            if (t <= TJ) face(t < TJ ? t + 1 : 0);
-        } else {
-            face(t + 1);                    // the right face of the lane's zone
-            if (t == 0) {
-                if constexpr (kGroupLeftFaces) {
-#pragma unroll
-                    for (int q = 0; q < NC; ++q) F[q][0] = Fl[q][gpos];
-                } else {
-                    face(0);
+        if (inside) fetch();
+        int count = (int)(end - lo);                          // zones this piece updates
+        if (__builtin_expect(__ballot(inside && prev == b - 1 && next == b) != ~0ull, 0)) {
+            b = b0;
+            z = p0;
+            bool cut = false;                                 // past an end of the piece's chain
+            if (a.pe) {
+                cut = z >= n;
+                z = min(max(z, 0), n - 1);
+            } else if (z < 0) {
+                const int pb = a.nbr[2 * b];
+                if (pb >= 0) { b = pb; z += n; }
+                else z = 0;
+            } else {
+                while (z >= n) {
+                    const int nb = a.nbr[2 * b + 1];
+                    cut |= nb < 0 || a.nbr[2 * nb] != b;
+                    if (nb >= 0) { b = nb; z -= n; }
+                    else z = n - 1;
                 }
             }
+            const unsigned long long other = __ballot(i >= 2 && (cut || (long)b * n + z != lo + (i - 2)));
+            if (other) count = min(count, __builtin_ctzll(other) - 2);
+            fetch();
         }
-        __syncthreads();
+        const bool mine = i >= 2 && i < 2 + min(count, kWindowStage1D);
 
-        const int z = c0 + t;
-        double* o = a.out + (size_t)b * NC * n + z;
+        bool ok = true;
+        R p[NC], pl[NC], pr[NC], f[NC];
+        if (a.pe) {
+            // extended-array mode (per-block compatibility): zones -2 .. n + 1 of
+            // the caller's primitive array
+            int e = min(p0, n + 1);
+            if (a.outflow_lower && e < 0) e = 0;
+            else if (!a.outflow_lower && a.outflow_upper && e >= n) e = n - 1;
+#pragma unroll
+            for (int q = 0; q < NC; ++q) p[q] = R(a.pe[(size_t)q * (n + 4) + e + 2]);
+        } else {
+            ok = Euler<R>::recover(u, prm, p);
+        }
+        // the left face of the lane's zone, from the half slopes of this zone
+        // and the one before
+#pragma unroll
+        for (int q = 0; q < NC; ++q) {
+            const R g = plm_half(lane_before(p[q]), p[q], lane_after(p[q]), theta);
+            pl[q] = lane_before(p[q] + g);
+            pr[q] = p[q] - g;
+        }
+        Euler<R>::template riemann<1>(pl, pr, prm, f);
         double wv[NC];
         const Divisor<double> by_dl(dl);
-        if (zone) for (int q = 0; q < NC; ++q) {
-            double dfx = double(F[q][t + 1]) - double(F[q][t]);
-            double res;
-            if constexpr (is_fp64<R>::value) res = uz[q] - by_dl(dfx * dt);
-            else res = uz[q] - dfx * (dt / dl);
-            if (a.u0) res = U0[q] * a.rk_b + res * (1.0 - a.rk_b);
-            o[(size_t)q * n] = res;
-            wv[q] = res;
+#pragma unroll
+        for (int q = 0; q < NC; ++q) {
+            const double dfx = double(lane_after(f[q])) - double(f[q]);
+            if constexpr (is_fp64<R>::value) wv[q] = u[q] - by_dl(dfx * dt);
+            else wv[q] = u[q] - dfx * (dt / dl);
+            if (a.u0) wv[q] = u0[q] * a.rk_b + wv[q] * (1.0 - a.rk_b);
         }
-        if (a.rate_slot && zone) rate = fmax(rate, Euler<double>::max_speed(wv, prm) * idl);
-        if (!ok) { report_error(a.err, 1, b, z); ok = true; }
-        // No barrier here: the next item writes P and Fl only after this
-        // item's flux barrier, which every read of them precedes, and F only
-        // after its own first barrier, which follows this item's update.
+        if (mine) {
+            double* o = a.out + (size_t)b * NC * n + z;
+#pragma unroll
+            for (int q = 0; q < NC; ++q) o[(size_t)q * n] = wv[q];
+            if (!ok) report_error(a.err, 1, b, z);
+            if (a.rate_slot) rate = fmax(rate, Euler<double>::max_speed(wv, prm) * (1.0 / dl));
+        }
+        lo += count;
     }
-    if (a.rate_slot) workgroup_atomic_max<NT>(rate, a.rate_slot);
+    if (a.rate_slot) workgroup_atomic_max<64 * kWindowGroup>(rate, a.rate_slot);
 }
 
 } // namespace m3p

@@ -362,9 +362,7 @@ def test_euler1d_mesh_every_block_size(n, nblk):
 
 @pytest.mark.parametrize("n,nblk", [(16, 512), (16, 700), (32, 530), (64, 513), (128, 520), (256, 530), (512, 300)])
 def test_euler1d_long_lists(n, nblk):
-    """Lists of items at and past two per CU, where workgroups of one item
-    each give way to the persistent list, in every tile width: FP64 equals the
-    oracle, mixed stays near it, and the CFL reduction of the second stage
+    """Long lists in blocks of every size: FP64 equals the oracle, mixed stays near it, and the CFL reduction of the second stage
     equals the separate one."""
     from mara3p_amd.mesh import EnsembleMesh1D
     from mara3p_amd.solvers import Euler1DEnsembleSolver
@@ -388,6 +386,55 @@ def test_euler1d_long_lists(n, nblk):
         else:
             assert rel_err(s.state(), ref.transpose(0, 2, 1)) <= 1e-5
         assert float(dt_next.item()) == float(s.cfl_dt(0.4).item())
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("n", [16, 32, 64, 128, 256])
+def test_euler1d_stage_follows_the_links(n, precision):
+    """Stages over tables whose links leave the storage order, against the same
+    chains stored in order, block by block: blocks stored backwards and
+    shuffled; and a table with links that do not lead back (every other block
+    an outflow start that its predecessor still reads), against the chains
+    that each block's own links describe."""
+    from mara3p_amd.mesh import EnsembleMesh1D
+    from mara3p_amd.solvers import Euler1DEnsembleSolver
+    rng = np.random.default_rng(n)
+    m = 11
+    rho, v, p = 1 + rng.random((m, n)), 0.5 * rng.standard_normal((m, n)), 0.5 + rng.random((m, n))
+    u0 = np.stack([rho, rho * v, 0 * v, 0.1 * rho, 0.5 * rho * (v * v + 0.01) + p / 0.4], axis=1)
+    dl = (1.0 + rng.random(m)) / (m * n)
+    dt = 0.05 * dl.min()
+    chain = np.stack([np.arange(m) - 1, np.where(np.arange(m) < m - 1, np.arange(m) + 1, -1)], axis=1)
+
+    def stage(nbr, order):
+        """One stage with a base; block k of the chain stored at order[k]."""
+        s = Euler1DEnsembleSolver(EnsembleMesh1D([m * n], n), precision=precision)
+        at = np.asarray(order)
+        table, spacing, state = np.empty((m, 2), np.int32), np.empty(m), np.empty_like(u0)
+        table[at] = np.where(nbr >= 0, at[np.maximum(nbr, 0)], -1)
+        spacing[at] = dl
+        state[at] = u0
+        s.nbr.copy_(torch.as_tensor(table))
+        s.dl.copy_(torch.as_tensor(spacing))
+        s.set_state(state)
+        s.stage(s.u, s.u, s.u1, dt)
+        s.check_errors()
+        return s.u1.cpu().numpy()[at]
+
+    ref = stage(chain, np.arange(m))
+    assert np.array_equal(stage(chain, np.arange(m)[::-1]), ref)
+    assert np.array_equal(stage(chain, rng.permutation(m)), ref)
+    # every other block starts at an outflow end that the block before reads
+    cut = chain.copy()
+    cut[1::2, 0] = -1
+    starts = chain.copy()
+    starts[1::2, 0] = -1
+    starts[0:-1:2, 1] = -1
+    apart = stage(starts, np.arange(m))
+    for order in (np.arange(m), rng.permutation(m)):
+        got = stage(cut, order)
+        assert np.array_equal(got[0::2], ref[0::2])
+        assert np.array_equal(got[1::2], apart[1::2])
 
 
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
