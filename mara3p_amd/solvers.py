@@ -355,7 +355,7 @@ class AmrEuler2DSolver(_StateSolver):
 
 class Euler1DEnsembleSolver(_StateSolver):
     """Many independent euler1d problems (outflow ends, cell spacing 1/L each)
-    advanced together by one persistent work-list launch per RK stage."""
+    advanced together by one work-list launch per RK stage."""
     nc = 5
 
     def __init__(self, mesh: EnsembleMesh1D, gamma=1.4, plm_theta=1.5, precision="fp64", device="cuda"):
