@@ -330,6 +330,10 @@ int m3p_srhd_riemann_array(const double* pl, const double* pr, double* f, long n
  * per (kind, precision), where it divides the block size. */
 int m3p_set_stage2d_tile(int kind, int precision, int tj, int h);
 int m3p_get_stage2d_tile(int kind, int precision, int* tj /* host */, int* h /* host */);
+/* The tile that a stage over nblk blocks of n x n zones takes now (the choice
+ * where it fits, else the library's); M3P_ERR_BAD_SHAPE for a block size that
+ * the stages refuse. */
+int m3p_stage2d_tile(int kind, int precision, int n, int nblk, int* tj /* host */, int* h /* host */);
 /* Time every variant that fits on the caller's mesh (u -> out, `reps`
  * launches each, blocking), keep the fastest and report it (host outputs). */
 int m3p_autotune_euler2d(const double* u, double* out, const int* nbr, int nblk, int n, double dl,

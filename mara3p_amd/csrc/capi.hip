@@ -222,6 +222,7 @@ bool tile_fits(TileShape v, int n) { return n % v.tj == 0 && n % v.h == 0 && v.h
 // HLLC 304 us, 314 with eight).
 TileShape pick_tile(int kind, int precision, int n, int nblk)
 {
+    if (n < 16) return {0, 0};             // also zero and below, which every width divides
     const int chosen = g_tile[kind][precision].load(std::memory_order_relaxed);
     if (chosen >= 0 && tile_fits(kTileVariants[chosen], n)) return kTileVariants[chosen];
     const double zones = (double)nblk * n * n;
@@ -238,12 +239,17 @@ TileShape pick_tile(int kind, int precision, int n, int nblk)
     return {0, 0};
 }
 
+int bad_block_size(int n)
+{
+    return fail(M3P_ERR_BAD_SHAPE, "m3p: 2D block size must be 16, 32 or a multiple of 64 (got " + std::to_string(n) + ")");
+}
+
 template<class S, class Ld>
 int launch_stage2d(int kind, const typename S::Params& prm, const Ld& ld, const StageArgs& a, hipStream_t s)
 {
     const int prec = is_fp64<typename S::Real>::value ? M3P_FP64 : M3P_MIXED;
     const TileShape ts = pick_tile(kind, prec, a.n, a.nblk);
-    if (ts.tj == 0) return fail(M3P_ERR_BAD_SHAPE, "m3p: 2D block size must be 16, 32 or a multiple of 64 (got " + std::to_string(a.n) + ")");
+    if (ts.tj == 0) return bad_block_size(a.n);
     return launch_stage2d_shape<S, Ld>(ts, prm, ld, a, s);
 }
 
@@ -1142,6 +1148,17 @@ int m3p_get_stage2d_tile(int kind, int precision, int* tj, int* h)
     if (kind < 0 || kind >= kNumKinds || precision < 0 || precision > 1) return fail(M3P_ERR_BAD_ARGUMENT, "m3p: bad kind/precision");
     const int i = g_tile[kind][precision].load(std::memory_order_relaxed);
     const TileShape v = i >= 0 ? kTileVariants[i] : kLargeTile[kind];
+    if (tj) *tj = v.tj;
+    if (h) *h = v.h;
+    return M3P_OK;
+}
+
+int m3p_stage2d_tile(int kind, int precision, int n, int nblk, int* tj, int* h)
+{
+    if (kind < 0 || kind >= kNumKinds || precision < 0 || precision > 1) return fail(M3P_ERR_BAD_ARGUMENT, "m3p: bad kind/precision");
+    if (nblk <= 0) return fail(M3P_ERR_BAD_ARGUMENT, "m3p: bad number of blocks");
+    const TileShape v = pick_tile(kind, precision, n, nblk);
+    if (v.tj == 0) return bad_block_size(n);
     if (tj) *tj = v.tj;
     if (h) *h = v.h;
     return M3P_OK;

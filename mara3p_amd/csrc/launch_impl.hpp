@@ -53,6 +53,7 @@ int launch_stage2d_shape(TileShape ts, const typename S::Params& prm, const Ld& 
 template<class S, class Ld>
 int launch_visc(const typename S::Params& prm, const Ld& ld, const StageArgs& a, double nu, hipStream_t s)
 {
+    if (a.n < 1) return fail(M3P_ERR_BAD_SHAPE, "m3p: 2D block size must be positive (got " + std::to_string(a.n) + ")");
     const int tiles = (a.n + kViscTile - 1) / kViscTile;
     hipLaunchKernelGGL((iso_visc_stage_kernel<S, Ld, kViscTile>), dim3(a.nblk * tiles * tiles),
                        dim3(kViscTile * kViscTile), 0, s, prm, ld, a, nu);

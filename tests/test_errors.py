@@ -152,3 +152,23 @@ def test_single_block_and_smallest_meshes():
     r1 = np.ascontiguousarray(np.moveaxis(u1, 1, -1))
     assert orc().orc_euler1d_mesh_rk2(P(r1), 1, 64, 1e-3, c.dl, 1.5, 1.4, 1, 1) == 0
     assert np.array_equal(c.state(), np.moveaxis(r1, -1, 1))
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a HIP device")
+@pytest.mark.parametrize("n", [0, -16, -64, -256])
+def test_block_sizes_below_one_are_refused(n):
+    """Nothing is launched for a block of no zones or of a negative size."""
+    L = lib()
+    a = torch.ones(64, dtype=torch.float64, device="cuda")
+    b = torch.ones_like(a)
+    nbr = torch.zeros((1, 4), dtype=torch.int32, device="cuda")
+    for precision in (M3P_FP64, M3P_MIXED):
+        assert L.m3p_euler2d_stage(_p(a), _p(None), _p(b), _p(nbr), 1, n, 1e-3, _p(None), 1.0, 0.5, 1.5, 1.4, 0,
+                                   precision, _s()) == M3P_ERR_BAD_SHAPE
+        assert L.m3p_euler2d_updated_conserved(_p(a), _p(a), _p(b), n, 1e-3, 1.0, 1.5, 1.4, 0, precision,
+                                               _s()) == M3P_ERR_BAD_SHAPE
+        for nu in (0.0, 1e-3):
+            assert L.m3p_locally_isothermal_stage(_p(a), _p(None), _p(b), _p(nbr), 1, n, 1e-3, _p(None), 1.0, 0.5,
+                                                  _p(a), _p(a), nu, precision, _s()) == M3P_ERR_BAD_SHAPE
+    torch.cuda.synchronize()
