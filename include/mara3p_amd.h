@@ -346,8 +346,9 @@ int m3p_autotune_minidisk(const double* u, double* out, const int* nbr, const in
 /* 1D Euler stage over a work-list of blocks of n zones that may belong to
  * many independent problems (an uneven ensemble): chain nbr [nblk][2] as
  * m3p_euler1d_stage (-1 = outflow end), cell spacing per block dl_blk
- * [nblk] (device).  One launch covers the list; dt_dev (device,
- * may be NULL) overrides dt. */
+ * [nblk] (device).  A link may name a block behind the list (u then holds
+ * more than nblk blocks; nbr, u0 and dl_blk have no rows for it).  One launch
+ * covers the list; dt_dev (device, may be NULL) overrides dt. */
 int m3p_euler1d_stage_blocks(const double* u, const double* u0, double* out, const int* nbr, const double* dl_blk,
                              int nblk, int n, double dt, const double* dt_dev, double rk_b,
                              double plm_theta, double gamma_law_index, int precision, void* stream);

@@ -16,12 +16,18 @@
 // of 128, 22.6 to 18.1; 1688 blocks of 32, 17.9 to 10.2; 1024 zones, a launch
 // 4.5 to 4.1.
 //
-// Zones of a window are one chain where every block boundary in it joins blocks
-// that are linked and consecutive in storage (nearly always).  Else the window is
-// done in pieces, each piece's lanes finding their zones from the piece's first
-// zone along the prev/next links: a neighbour stored elsewhere, or a copy of the
-// edge zone past an outflow end.  A piece ends where the next block's own prev
-// link does not lead back (its guard zones are not this chain's).
+// A window is one chain where every block boundary in it joins blocks that are
+// linked both ways and consecutive in storage.  At any other boundary (an end of
+// a chain, a neighbour stored elsewhere, links that do not lead back) the lanes
+// on its two sides load the two guard zones of their own block's link
+// themselves: blocks are at least 16 zones, so a lane has one such side at
+// most, and one more pass of the left face's arithmetic gives the right faces
+// of all chains that end in the window.  Links are read for blocks of the list
+// only; a neighbour may be stored behind the list, with no row of its own.  Both
+// stages, mixed: the 512 problems above in shuffled order 91 us (76 in order),
+// blocks of 16 of 512 problems of 64 to 1024 zones 21 (17), 4096 problems of one
+// block of 64 zones 19.6; done in pieces, each from its first zone along the
+// links, they took 141, 60 and 24.
 #pragma once
 #include "physics.hpp"
 
@@ -48,8 +54,10 @@ struct Stage1DArgs {
 constexpr int kWindowStage1D = 60;     // zones a wave updates
 constexpr int kWindowGroup = 4;        // waves of a workgroup
 
+// FP64 at four waves per SIMD (124 VGPRs): left to itself the compiler takes 132
+// and three waves (512 problems in order 102 us, 90 at four).
 template<typename R>
-__global__ void __launch_bounds__(64 * kWindowGroup)
+__global__ void __launch_bounds__(64 * kWindowGroup) __attribute__((amdgpu_waves_per_eu(is_fp64<R>::value ? 4 : 6, 8)))
 stage1d_kernel(EulerParams prm, Stage1DArgs a)
 {
     constexpr int NC = 5;
@@ -59,102 +67,137 @@ stage1d_kernel(EulerParams prm, Stage1DArgs a)
     // The second RK stage (u0 given) walks the list backwards: its first reads
     // are what the first stage wrote last (likeliest to be cached).
     const long group = a.u0 ? (long)gridDim.x - 1 - blockIdx.x : blockIdx.x;
-    const long first = (group * kWindowGroup + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * kWindowStage1D;
-    const long end = first + kWindowStage1D < total ? first + kWindowStage1D : total;
+    const long lo = (group * kWindowGroup + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * kWindowStage1D;
+    const long end = lo + kWindowStage1D < total ? lo + kWindowStage1D : total;
     const R theta = R(prm.theta);
     const double dt = a.dt_dev ? *a.dt_dev : a.dt;
     double rate = 0.0;                      // fused CFL reduction
 
-    for (long lo = first; lo < end;) {
-        // block and zone of lo, then of each lane along the storage order
+    if (lo < end) {
+        // block and zone of lo, then of each lane along the storage order; a
+        // lane before the list or past it holds a zone inside, of no use
         const int b0 = total < (1l << 31) ? (int)((unsigned)lo / (unsigned)n) : (int)(lo / n);
         const int p0 = (int)(lo - (long)b0 * n) + i - 2;      // the lane's zone counted from block b0's first
         int b = b0, z = p0;
         while (z >= n) { ++b; z -= n; }
         if (z < 0) { --b; z += n; }
-        const bool inside = !a.pe && lo >= 2 && lo + 62 <= total;
-        int prev = b - 1, next = b;                           // the links across the boundary before the lane's zone
-        if (inside && i > 0 && z == 0) { prev = a.nbr[2 * b]; next = a.nbr[2 * (b - 1) + 1]; }
-        // the state is fetched before the links are known (the latencies
-        // overlap), and again by the pieces that do not follow the storage
+        const bool there = b >= 0 && b < a.nblk;
+        const bool edge = !a.pe && i > 0 && z == 0 && b >= 0 && b <= a.nblk;   // a boundary before the lane's zone
+        int prev = -1, next = -1;                             // the links across it
+        if (edge) {
+            if (there) prev = a.nbr[2 * b];
+            if (b > 0) next = a.nbr[2 * (b - 1) + 1];
+        }
+        const bool cut = edge && !(there && b > 0 && prev == b - 1 && next == b);
+        if (!there) { b = b0; z = min(max(p0, 0), n - 1); }
+        const size_t at = (size_t)b * NC * n + z;
         double u[NC], u0[NC] = {};
         double dl = a.dl;
-        auto fetch = [&] () {
-            const size_t at = (size_t)b * NC * n + z;
 #pragma unroll
-            for (int q = 0; q < NC; ++q) u[q] = a.u[at + (size_t)q * n];
-            if (a.u0) {
+        for (int q = 0; q < NC; ++q) u[q] = a.u[at + (size_t)q * n];
+        if (a.u0) {
 #pragma unroll
-                for (int q = 0; q < NC; ++q) u0[q] = a.u0[at + (size_t)q * n];
-            }
-            if (a.dl_blk) dl = a.dl_blk[b];
-        };
-        if (inside) fetch();
-        int count = (int)(end - lo);                          // zones this piece updates
-        if (__builtin_expect(__ballot(inside && prev == b - 1 && next == b) != ~0ull, 0)) {
-            b = b0;
-            z = p0;
-            bool cut = false;                                 // past an end of the piece's chain
-            if (a.pe) {
-                cut = z >= n;
-                z = min(max(z, 0), n - 1);
-            } else if (z < 0) {
-                const int pb = a.nbr[2 * b];
-                if (pb >= 0) { b = pb; z += n; }
-                else z = 0;
-            } else {
-                while (z >= n) {
-                    const int nb = a.nbr[2 * b + 1];
-                    cut |= nb < 0 || a.nbr[2 * nb] != b;
-                    if (nb >= 0) { b = nb; z -= n; }
-                    else z = n - 1;
-                }
-            }
-            const unsigned long long other = __ballot(i >= 2 && (cut || (long)b * n + z != lo + (i - 2)));
-            if (other) count = min(count, __builtin_ctzll(other) - 2);
-            fetch();
+            for (int q = 0; q < NC; ++q) u0[q] = a.u0[at + (size_t)q * n];
         }
-        const bool mine = i >= 2 && i < 2 + min(count, kWindowStage1D);
+        if (a.dl_blk) dl = a.dl_blk[b];
+        const bool mine = i >= 2 && i < 2 + (int)(end - lo);
 
         bool ok = true;
-        R p[NC], pl[NC], pr[NC], f[NC];
-        if (a.pe) {
-            // extended-array mode (per-block compatibility): zones -2 .. n + 1 of
-            // the caller's primitive array
-            int e = min(p0, n + 1);
-            if (a.outflow_lower && e < 0) e = 0;
-            else if (!a.outflow_lower && a.outflow_upper && e >= n) e = n - 1;
+        R p[NC];
+        // dF of the lane's zone.  CUT: with first and last, the lanes on the two
+        // sides of a boundary that joins nothing, and their blocks' link there.
+        double dfx[NC];
+        auto fluxes = [&] (auto cut_c, bool first, bool last, int link) {
+            constexpr bool CUT = decltype(cut_c)::value;
+            // the two guard zones, fetched before the zone's own values arrive
+            // (copies of the edge zone at an outflow end)
+            double g1[NC] = {}, g2[NC] = {};
+            const bool away = CUT && (first || last) && link >= 0;
+            if constexpr (CUT) {
+                if (away) {
+                    const double* src = a.u + (size_t)link * NC * n + (last ? 0 : n - 1);
+                    const int step = last ? 1 : -1;
 #pragma unroll
-            for (int q = 0; q < NC; ++q) p[q] = R(a.pe[(size_t)q * (n + 4) + e + 2]);
+                    for (int q = 0; q < NC; ++q) { g1[q] = src[(size_t)q * n]; g2[q] = src[(size_t)q * n + step]; }
+                }
+            }
+            if (a.pe) {
+                // extended-array mode (per-block compatibility): zones -2 .. n + 1 of
+                // the caller's primitive array
+                int e = min(p0, n + 1);
+                if (a.outflow_lower && e < 0) e = 0;
+                else if (!a.outflow_lower && a.outflow_upper && e >= n) e = n - 1;
+#pragma unroll
+                for (int q = 0; q < NC; ++q) p[q] = R(a.pe[(size_t)q * (n + 4) + e + 2]);
+            } else {
+                ok = Euler<R>::recover(u, prm, p);
+            }
+            // the nearest guard zone's primitives, and its face state
+            R gp[NC] = {}, gs[NC] = {};
+            if constexpr (CUT) {
+                if (first || last) {
+                    R gq[NC];
+#pragma unroll
+                    for (int q = 0; q < NC; ++q) { g1[q] = away ? g1[q] : u[q]; g2[q] = away ? g2[q] : u[q]; }
+                    bool gok = Euler<R>::recover(g1, prm, gp);
+                    gok &= Euler<R>::recover(g2, prm, gq);
+                    // a guard zone behind the list has no lane of its own to report it
+                    if (away && link >= a.nblk && !gok) report_error(a.err, 1, b, z);
+#pragma unroll
+                    for (int q = 0; q < NC; ++q) {
+                        const R h = plm_half(first ? gq[q] : p[q], gp[q], first ? p[q] : gq[q], theta);
+                        gs[q] = first ? gp[q] + h : gp[q] - h;
+                    }
+                }
+            }
+            // the left face of the lane's zone, from the half slopes of this
+            // zone and the one before
+            R pl[NC], pr[NC], up[NC], f[NC];
+#pragma unroll
+            for (int q = 0; q < NC; ++q) {
+                R below = lane_before(p[q]), above = lane_after(p[q]);
+                if constexpr (CUT) { below = first ? gp[q] : below; above = last ? gp[q] : above; }
+                const R g = plm_half(below, p[q], above, theta);
+                up[q] = p[q] + g;
+                pl[q] = lane_before(up[q]);
+                if constexpr (CUT) pl[q] = first ? gs[q] : pl[q];
+                pr[q] = p[q] - g;
+            }
+            Euler<R>::template riemann<1>(pl, pr, prm, f);
+            R fr[NC];
+            if constexpr (CUT) {
+                if (last) Euler<R>::template riemann<1>(up, gs, prm, fr);
+            }
+#pragma unroll
+            for (int q = 0; q < NC; ++q) {
+                R upper = lane_after(f[q]);
+                if constexpr (CUT) upper = last ? fr[q] : upper;
+                dfx[q] = double(upper) - double(f[q]);
+            }
+        };
+        const unsigned long long cuts = __ballot(cut);
+        if (__builtin_expect(cuts != 0, 0)) {
+            const int above = lane_after(next);               // the next link of a last lane's block
+            fluxes(std::true_type{}, there && cut, there && (cuts >> i) >> 1 & 1, cut ? prev : above);
         } else {
-            ok = Euler<R>::recover(u, prm, p);
+            fluxes(std::false_type{}, false, false, -1);
         }
-        // the left face of the lane's zone, from the half slopes of this zone
-        // and the one before
-#pragma unroll
-        for (int q = 0; q < NC; ++q) {
-            const R g = plm_half(lane_before(p[q]), p[q], lane_after(p[q]), theta);
-            pl[q] = lane_before(p[q] + g);
-            pr[q] = p[q] - g;
-        }
-        Euler<R>::template riemann<1>(pl, pr, prm, f);
+
         double wv[NC];
         const Divisor<double> by_dl(dl);
 #pragma unroll
         for (int q = 0; q < NC; ++q) {
-            const double dfx = double(lane_after(f[q])) - double(f[q]);
-            if constexpr (is_fp64<R>::value) wv[q] = u[q] - by_dl(dfx * dt);
-            else wv[q] = u[q] - dfx * (dt / dl);
+            if constexpr (is_fp64<R>::value) wv[q] = u[q] - by_dl(dfx[q] * dt);
+            else wv[q] = u[q] - dfx[q] * (dt / dl);
             if (a.u0) wv[q] = u0[q] * a.rk_b + wv[q] * (1.0 - a.rk_b);
         }
         if (mine) {
-            double* o = a.out + (size_t)b * NC * n + z;
+            double* o = a.out + at;
 #pragma unroll
             for (int q = 0; q < NC; ++q) o[(size_t)q * n] = wv[q];
             if (!ok) report_error(a.err, 1, b, z);
             if (a.rate_slot) rate = fmax(rate, Euler<double>::max_speed(wv, prm) * (1.0 / dl));
         }
-        lo += count;
     }
     if (a.rate_slot) workgroup_atomic_max<64 * kWindowGroup>(rate, a.rate_slot);
 }

@@ -438,6 +438,49 @@ def test_euler1d_stage_follows_the_links(n, precision):
 
 
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("n", [16, 64, 256])
+def test_euler1d_stage_reads_neighbours_behind_the_list(n, precision):
+    """A list whose outer neighbours are stored behind it, with no rows in the
+    link table, in the base state or in the cell spacings: its blocks equal the
+    same blocks of the whole chain, and a negative density in a guard zone there
+    is reported."""
+    from mara3p_amd._lib import NegativeDensityError, PRECISIONS, check, check_kernel_errors, lib
+    rng = np.random.default_rng(n)
+    m = 7
+    rho, v, p = 1 + rng.random((m, n)), 0.5 * rng.standard_normal((m, n)), 0.5 + rng.random((m, n))
+    u = np.stack([rho, rho * v, 0 * v, 0.1 * rho, 0.5 * rho * (v * v + 0.01) + p / 0.4], axis=1)
+    dl = (1.0 + rng.random(m)) / (m * n)
+    dt = 0.05 * dl.min()
+    dev = lambda x, t: torch.as_tensor(np.ascontiguousarray(x), dtype=t, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def stage(state, base, nbr, spacing):
+        k = len(nbr)
+        us, bs, ns, ds = (dev(state, torch.float64), dev(base, torch.float64), dev(nbr, torch.int32),
+                          dev(spacing, torch.float64))
+        out = torch.empty((k, 5, n), dtype=torch.float64, device="cuda")
+        check(lib().m3p_euler1d_stage_blocks(us.data_ptr(), bs.data_ptr(), out.data_ptr(), ns.data_ptr(),
+                                             ds.data_ptr(), k, n, dt, None, 0.5, 1.5, 1.4, PRECISIONS[precision], stream))
+        check_kernel_errors(stream)
+        return out.cpu().numpy()
+
+    b = np.arange(m)
+    chain = np.stack([b - 1, np.where(b < m - 1, b + 1, -1)], axis=1)
+    whole = stage(u, u, chain, dl)
+    # blocks 1 .. m - 2 of the chain as a list, block 0 and block m - 1 behind it
+    order = np.concatenate([b[1:-1], [0, m - 1]])
+    k = m - 2
+    part = np.stack([b[:k] - 1, b[:k] + 1], axis=1)
+    part[0, 0], part[-1, 1] = k, k + 1
+    assert np.array_equal(stage(u[order], u[1:-1], part, dl[1:-1]), whole[1:-1])
+    for block, zone in ((k, n - 2), (k + 1, 1)):
+        bad = u[order].copy()
+        bad[block, 0, zone] = -1.0
+        with pytest.raises(NegativeDensityError):
+            stage(bad, u[1:-1], part, dl[1:-1])
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
 def test_sod_to_t_0_2(precision):
     """The Sod configuration (1024 zones, gamma 1.4, PLM 1.5, HLLE, RK2, CFL
     0.4 by the signal-speed bound 2.2, outflow ends) integrated to t = 0.2:
