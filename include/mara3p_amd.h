@@ -412,7 +412,8 @@ int m3p_euler2d_rk2_step_cfl(const double* u, double* out, const int* nbr, int n
  * m3p_euler1d_stage_blocks(u1, u -> out) with the same dt (or dt_dev),
  * dl_blk, theta and gamma.  The prev/next links of nbr must be mutual where
  * both blocks exist (chains and rings; otherwise the error latch receives
- * M3P_ERR_BAD_SHAPE); blocks of 16, 32, 64, 128 or a multiple of 256 zones,
+ * M3P_ERR_BAD_SHAPE; a link may name a block behind the list, whose rows nbr
+ * and dl_blk then hold too); blocks of 16, 32, 64, 128 or a multiple of 256 zones,
  * M3P_MIXED only (otherwise M3P_ERR_BAD_ARGUMENT or M3P_ERR_BAD_SHAPE); out
  * must not alias u.  The _cfl form also writes the time step of `out` to
  * dt_next (device double), as m3p_euler1d_stage_blocks_cfl does. */

@@ -21,11 +21,17 @@
 // with the CFL reduction 48.
 //
 // Zones of a window are one chain where every block boundary in it joins
-// blocks that are linked and consecutive in storage (nearly always).  Else the
-// window is done in pieces, each piece's lanes finding their zones along the
-// prev/next links from the piece's first zone: a neighbour stored elsewhere,
-// or, past an outflow end, a copy of the edge zone, whose lanes take the edge
-// zone's U1 in the second stage as the two-stage guard fill does.
+// blocks that are linked both ways and consecutive in storage (nearly always).
+// Else the window is cut there, and each part takes the two stages in turn
+// with its zones in their lanes; the lanes beside it hold its guard zones for
+// the while, found once for the whole window: blocks are at least 16 zones,
+// so a lane stands beside one cut at most.  The guard zones lie across the
+// part's own prev/next link or, past an outflow end, copy the edge zone, whose
+// lanes take the edge zone's U1 in the second stage as the two-stage guard fill
+// does.  The list above in shuffled order (two parts a window) takes 63 us, in
+// order 39.6; blocks of 16 of 512 problems of 64 to 1024 zones 20 and 9.8.  Parts
+// that found their zones along the links one after the other took 71 and 27; a
+// workgroup per block 50 and 25, whatever the order.
 //
 // Every U1 value is the one the two-stage path computes: a zone of another
 // block is updated with that block's cell spacing from the same operands (its
@@ -50,118 +56,137 @@ rk2_fused_1d_kernel(EulerParams prm, Stage1DArgs a)
     const int n = a.n;
     const int i = threadIdx.x & 63;
     const long total = (long)a.nblk * n;
-    const long first = ((long)blockIdx.x * kWindowGroup + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * kWindow1D;
-    const long end = first + kWindow1D < total ? first + kWindow1D : total;
+    const long lo = ((long)blockIdx.x * kWindowGroup + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * kWindow1D;
+    const long end = lo + kWindow1D < total ? lo + kWindow1D : total;
     const R theta = R(prm.theta);
     const double dt = a.dt_dev ? *a.dt_dev : a.dt;
     double rate = 0.0;                      // fused CFL reduction
 
-    for (long lo = first; lo < end;) {
-        // block and zone of lo, then of each lane along the storage order
+    if (lo < end) {
+        // block and zone of lo, then of each lane along the storage order; a
+        // lane before the list or past it holds a zone inside, of no use
         const int b0 = total < (1l << 31) ? (int)((unsigned)lo / (unsigned)n) : (int)(lo / n);
         const int p0 = (int)(lo - (long)b0 * n) + i - 4;      // the lane's zone counted from block b0's first
         int b = b0, z = p0;
         while (z >= n) { ++b; z -= n; }
         if (z < 0) { --b; z += n; }
-        const bool inside = lo >= 4 && lo + 60 <= total;
-        int prev = b - 1, next = b;                           // the links across the boundary before the lane's zone
-        if (inside && i > 0 && z == 0) { prev = a.nbr[2 * b]; next = a.nbr[2 * (b - 1) + 1]; }
-        // the state is fetched before the links are known (the latencies
-        // overlap), and again by the pieces that do not follow the storage
-        double u0[NC];
-        auto fetch = [&] () {
-            const double* src = a.u + (size_t)b * NC * n + z;
+        const bool there = b >= 0 && b < a.nblk;
+        const bool edge = i > 0 && z == 0 && b >= 0 && b <= a.nblk;   // a boundary before the lane's zone
+        int prev = -1, next = -1;                             // the links across it
+        if (edge) {
+            if (there) prev = a.nbr[2 * b];
+            if (b > 0) next = a.nbr[2 * (b - 1) + 1];
+        }
+        const bool cut = edge && !(there && b > 0 && prev == b - 1 && next == b);
+        if (!there) { b = b0; z = min(max(p0, 0), n - 1); }
+        const size_t at = (size_t)b * NC * n + z;
+        const int stop = 4 + (int)(end - lo);                 // lanes 4 .. stop - 1 are the window's own
+        // the state is fetched before the links are known (the latencies overlap)
+        double u0[NC], dl = a.dl;
 #pragma unroll
-            for (int q = 0; q < NC; ++q) u0[q] = src[(size_t)q * n];
-        };
-        double dl = a.dl;
-        if (inside) {
-            fetch();
-            if (a.dl_blk) dl = a.dl_blk[b];
-        }
-        int count = (int)(end - lo);                          // zones this piece updates
-        unsigned long long low = 0, high = 0;                 // lanes past an outflow end
-        if (__builtin_expect(__ballot(inside && prev == b - 1 && next == b) != ~0ull, 0)) {
-            b = b0;
-            z = p0;
-            bool out_lo = false, out_hi = false;
-            if (z < 0) {
-                const int pb = a.nbr[2 * b];
-                const bool mutual = pb < 0 || a.nbr[2 * pb + 1] == b;
-                if (!mutual) report_error(a.err, 4, b, -1);
-                if (pb >= 0 && mutual) { b = pb; z += n; }
-                else { z = 0; out_lo = true; }
-            }
-            while (z >= n) {
-                const int nb = a.nbr[2 * b + 1];
-                const bool mutual = nb < 0 || a.nbr[2 * nb] == b;
-                if (!mutual) report_error(a.err, 4, b, n);
-                if (nb >= 0 && mutual) { b = nb; z -= n; }
-                else { z = n - 1; out_hi = true; }
-            }
-            low = __ballot(out_lo);
-            high = __ballot(out_hi);
-            // the piece ends at the first lane whose zone is not the storage's
-            const unsigned long long other = __ballot(i >= 4 && (out_hi || (long)b * n + z != lo + (i - 4)));
-            if (other) count = min(count, __builtin_ctzll(other) - 4);
-            fetch();
-            if (a.dl_blk) dl = a.dl_blk[b];
-        }
-        const bool mine = i >= 4 && i < 4 + min(count, kWindow1D);
-        const double dtdl = dt / dl;
-        double u1[NC];
-        R p[NC], f[NC];
+        for (int q = 0; q < NC; ++q) u0[q] = a.u[at + (size_t)q * n];
+        if (a.dl_blk) dl = a.dl_blk[b];
 
-        // the left face of the lane's zone, from the half slopes of this zone
-        // and the one before, with the operands and order of stage1d_kernel
-        auto face = [&] () {
-            R pl[NC], pr[NC];
-#pragma unroll
-            for (int q = 0; q < NC; ++q) {
-                const R g = plm_half(lane_before(p[q]), p[q], lane_after(p[q]), theta);
-                pl[q] = lane_before(p[q] + g);
-                pr[q] = p[q] - g;
+        const unsigned long long cuts = __ballot(cut);
+        int gb = b;                                           // the guard zone that the lane holds for a part
+        size_t gat = at;                                      // beside it
+        unsigned long long outflow = 0;
+        if (__builtin_expect(cuts != 0, 0)) {
+            // the cut at or below the lane and the next one above it: within four
+            // lanes of one, the lane is beside the part on its other side
+            const unsigned long long upto = (2ull << i) - 1, below = cuts & upto, above = cuts & ~upto;
+            const int kd = below ? 63 - __builtin_clzll(below) : 0, ku = above ? __builtin_ctzll(above) : 64;
+            const bool starts = __shfl((int)there, ku & 63, 64);
+            const bool up = below && i - kd < 4;              // past the end of the part below
+            const bool dn = above && ku - 1 - i < 4 && starts;
+            const int eb = __shfl(b, up ? kd - 1 : ku & 63, 64);      // that part's block
+            const int from_below = __shfl(next, kd, 64), from_above = __shfl(prev, ku & 63, 64);
+            int link = -1;
+            if (up || dn) {
+                link = up ? from_below : from_above;
+                if (link >= 0 && a.nbr[2 * link + (up ? 0 : 1)] != eb) {
+                    report_error(a.err, 4, eb, up ? n : -1);
+                    link = -1;
+                }
+                gb = link < 0 ? eb : link;
+                const int gz = link < 0 ? (up ? n - 1 : 0) : (up ? i - kd : n - ku + i);
+                gat = (size_t)gb * NC * n + gz;
             }
-            Euler<R>::template riemann<1>(pl, pr, prm, f);
-        };
-        auto flux_difference = [&] (int q) { return double(lane_after(f[q])) - double(f[q]); };
+            outflow = __ballot((up || dn) && link < 0);
+        }
 
-        bool ok = Euler<R>::recover(u0, prm, p);
-        face();
+        // The two stages of the zones in lanes ka .. kb - 1 (one part, all of
+        // them, where nothing is cut), the window's own among them stored.
+        for (int ka = 0; ka < stop;) {
+            const unsigned long long rest = cuts & ~((2ull << ka) - 1);
+            const int kb = rest ? __builtin_ctzll(rest) : 64;
+            const int la = ka;
+            ka = kb;
+            if (kb <= 4) continue;
+            const bool in = i >= la && i < kb;
+            if (cuts) {
+                const double* src = a.u + (in ? at : gat);
 #pragma unroll
-        for (int q = 0; q < NC; ++q) u1[q] = u0[q] - flux_difference(q) * dtdl;
-        ok &= Euler<R>::recover(u1, prm, p);
-        if (low) {          // the lanes below take the edge zone's, the first lane of the chain
-            const int e = 64 - __builtin_clzll(low);
+                for (int q = 0; q < NC; ++q) u0[q] = src[(size_t)q * n];
+                if (a.dl_blk) dl = a.dl_blk[in ? b : gb];
+            }
+            const double dtdl = dt / dl;
+            double u1[NC];
+            R p[NC], f[NC];
+
+            // the left face of the lane's zone, from the half slopes of this zone
+            // and the one before, with the operands and order of stage1d_kernel
+            auto face = [&] () {
+                R pl[NC], pr[NC];
+#pragma unroll
+                for (int q = 0; q < NC; ++q) {
+                    const R g = plm_half(lane_before(p[q]), p[q], lane_after(p[q]), theta);
+                    pl[q] = lane_before(p[q] + g);
+                    pr[q] = p[q] - g;
+                }
+                Euler<R>::template riemann<1>(pl, pr, prm, f);
+            };
+            auto flux_difference = [&] (int q) { return double(lane_after(f[q])) - double(f[q]); };
+
+            const bool ok0 = Euler<R>::recover(u0, prm, p);
+            face();
+#pragma unroll
+            for (int q = 0; q < NC; ++q) u1[q] = u0[q] - flux_difference(q) * dtdl;
+            const bool ok1 = Euler<R>::recover(u1, prm, p);
+            if (cuts) {
+                // a guard zone behind the list has no lane of its own to report it
+                if (!in && gb >= a.nblk && i >= la - 4 && i < kb + 4 && (!ok0 || (!ok1 && i >= la - 2 && i < kb + 2)))
+                    report_error(a.err, 1, b, z);
+                if (la > 0 && outflow >> (la - 1) & 1) {      // the lanes below take the edge zone's, the part's first
+#pragma unroll
+                    for (int q = 0; q < NC; ++q) {
+                        const R v = __shfl(p[q], la, 64);
+                        if (i < la) p[q] = v;
+                    }
+                }
+                if (kb < 64 && outflow >> kb & 1) {           // and those above the last one's
+#pragma unroll
+                    for (int q = 0; q < NC; ++q) {
+                        const R v = __shfl(p[q], kb - 1, 64);
+                        if (i >= kb) p[q] = v;
+                    }
+                }
+            }
+            face();
+            double wv[NC];
 #pragma unroll
             for (int q = 0; q < NC; ++q) {
-                const R v = __shfl(p[q], e, 64);
-                if (i < e) p[q] = v;
+                const double res = u1[q] - flux_difference(q) * dtdl;
+                wv[q] = u0[q] * a.rk_b + res * (1.0 - a.rk_b);
+            }
+            if (in && i >= 4 && i < stop) {
+                double* o = a.out + at;
+#pragma unroll
+                for (int q = 0; q < NC; ++q) o[(size_t)q * n] = wv[q];
+                if (!ok0 || !ok1) report_error(a.err, 1, b, z);
+                if (a.rate_slot) rate = fmax(rate, Euler<double>::max_speed(wv, prm) * (1.0 / dl));
             }
         }
-        if (high) {         // and those above the last lane's
-            const int e = __builtin_ctzll(high) - 1;
-#pragma unroll
-            for (int q = 0; q < NC; ++q) {
-                const R v = __shfl(p[q], e, 64);
-                if (i > e) p[q] = v;
-            }
-        }
-        face();
-        double wv[NC];
-#pragma unroll
-        for (int q = 0; q < NC; ++q) {
-            const double res = u1[q] - flux_difference(q) * dtdl;
-            wv[q] = u0[q] * a.rk_b + res * (1.0 - a.rk_b);
-        }
-        if (mine) {
-            double* o = a.out + (size_t)b * NC * n + z;
-#pragma unroll
-            for (int q = 0; q < NC; ++q) o[(size_t)q * n] = wv[q];
-            if (!ok) report_error(a.err, 1, b, z);
-            if (a.rate_slot) rate = fmax(rate, Euler<double>::max_speed(wv, prm) * (1.0 / dl));
-        }
-        lo += count;
     }
     if (a.rate_slot) workgroup_atomic_max<64 * kWindowGroup>(rate, a.rate_slot);
 }

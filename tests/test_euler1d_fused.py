@@ -192,3 +192,42 @@ def test_fused_rk2_refuses_what_it_does_not_compute():
     with pytest.raises(M3PError) as e:
         one.check_errors()
     assert e.value.code == 4
+
+
+@pytest.mark.parametrize("n", [16, 64, 256])
+def test_fused_rk2_neighbours_behind_the_list(n):
+    """A list whose outer neighbours are stored behind it (with rows of their own
+    in the link table and the cell spacings): its blocks equal the same blocks
+    of the whole chain's fused step, and a negative density in any of the four
+    guard zones there is reported."""
+    from mara3p_amd._lib import M3P_MIXED, NegativeDensityError, check, check_kernel_errors, lib
+    rng = np.random.default_rng(n)
+    m = 7
+    rho, v, p = 1 + rng.random((m, n)), 0.5 * rng.standard_normal((m, n)), 0.5 + rng.random((m, n))
+    u = np.stack([rho, rho * v, 0 * v, 0.1 * rho, 0.5 * rho * (v * v + 0.01) + p / 0.4], axis=1)
+    dl = (1.0 + rng.random(m)) / (m * n)
+    dt = 0.05 * dl.min()
+    dev = lambda x, t: torch.as_tensor(np.ascontiguousarray(x), dtype=t, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def step(state, nbr, spacing, k):
+        us, ns, ds = dev(state, torch.float64), dev(nbr, torch.int32), dev(spacing, torch.float64)
+        out = torch.empty((k, 5, n), dtype=torch.float64, device="cuda")
+        check(lib().m3p_euler1d_rk2_step_blocks(us.data_ptr(), out.data_ptr(), ns.data_ptr(), ds.data_ptr(), k, n,
+                                                dt, None, 0.5, 1.5, 1.4, M3P_MIXED, stream))
+        check_kernel_errors(stream)
+        return out.cpu().numpy()
+
+    b = np.arange(m)
+    chain = np.stack([b - 1, np.where(b < m - 1, b + 1, -1)], axis=1)
+    whole = step(u, chain, dl, m)
+    # blocks 1 .. m - 2 of the chain as a list, block 0 and block m - 1 behind it
+    order = np.concatenate([b[1:-1], [0, m - 1]])
+    at = np.argsort(order)
+    table = np.where(chain[order] >= 0, at[np.maximum(chain[order], 0)], -1)
+    assert np.array_equal(step(u[order], table, dl[order], m - 2), whole[1:-1])
+    for block, zone in ((m - 2, n - 4), (m - 2, n - 1), (m - 1, 0), (m - 1, 3)):
+        bad = u[order].copy()
+        bad[block, 0, zone] = -1.0
+        with pytest.raises(NegativeDensityError):
+            step(bad, table, dl[order], m - 2)
