@@ -327,8 +327,12 @@ int m3p_srhd_riemann_array(const double* pl, const double* pr, double* f, long n
  * in {256x128, 256x64, 256x32, 256x16, 128x64, 128x32, 64x64, 64x32, 64x16,
  * 64x8, 64x4, 64x2, 32x32, 32x16, 32x8, 32x4, 16x16, 16x8}.  Without a choice
  * the library picks by the size of the mesh; a choice holds for the process,
- * per (kind, precision), where it divides the block size. */
+ * per (kind, precision), where it divides the block size.  256x16 (64x16 for
+ * the quad-tree) stands for no choice: m3p_get_stage2d_tile reports it then, and
+ * setting it takes a choice back, so what was read can be written back.
+ * m3p_pin_stage2d_tile takes that shape as a choice like any other. */
 int m3p_set_stage2d_tile(int kind, int precision, int tj, int h);
+int m3p_pin_stage2d_tile(int kind, int precision, int tj, int h);
 int m3p_get_stage2d_tile(int kind, int precision, int* tj /* host */, int* h /* host */);
 /* The tile that a stage over nblk blocks of n x n zones takes now (the choice
  * where it fits, else the library's); M3P_ERR_BAD_SHAPE for a block size that

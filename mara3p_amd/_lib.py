@@ -108,6 +108,7 @@ SIGNATURES = {
     "m3p_euler1d_stage": (_I, [_P, _P, _P, _P, _I, _I, _D, _D, _D, _D, _D, _I, _P]),
     "m3p_euler_cfl_dt": (_I, [_P, _I, _L, _D, _D, _D, _P, _P]),
     "m3p_set_stage2d_tile": (_I, [_I, _I, _I, _I]),
+    "m3p_pin_stage2d_tile": (_I, [_I, _I, _I, _I]),
     "m3p_get_stage2d_tile": (_I, [_I, _I, ctypes.POINTER(_I), ctypes.POINTER(_I)]),
     "m3p_stage2d_tile": (_I, [_I, _I, _I, _I, ctypes.POINTER(_I), ctypes.POINTER(_I)]),
     "m3p_autotune_euler2d": (_I, [_P, _P, _P, _I, _I, _D, _D, _I, _I, ctypes.POINTER(_I), ctypes.POINTER(_I),

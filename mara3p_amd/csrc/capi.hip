@@ -192,9 +192,11 @@ constexpr int tile_index(int tj, int h)
         if (kTileVariants[i].tj == tj && kTileVariants[i].h == h) return i;
     return -1;
 }
-// What m3p_get_stage2d_tile reports while no caller has chosen a shape; g_tile
-// ([kind][precision]) holds a caller's choice, or -1.
-constexpr TileShape kLargeTile[kNumKinds] = { {256, 16}, {256, 16}, {64, 16} };
+// The shape that stands for no choice in m3p_get_stage2d_tile and
+// m3p_set_stage2d_tile, so that a caller who reads the table, sets a shape and
+// writes back what it read has the rule back; g_tile ([kind][precision]) holds a
+// choice, or -1.
+constexpr TileShape kNoChoice[kNumKinds] = { {256, 16}, {256, 16}, {64, 16} };
 std::atomic<int> g_tile[kNumKinds][2] = { { -1, -1 }, { -1, -1 }, { -1, -1 } };
 
 bool tile_fits(TileShape v, int n) { return n % v.tj == 0 && n % v.h == 0 && v.h <= n; }
@@ -1135,19 +1137,25 @@ int m3p_graph_destroy(void* graph_exec)
     return hip_check(hipGraphExecDestroy((hipGraphExec_t)graph_exec), "hipGraphExecDestroy");
 }
 
-int m3p_set_stage2d_tile(int kind, int precision, int tj, int h)
+static int choose_tile(int kind, int precision, int tj, int h, bool may_clear)
 {
     if (kind < 0 || kind >= kNumKinds || precision < 0 || precision > 1) return fail(M3P_ERR_BAD_ARGUMENT, "m3p: bad kind/precision");
-    const int i = tile_index(tj, h);
-    if (i >= 0) { g_tile[kind][precision].store(i, std::memory_order_relaxed); return M3P_OK; }
-    return fail(M3P_ERR_BAD_ARGUMENT, "m3p: tile " + std::to_string(tj) + "x" + std::to_string(h) + " is not a compiled variant");
+    int i = tile_index(tj, h);
+    if (i < 0) return fail(M3P_ERR_BAD_ARGUMENT, "m3p: tile " + std::to_string(tj) + "x" + std::to_string(h) + " is not a compiled variant");
+    if (may_clear && tj == kNoChoice[kind].tj && h == kNoChoice[kind].h) i = -1;
+    g_tile[kind][precision].store(i, std::memory_order_relaxed);
+    return M3P_OK;
 }
+
+int m3p_set_stage2d_tile(int kind, int precision, int tj, int h) { return choose_tile(kind, precision, tj, h, true); }
+
+int m3p_pin_stage2d_tile(int kind, int precision, int tj, int h) { return choose_tile(kind, precision, tj, h, false); }
 
 int m3p_get_stage2d_tile(int kind, int precision, int* tj, int* h)
 {
     if (kind < 0 || kind >= kNumKinds || precision < 0 || precision > 1) return fail(M3P_ERR_BAD_ARGUMENT, "m3p: bad kind/precision");
     const int i = g_tile[kind][precision].load(std::memory_order_relaxed);
-    const TileShape v = i >= 0 ? kTileVariants[i] : kLargeTile[kind];
+    const TileShape v = i >= 0 ? kTileVariants[i] : kNoChoice[kind];
     if (tj) *tj = v.tj;
     if (h) *h = v.h;
     return M3P_OK;

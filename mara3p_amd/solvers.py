@@ -40,7 +40,7 @@ def autotune_tiles(kind, precision, n, run, reps=5):
     for tj, h in TILE_VARIANTS:
         if n % tj or n % h:
             continue
-        check(lib().m3p_set_stage2d_tile(kind, precision, tj, h))
+        check(lib().m3p_pin_stage2d_tile(kind, precision, tj, h))
         run()
         e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
         e0.record()
@@ -51,7 +51,7 @@ def autotune_tiles(kind, precision, n, run, reps=5):
         ms = e0.elapsed_time(e1) / reps
         if best is None or ms < best[2]:
             best = (tj, h, ms)
-    check(lib().m3p_set_stage2d_tile(kind, precision, best[0], best[1]))
+    check(lib().m3p_pin_stage2d_tile(kind, precision, best[0], best[1]))
     return best
 
 

@@ -228,6 +228,52 @@ def test_every_tile_shape_gives_the_same_minidisk_step(precision):
         assert err <= 1e-12, err
 
 
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("scheme", ["euler2d", "minidisk"])
+def test_pinned_tiles_give_the_same_stage(scheme, precision):
+    """The shapes that stand for no choice (256 x 16, 64 x 16), pinned, compute
+    the stages that the library's own tiles compute, and the rule is back after
+    them."""
+    from mara3p_amd import MinidiskData, problems
+    from mara3p_amd._lib import M3P_KIND_EULER2D, M3P_KIND_MINIDISK, PRECISIONS, lib
+    from mara3p_amd.solvers import Euler2DSolver, MinidiskSolver
+    depth, n = 1, 256
+    kind, prec = M3P_KIND_EULER2D if scheme == "euler2d" else M3P_KIND_MINIDISK, PRECISIONS[precision]
+    if scheme == "euler2d":
+        mesh, u0 = problems.kelvin_helmholtz(depth=depth, block_size=n, seed=11)
+        s = Euler2DSolver(depth, n, precision=precision)
+        dt = 0.4 * s.dl / 2.0
+    else:
+        data = MinidiskData.defaults(block_size=n, depth=depth, domain_radius=2.0)
+        mesh, u0 = problems.minidisk(data, seed=13)
+        s = MinidiskSolver(data, precision)
+        dt = problems.minidisk_dt(data, 0.0)
+
+    def in_use():
+        tj, h = ctypes.c_int(0), ctypes.c_int(0)
+        assert lib().m3p_stage2d_tile(kind, prec, n, mesh.nblk, ctypes.byref(tj), ctypes.byref(h)) == 0
+        return tj.value, h.value
+
+    def step():
+        s.set_state(u0)
+        s.time = 0.0
+        s.step(dt)
+        s.check_errors()
+        return s.state()
+
+    rule = in_use()
+    assert rule != (256, 16)
+    first = step()
+    for shape in ((256, 16), (64, 16)):
+        assert lib().m3p_pin_stage2d_tile(kind, prec, *shape) == 0
+        try:
+            assert in_use() == shape
+            assert np.array_equal(step(), first)
+        finally:
+            assert lib().m3p_set_stage2d_tile(kind, prec, 256, 16) == 0
+    assert in_use() == rule
+
+
 @pytest.mark.parametrize("lo, hi", [(-8, 8), (-900, 400), (-1032, -960)])
 def test_quotients_by_one_denominator(lo, hi):
     """The FP64 recovery takes the reciprocal of the density once: its four

@@ -33,3 +33,43 @@ def test_every_block_size_has_a_tile_that_divides_it(n, nblk):
         for precision in (M3P_FP64, M3P_MIXED):
             st, tj, h = tile_of(kind, precision, n, nblk)
             assert st == 0 and n % tj == 0 and n % h == 0, (kind, precision, tj, h)
+
+
+SIZES = ((16, 64), (32, 64), (64, 16), (64, 1024), (64, 4096), (128, 256), (256, 4), (256, 64), (256, 256), (4096, 1))
+
+
+@pytest.fixture
+def no_choice():
+    """Leave every (kind, precision) without a choice afterwards."""
+    yield
+    for kind in KINDS:
+        for precision in (M3P_FP64, M3P_MIXED):
+            lib().m3p_set_stage2d_tile(kind, precision, *((64, 16) if kind == M3P_KIND_AMR_EULER2D else (256, 16)))
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("precision", [M3P_FP64, M3P_MIXED])
+def test_a_tile_choice_can_be_put_back(kind, precision, no_choice):
+    """Read, set another shape, write back what was read: the library's own rule
+    again, at every size; a pinned shape holds, whichever it is."""
+    def rule():
+        return [tile_of(kind, precision, n, nblk) for n, nblk in SIZES]
+
+    def read():
+        tj, h = ctypes.c_int(0), ctypes.c_int(0)
+        assert lib().m3p_get_stage2d_tile(kind, precision, ctypes.byref(tj), ctypes.byref(h)) == 0
+        return tj.value, h.value
+
+    before, saved = rule(), read()
+    for shape in ((64, 64), (32, 32), (16, 16), (64, 2)):
+        assert lib().m3p_set_stage2d_tile(kind, precision, *shape) == 0
+        assert read() == shape
+        assert tile_of(kind, precision, 64, 1024) == (0,) + shape
+        assert lib().m3p_set_stage2d_tile(kind, precision, *saved) == 0
+        assert rule() == before and read() == saved
+    # the shape that stands for no choice, as a choice
+    assert lib().m3p_pin_stage2d_tile(kind, precision, *saved) == 0
+    assert all(tile_of(kind, precision, 256, nblk) == (0,) + saved for nblk in (1, 16, 256))
+    assert lib().m3p_set_stage2d_tile(kind, precision, *saved) == 0
+    assert rule() == before
+    assert lib().m3p_pin_stage2d_tile(kind, precision, 48, 16) == M3P_ERR_BAD_ARGUMENT
