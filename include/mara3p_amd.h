@@ -56,7 +56,15 @@ extern "C" {
  * exp, reciprocal forms of its sources and Newton-refined hardware
  * reciprocals and square roots differ from glibc and from the reference's
  * divisions by a few ulp; MHD: the same forms in the wave speeds, the HLLE
- * flux and the primitive recovery).  M3P_MIXED computes primitives, slopes
+ * flux and the primitive recovery).  The stages' bit-for-bit quotients and
+ * roots hold while densities, wave-speed widths and cell spacings are normal
+ * numbers below 2^958, nonzero numerators lie between 2^-1033 and 2^958,
+ * quotients neither overflow nor come out subnormal and squared sound speeds
+ * are zero or at least 2^-960; past that a quotient that overflows is NaN, not
+ * infinite, and one by a subnormal is not to be relied on.  Of a state that is
+ * not finite the fluxes leave out the products with the zero components of the
+ * face normal.  The array functions divide as IEEE for every operand.
+ * M3P_MIXED computes primitives, slopes
  * and fluxes in FP32 and keeps the conserved state and flux differences in
  * FP64. */
 #define M3P_FP64   0

@@ -88,9 +88,10 @@ template<typename R> __device__ __forceinline__ R fsqrt(R a)
 // hardware estimates (v_rcp_f64, v_rsq_f64) refined by two Newton steps each
 // (quadratic convergence from the estimate's ~2^-22 to the last bit or two):
 // a few ulp instead of IEEE rounding, at a third of the instructions of the
-// IEEE division and square root sequences.  For the FP64 kernels whose bar
-// against the reference is 1e-12 relative (minidisk, MHD), never for the
-// ones that equal it bit for bit.
+// IEEE division and square root sequences.  As they are, for the FP64 kernels
+// whose bar against the reference is 1e-12 relative (minidisk, MHD); the kernels
+// that equal it bit for bit take quotients and roots that correct the estimate
+// by a remainder (Divisor, sqrt_ieee).
 __device__ __forceinline__ double rcp_nr(double b)
 {
     double r = __builtin_amdgcn_rcp(b);
@@ -147,12 +148,31 @@ template<> struct Divisor<double> {
     }
 };
 
-// The IEEE square root by the compiler's own steps (reciprocal square root
-// estimate and three corrections) without the scaling it puts around them for
-// arguments below 2^-767: a scaling by a power of four changes no rounding
-// while the remainders stay normal, so the root is the same bit for bit for
-// x >= 2^-960; +-0, +inf, NaN and negative x as IEEE.  Five instructions less
-// on the chain from the sound speed to the flux.
+// The same for every operand: IEEE's a / b outside the range above (operands of
+// extreme size, quotients that overflow or come out subnormal).  For functions
+// of arrays that hold anything; a stage kernel's recovery with it would pay a
+// test and a branch per quotient.
+struct WideDivisor {
+    Divisor<double> by;
+    bool usual;
+    __device__ __forceinline__ explicit WideDivisor(double d) : by(d), usual(fabs(d) >= 0x1p-1022 && fabs(d) < 0x1p958) {}
+    __device__ __forceinline__ double operator()(double a) const
+    {
+        const double q = by(a), m = fabs(a);
+        const bool in = usual && m < 0x1p958 && (a == 0.0 || (m >= 0x1p-1033 && fabs(q) >= 0x1p-1022 && fabs(q) < __builtin_inf()));
+        return in ? q : a / by.b;
+    }
+};
+
+// The IEEE square root: the coupled iteration for g -> sqrt(x) and
+// h -> 1 / (2 sqrt(x)) from one estimate of the reciprocal root, closed by two
+// corrections of g by its remainder x - g g, the last of which rounds correctly
+// (Markstein, IBM J. Res. Dev. 34, 1990).  Nothing is scaled, so the remainders
+// must be normal numbers: the root is IEEE's bit for bit for x >= 2^-960; +-0,
+// +inf, NaN and negative x as IEEE.  sqrt() scales every argument for the sake
+// of those below 2^-767, five instructions on the chain from the sound speed
+// to the flux (FP64 Kelvin-Helmholtz 4096^2, with the shared reciprocals: 1.16
+// to 1.09 ms a step).
 __device__ __forceinline__ double sqrt_ieee(double x)
 {
     const double y = __builtin_amdgcn_rsq(x);

@@ -17,7 +17,7 @@ euler_recover_array_kernel(const double* u, double* p, long nz, double gamma, in
     double uu[5], pp[5];
     for (int q = 0; q < 5; ++q) uu[q] = u[q * nz + z];
     EulerParams prm{ gamma, 0.0, 0 };
-    bool ok = Euler<double>::recover(uu, prm, pp);
+    bool ok = Euler<double>::recover<WideDivisor>(uu, prm, pp);
     for (int q = 0; q < 5; ++q) p[q * nz + z] = pp[q];
     if (!ok) report_error(err, 1, 0, (int)z);
 }
@@ -28,7 +28,7 @@ iso2d_recover_array_kernel(const double* u, double* p, long nz)
     long z = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (z >= nz) return;
     double uu[3] = { u[z], u[nz + z], u[2 * nz + z] }, pp[3];
-    Iso2d<double>::recover(uu, pp);
+    Iso2d<double>::recover<WideDivisor>(uu, pp);
     for (int q = 0; q < 3; ++q) p[q * nz + z] = pp[q];
 }
 

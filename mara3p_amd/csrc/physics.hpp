@@ -26,12 +26,14 @@ struct Euler {
     using Params = EulerParams;
 
     // recover_primitive, src/physics_euler.hpp:156-169.  Returns false on D < 0.
+    // Div: Divisor, or WideDivisor for operands of any size (FP64).
+    template<class Div = Divisor<double>>
     __device__ static __forceinline__ bool recover(const double* u, const Params& prm, R* p)
     {
         if constexpr (is_fp64<R>::value) {
             double D = u[0], S1 = u[1], S2 = u[2], S3 = u[3], E = u[4];
             double ls = (S1 * S1 + S2 * S2) + S3 * S3;
-            const Divisor<double> by_D(D);
+            const Div by_D(D);
             double ke = by_D(0.5 * ls);
             p[0] = D;
             p[1] = by_D(S1);
@@ -220,10 +222,11 @@ struct Iso2d {
     static constexpr int NC = 3;
 
     // recover_primitive :119-125 (no negative-density check in the reference)
+    template<class Div = Divisor<double>>
     __device__ static __forceinline__ void recover(const double* u, R* p)
     {
         if constexpr (is_fp64<R>::value) {
-            const Divisor<double> by_sigma(u[0]);
+            const Div by_sigma(u[0]);
             p[0] = u[0];
             p[1] = by_sigma(u[1]);
             p[2] = by_sigma(u[2]);

@@ -308,6 +308,64 @@ def test_quotients_by_one_denominator(lo, hi):
         assert np.array_equal(a[usual], b[usual], equal_nan=True)
 
 
+def test_array_recoveries_divide_as_ieee_everywhere():
+    """The recoveries of arrays equal IEEE division bit for bit for every
+    operand: exponents over the whole range, subnormal densities and momenta,
+    quotients that overflow or come out subnormal, zeros, infinities, NaN."""
+    from mara3p_amd import check, lib
+    rng = np.random.default_rng(23)
+    n = 200000
+
+    def values():
+        x = np.ldexp(1.0 + rng.random(n), rng.integers(-1074, 1024, n)) * rng.choice([-1.0, 1.0], n)
+        x[:n // 4] = np.ldexp(1.0 + rng.random(n // 4), rng.integers(-60, 60, n // 4))
+        for k, v in enumerate((0.0, -0.0, np.inf, -np.inf, np.nan, 5e-324, -2.0 ** -1022, 1.7976931348623157e308)):
+            x[rng.integers(0, n, 1500)] = v
+        return x
+    D = np.abs(values())                  # a negative density is an error
+    S = [values() for _ in range(3)]
+    E = values()
+    u = torch.as_tensor(np.stack([D, *S, E]), device="cuda")
+    p = torch.empty_like(u)
+    check(lib().m3p_euler_recover_primitive_array(u.data_ptr(), p.data_ptr(), n, 5.0 / 3.0, None))
+    with np.errstate(all="ignore"):
+        ke = 0.5 * ((S[0] * S[0] + S[1] * S[1]) + S[2] * S[2]) / D
+        ref = np.stack([D, S[0] / D, S[1] / D, S[2] / D, (E - ke) * (5.0 / 3.0 - 1.0)])
+    assert np.array_equal(p.cpu().numpy(), ref, equal_nan=True)
+    q = torch.empty((3, n), dtype=torch.float64, device="cuda")
+    check(lib().m3p_iso2d_recover_primitive_array(u.data_ptr(), q.data_ptr(), n, None))
+    assert np.array_equal(q.cpu().numpy(), ref[:3], equal_nan=True)
+
+
+@pytest.mark.parametrize("kp, kd", [(0, 0), (400, 0), (-300, 0), (-300, 300), (-500, 400), (-530, 427), (200, -400),
+                                    (None, 0), ("negative", 0)])
+def test_sound_speed_roots_over_their_range(kp, kd):
+    """FP64 fluxes equal the oracle's bit for bit where the squared sound speed
+    lies anywhere between 2^-957 and 2^600, is zero or is negative (no root):
+    pressures near 2^kp, densities near 2^kd, gas at rest (the flux is then the
+    speeds' own rounding), and moving where there is no pressure."""
+    m3p = _m3p()
+    n = 256
+    for seed in range(8):
+        rng = np.random.default_rng(100 * seed + 7)
+        pe = np.zeros((n + 4, 5))
+        pe[:, 0] = np.ldexp(1.0 + rng.random(n + 4), kd)
+        pe[:, 4] = 0.0 if kp is None else -1.0 - rng.random(n + 4) if kp == "negative" else np.ldexp(1.0 + rng.random(n + 4), kp)
+        if kp is None:
+            pe[:, 1] = 1.0 + rng.random(n + 4)
+        uc, pe = np.zeros((n, 5)), c(pe)
+        ref = np.zeros_like(uc)
+        orc().orc_euler1d_updated_conserved(P(uc), P(pe), n, 1.0, 1.0, 1.5, 1.4, 0, 0, P(ref))
+        out = torch.empty((5, n), dtype=torch.float64, device="cuda")
+        d_uc, d_pe = dev(uc.T), dev(pe.T)
+        m3p.check(m3p.lib().m3p_euler1d_updated_conserved(ptr(d_uc), ptr(d_pe), ptr(out), n, 1.0, 1.0, 1.5, 1.4, 0, 0,
+                                                          m3p.M3P_FP64, stream()))
+        got = out.cpu().numpy().T
+        assert np.array_equal(got, ref, equal_nan=True)
+        if kp != "negative":
+            assert np.all(np.isfinite(ref)) and np.any(ref != 0.0)
+
+
 @pytest.mark.parametrize("n, depth", [(16, 0), (16, 5), (32, 1), (32, 5), (48, 1), (64, 0), (64, 3), (64, 4), (64, 5),
                                       (96, 2), (128, 4), (192, 1), (192, 3), (256, 3)])
 def test_tile_of_each_mesh_size(n, depth):
