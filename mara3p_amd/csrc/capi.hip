@@ -217,11 +217,18 @@ bool tile_fits(TileShape v, int n) { return n % v.tj == 0 && n % v.h == 0 && v.h
 // against 1030 with eight rows and 1059 with 256 x 16 tiles, HLLE 968, 1020 and
 // 1034, minidisk 674, 708 and 720; 2048^2 in 64^2 blocks: HLLC 272 with sixteen,
 // 264 with eight), the quad-tree's leaves and mixed precision staying at eight
-// (tree of 1408 leaves: mixed 214 us, 236 with sixteen; FP64 362 and 376; mixed
-// HLLC, 4096^2: 677 us, 692 with sixteen, 685 with 256 x 16 tiles), but for the
-// mixed minidisk, whose wide tiles read fewer halos (4096^2: 399 us, 405 with 64
-// x 8).  Blocks of 32^2 take sixteen rows from 4096 waves on in FP64 (2048^2:
-// HLLC 304 us, 314 with eight).
+// (tree of 1408 leaves: mixed 214 us, 236 with sixteen; FP64 362 and 376), but
+// where wide tiles read fewer halos of rows that lie far apart in memory: mixed
+// Euler in blocks that 256 divides from 8192 waves of sixteen rows on (4096^2,
+// HLLC with 256 x 16 and 64 x 8 tiles: one block 650 us and 686, 512^2 blocks 646
+// and 677, 256^2 blocks 669 and 672; 2048^2: one block 181 and 181, 256^2 blocks
+// 183 and 175), and the mixed minidisk there at every size with sixteen rows
+// (4096^2: 392 us, 405 with 64 x 8).  In blocks that only 128 divides it is 128 x 32
+// tiles, in mixed precision, where those give every CU four workgroups or close
+// to it (2048^2: minidisk 102 us, 110 with 64 x 8, HLLC 170 and 175); one and a
+// half times as many leave some CUs a workgroup more than others (2560^2: HLLC
+// 325 us, 271 with 64 x 8).  Blocks of 32^2 take sixteen rows from 4096 waves on in FP64 (2048^2: HLLC 304
+// us, 314 with eight).
 TileShape pick_tile(int kind, int precision, int n, int nblk)
 {
     if (n < 16) return {0, 0};             // also zero and below, which every width divides
@@ -230,9 +237,13 @@ TileShape pick_tile(int kind, int precision, int n, int nblk)
     const double zones = (double)nblk * n * n;
     auto waves = [&] (int rows) { return zones / (64.0 * rows); };
     int rows = waves(16) >= 4096 ? 16 : waves(8) >= 2048 ? 8 : waves(4) >= 2048 ? 4 : 2;
-    if (rows == 16 && kind == M3P_KIND_MINIDISK && precision == M3P_MIXED && n % 256 == 0) return {256, 16};
+    const bool large = waves(16) >= 8192;
+    if (rows == 16 && precision == M3P_MIXED && kind != M3P_KIND_AMR_EULER2D) {
+        if (n % 256 == 0 && (large || kind == M3P_KIND_MINIDISK)) return {256, 16};
+        if (n % 256 != 0 && n % 128 == 0 && zones > 960.0 * 128 * 32 && zones <= 1024.0 * 128 * 32) return {128, 32};
+    }
     if (n % 64 == 0) {
-        const bool long_strips = precision == M3P_FP64 && kind != M3P_KIND_AMR_EULER2D && waves(16) >= 8192;
+        const bool long_strips = precision == M3P_FP64 && kind != M3P_KIND_AMR_EULER2D && large;
         return {64, rows == 16 && !long_strips ? 8 : rows};
     }
     if (rows == 16 && (precision == M3P_MIXED || kind == M3P_KIND_AMR_EULER2D)) rows = 8;

@@ -73,3 +73,29 @@ def test_a_tile_choice_can_be_put_back(kind, precision, no_choice):
     assert lib().m3p_set_stage2d_tile(kind, precision, *saved) == 0
     assert rule() == before
     assert lib().m3p_pin_stage2d_tile(kind, precision, 48, 16) == M3P_ERR_BAD_ARGUMENT
+
+
+E, D, T = M3P_KIND_EULER2D, M3P_KIND_MINIDISK, M3P_KIND_AMR_EULER2D
+
+
+@pytest.mark.parametrize("kind, precision, n, nblk, tile", [
+    # strips of two, four and eight rows by the number of waves
+    (E, M3P_FP64, 64, 127, (64, 2)), (E, M3P_FP64, 64, 128, (64, 4)), (E, M3P_FP64, 64, 255, (64, 4)),
+    (E, M3P_FP64, 64, 256, (64, 8)), (E, M3P_MIXED, 64, 256, (64, 8)), (T, M3P_FP64, 64, 1408, (64, 8)),
+    # sixteen rows in FP64 on meshes that fill the device
+    (E, M3P_FP64, 64, 2047, (64, 8)), (E, M3P_FP64, 64, 2048, (64, 16)), (D, M3P_FP64, 256, 256, (64, 16)),
+    (D, M3P_FP64, 4096, 1, (64, 16)), (T, M3P_FP64, 64, 4096, (64, 8)),
+    # wide tiles in mixed precision
+    (E, M3P_MIXED, 256, 127, (64, 8)), (E, M3P_MIXED, 256, 128, (256, 16)), (E, M3P_MIXED, 4096, 1, (256, 16)),
+    (E, M3P_MIXED, 2048, 1, (64, 8)), (D, M3P_MIXED, 256, 63, (64, 8)), (D, M3P_MIXED, 256, 64, (256, 16)),
+    (T, M3P_MIXED, 256, 256, (64, 8)), (E, M3P_FP64, 256, 64, (64, 8)),
+    # blocks that only 128 divides, where 128 x 32 loads every CU alike
+    (E, M3P_MIXED, 128, 255, (64, 8)), (E, M3P_MIXED, 128, 256, (128, 32)), (D, M3P_MIXED, 128, 256, (128, 32)),
+    (D, M3P_MIXED, 128, 257, (64, 8)), (D, M3P_MIXED, 640, 16, (64, 8)), (D, M3P_MIXED, 128, 1024, (64, 8)),
+    (T, M3P_MIXED, 128, 256, (64, 8)), (D, M3P_FP64, 128, 256, (64, 8)),
+    # narrow blocks
+    (E, M3P_FP64, 32, 64, (32, 4)), (E, M3P_FP64, 32, 4096, (32, 32)), (E, M3P_MIXED, 32, 4096, (32, 16)),
+    (E, M3P_FP64, 16, 64, (16, 8)), (E, M3P_FP64, 48, 4096, (16, 16))])
+def test_the_rule_by_size(kind, precision, n, nblk, tile):
+    """The library's own choice on both sides of each line of the rule."""
+    assert tile_of(kind, precision, n, nblk) == (0,) + tile
