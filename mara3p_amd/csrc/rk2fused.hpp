@@ -96,9 +96,11 @@ rk2_fused_kernel(typename S::Params p1, typename S::Params p2, MeshLoader<S> ld,
     // read again three rows later it had partly left the L2, and the launch
     // fetched 1.05 GB for the 0.40 GB of U0 (minidisk, 4096^2: 314 to 303 us
     // with the queue).  Its LDS must not cost a workgroup per CU: the y fluxes
-    // then pass between lanes by a wave shift instead of an LDS row.  Euler's
-    // five components fit too, but the step takes 217 registers and is 4 %
-    // slower (4096^2: 552 us against 530).
+    // then pass between lanes by a wave shift instead of an LDS row.  Narrower
+    // blocks do better without (minidisk in 128^2 blocks, 2048^2 and 4096^2: 97
+    // and 360 us, 103 and 418 with it; in 64^2 blocks 116 and 419, 130 and 439).
+    // Euler's five components fit too, but the step takes 217 registers and is
+    // 4 % slower (4096^2: 552 us against 530).
     constexpr bool kQueue = S::kFusedQueue && TJ == 256 && H == 32;
     __shared__ double u1q[3][NC][TJ];
     __shared__ double u0q[kQueue ? 3 : 1][NC][kQueue ? TJ : 1];

@@ -14,9 +14,9 @@ namespace m3p {
 // fill it want the fewest extra rows (four of the first stage per workgroup):
 // 32 (4096^2 in 256^2 blocks: minidisk 323 us, 346 with 16; 64 rows need
 // about 55 KB of LDS and run 14 % slower), but 16 in blocks of 64, whose
-// one-wave workgroups then share the work more evenly (2048^2: euler2d 192 us
-// against 303 with 32, minidisk 123 against 121; 4096^2: 732 against 800, 423
-// against 444).
+// one-wave workgroups then share the work more evenly (2048^2: euler2d 190 us
+// against 302 with 32, minidisk 116 with either; 4096^2: 738 against 799, 419
+// against 448).
 template<class S>
 int launch_rk2_fused(const typename S::Params& p1, const typename S::Params& p2, const MeshLoader<S>& ld,
                      const StageArgs& a, hipStream_t s)

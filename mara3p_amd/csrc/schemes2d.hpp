@@ -424,7 +424,6 @@ struct IsoTableScheme {
     }
     template<int H, int TJ>
     __device__ static __forceinline__ void setup(TileData<H, TJ>&, const Params&, const TileCtx&) {}
-    __device__ static __forceinline__ void setup_zone(TileData<1, 1>&, const Params&, const TileCtx&) {}
 
     template<int AXIS, int H, int TJ>
     __device__ static __forceinline__ void face(const R* pl, const R* pr, const Params& prm,

@@ -365,13 +365,13 @@ stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
 
     __shared__ typename S::template TileData<H, TJ> td;
     __shared__ R hraw[7][NC][H];     // pre-pass primitives at 7 edge columns
-    __shared__ R hG[NC][H];          // y half slope at column c0-1
-    __shared__ R hF[NC][H];          // y flux at face c0+TJ
     // one wave (kShift): what the edge lanes of a row take from beyond the
     // tile, the primitives at column c0-1, their sum with the half slope
     // there, the primitives at column c0+TJ and the flux at face c0+TJ
     __shared__ alignas(16) R edge[kShift ? H : 1][kShift ? 4 : 1][NC];
-    // several waves: rows of LDS
+    // several waves: the y half slope at column c0-1, the y flux at face c0+TJ
+    // and rows of LDS
+    __shared__ R hG[NC][kShift ? 1 : H], hF[NC][kShift ? 1 : H];
     __shared__ R rowP[NC][kShift ? 1 : TJ + 2];   // [t+1] = column c0+t; [0], [TJ+1] from hraw
     __shared__ R rowG[NC][kShift ? 1 : TJ + 1];   // [t+1] = half slope at column c0+t; [0] from hG
     __shared__ R rowF[NC][kShift ? 1 : TJ + 1];   // [t] = y flux at face c0+t; [TJ] from hF
@@ -391,10 +391,10 @@ stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
     __syncthreads();
     const R theta = R(S::theta(prm));
     for (int r = lane; r < H; r += NT) {
-        R pl[NC], pr[NC], f[NC];
+        R g0[NC], pl[NC], pr[NC], f[NC];
 #pragma unroll
         for (int m = 0; m < NC; ++m) {
-            hG[m][r] = plm_half(hraw[0][m][r], hraw[1][m][r], hraw[2][m][r], theta);
+            g0[m] = plm_half(hraw[0][m][r], hraw[1][m][r], hraw[2][m][r], theta);
             R g1 = plm_half(hraw[3][m][r], hraw[4][m][r], hraw[5][m][r], theta);
             R g2 = plm_half(hraw[4][m][r], hraw[5][m][r], hraw[6][m][r], theta);
             pl[m] = hraw[4][m][r] + g1;
@@ -403,12 +403,14 @@ stage2d_kernel(typename S::Params prm, Ld ld_arg, StageArgs a)
         S::template face<2>(pl, pr, prm, td, tc, tc.k0 + r, tc.c0 + TJ, f);
 #pragma unroll
         for (int m = 0; m < NC; ++m) {
-            hF[m][r] = f[m];
             if constexpr (kShift) {
                 edge[r][0][m] = hraw[1][m][r];
-                edge[r][1][m] = hraw[1][m][r] + hG[m][r];
+                edge[r][1][m] = hraw[1][m][r] + g0[m];
                 edge[r][2][m] = hraw[5][m][r];
                 edge[r][3][m] = f[m];
+            } else {
+                hG[m][r] = g0[m];
+                hF[m][r] = f[m];
             }
         }
         if (Ld::kEdgeFluxes && a.flux_reg && tc.c0 + TJ == n) store_edge_flux<NC>(a.flux_reg, b, 3, n, tc.k0 + r, f);

@@ -64,7 +64,8 @@ struct ViscousTerms {
 // with all its operands in registers recovered 13 zones, took ten slopes and
 // computed every face twice, at two waves per SIMD: FP64 151 us a step at
 // 1024^2 (83 by tiles), mixed 94 (61), FP64 512^2 43 (28).  Tiles that reach
-// past the block clamp their loads and store nothing there.
+// past the block clamp their loads and store nothing there.  The isothermal
+// recoveries report no error (as the reference's), so nothing here does.
 constexpr int kViscTile = 16;
 
 template<class S, class Ld, int T>
@@ -105,12 +106,11 @@ iso_visc_stage_kernel(typename S::Params prm, Ld ld_arg, StageArgs a, double nu)
     const Divisor<double> by_dl(dl);
     const R idl = R(1.0 / dl);
     const R theta = R(S::theta(prm));
-    bool ok = true;
 
     for (int i = t; i < EP * EP; i += T * T) {
         const int r = i / EP, q = i % EP;
         R p[NC];
-        ok &= ld.prim(b, min(tc.k0 + r - 2, n + 1), min(tc.c0 + q - 2, n + 1), prm, p);
+        (void)ld.prim(b, min(tc.k0 + r - 2, n + 1), min(tc.c0 + q - 2, n + 1), prm, p);
 #pragma unroll
         for (int m = 0; m < NC; ++m) P[m][r][q] = p[m];
     }
@@ -185,7 +185,6 @@ iso_visc_stage_kernel(typename S::Params prm, Ld ld_arg, StageArgs a, double nu)
         for (int m = 0; m < NC; ++m)
             o[(size_t)m * n * n] = a.u0 ? u0[m] * a.rk_b + res[m] * (1.0 - a.rk_b) : res[m];
     }
-    if (!ok) report_error(a.err, 1, b, min(k, n - 1) * n + min(c, n - 1));
 }
 
 } // namespace m3p
