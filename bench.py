@@ -171,16 +171,15 @@ def minidisk_mass_drift(steps, fused=False):
     return out
 
 
-def tile_in_use(workload, precision, autotuned):
-    """The stage kernel's tile shape (columns, rows) that --autotune chose;
-    without it the library picks one by the size of the mesh."""
-    from mara3p_amd._lib import lib, PRECISIONS
+def tile_in_use(s, workload):
+    """The stage kernel's tile shape (columns, rows) on the solver's mesh: what
+    --autotune chose, or the library's choice by the size of the mesh."""
+    from mara3p_amd._lib import check, lib
     if workload not in TILE_KIND:
         return None
-    if not autotuned:
-        return "by mesh size"
+    n, nblk = s.u.shape[-1], s.u.shape[0]
     tj, h = ctypes.c_int(0), ctypes.c_int(0)
-    lib().m3p_get_stage2d_tile(TILE_KIND[workload], PRECISIONS[precision], ctypes.byref(tj), ctypes.byref(h))
+    check(lib().m3p_stage2d_tile(TILE_KIND[workload], s.precision, n, nblk, ctypes.byref(tj), ctypes.byref(h)))
     return [tj.value, h.value]
 
 
@@ -532,7 +531,7 @@ def main():
     s, u0, dt_of, nc = make_solver(args.workload, "mixed")
     zones = s.zones
     wall, d1, d2 = timed_run(s, dt_of, args.steps, args.warmup, args.autotune, args.settle_seconds)
-    tile = tile_in_use(args.workload, "mixed", args.autotune)
+    tile = tile_in_use(s, args.workload)
     graph = None
     if not args.no_graph:
         if args.workload in ("kh", "sedov_amr", "ensemble"):
@@ -552,7 +551,7 @@ def main():
         # the headline: one fused launch per RK2 step, the two stage launches
         # (equal value for value) reported beside it
         two_stage = {"value": value, "ms_per_step": ms_per_step, "stage_ms": {"stage1": d1, "stage2": d2},
-                     "tile": tile_in_use(args.workload, "mixed", args.autotune),
+                     "tile": tile,
                      "roofline": {"achieved": achieved, "frac": achieved / HBM_PEAK_GBS, "traffic": traffic}}
         fw, fms = fused_run(s, dt_of, args.steps, args.warmup, args.settle_seconds)
         value = zones * args.steps / fw
@@ -615,7 +614,7 @@ def main():
         s64, _, _, _ = make_solver(args.workload, "fp64")
         k64 = max(10, args.steps // 4)
         wall64, e1, e2 = timed_run(s64, dt_of, k64, max(2, args.warmup // 4), args.autotune, args.settle_seconds)
-        tile64 = tile_in_use(args.workload, "fp64", args.autotune)
+        tile64 = tile_in_use(s64, args.workload)
         v64 = zones * k64 / wall64
         result["fp64"] = {"value": v64, "ms_per_step": 1e3 * wall64 / k64, "stage_ms": {"stage1": e1, "stage2": e2},
                           "tile": tile64,

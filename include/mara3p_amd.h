@@ -26,7 +26,7 @@
  * stream's state is created by its first call, which must come before any
  * graph capture on it (m3p_graph_begin makes it).  Graph replays report
  * kernel errors to the latch of the stream they were captured on.  The tile
- * table (m3p_set_stage2d_tile, m3p_autotune_*) is read and written
+ * table (m3p_set_stage2d_tile, m3p_pin_stage2d_tile, m3p_autotune_*) is read and written
  * atomically.
  */
 #ifndef MARA3P_AMD_H
@@ -99,7 +99,7 @@ typedef struct {
     int    depth;
     double omega_frame;
     double mach_number;
-    double kinematic_viscosity;   /* viscous stress when != 0 (per-zone kernel) */
+    double kinematic_viscosity;   /* viscous stress when != 0 (a kernel of its own) */
     double domain_radius;
     double softening_length;
     double eccentricity;

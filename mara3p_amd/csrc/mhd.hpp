@@ -399,9 +399,10 @@ constexpr int kMhdTileHalo = 448, kMhdTileF2 = 296, kMhdTileF3 = 272;   // LDS o
 // 250 cells, where 8 x 32 takes 52 that reach past the cube).  It is taken where
 // that is at most 5/6 of the tiles, for cubes that the cache holds, whose pass
 // is bound by its arithmetic, and that give the device more than a few
-// workgroups: RK2 step of 100^3 mixed 192 to 173 us, FP64 322 to 283; 80^3 106
-// to 98 and 180 to 162; 65^3 78 to 75 and 129 to 118; 45^3 53 to 51 and 74 to 62.
-// With every ragged cube so, 110^3 mixed 234 to 239, 25^3 FP64 49 to 51, and,
+// workgroups: two stages on one state, 100^3 mixed 182 to 165 us, FP64 317 to
+// 278; 80^3 104 to 96 and 180 to 162; 65^3 77 to 72 and 129 to 118; 45^3 52 to 51
+// and 75 to 63 (a step of a run, whose states alternate, of 100^3 mixed 195 to
+// 183).  With every ragged cube so, 110^3 mixed 234 to 239, 25^3 FP64 49 to 51, and,
 // bound by memory, where rows of partial cache lines cost more, 250^3 mixed
 // 2684 to 3265.
 struct MhdTile { int tj, tk; };

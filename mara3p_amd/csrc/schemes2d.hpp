@@ -24,10 +24,10 @@ template<typename R>
 struct EulerScheme {
     static constexpr int NC = 5;
     // The march's schedule, by the rows of a strip.  FP64 strips of eight rows
-    // or more run at three waves per SIMD (166 VGPRs, no spills), which takes
-    // the RK base at the update, one row of loads ahead and one row per
-    // iteration: 4096^2 Kelvin-Helmholtz 1.08 to 1.01 ms a step, 1408 leaves
-    // of 64^2 434 to 400 us.  Shorter strips, on meshes that do not fill the
+    // or more run at three waves per SIMD (168 VGPRs; the one-wave second stage
+    // spills two, the quad-tree's stages 18 and 22), which takes the RK base at
+    // the update, one row of loads ahead and one row per iteration: 4096^2
+    // Kelvin-Helmholtz 1.08 to 1.01 ms a step, 1408 leaves of 64^2 434 to 400 us.  Shorter strips, on meshes that do not fill the
     // device, keep two waves, the base at the top of the row, two rows ahead
     // and two per iteration (22.2 to 21.5 us at 256^2 in 32^2 blocks).  Mixed:
     // three waves, two rows per iteration; two rows ahead made stage 1 2 %
