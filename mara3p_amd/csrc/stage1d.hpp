@@ -17,9 +17,10 @@
 // 4.5 to 4.1.
 //
 // A window is one chain where every block boundary in it joins blocks that are
-// linked both ways and consecutive in storage.  At any other boundary (an end of
-// a chain, a neighbour stored elsewhere, links that do not lead back) the lanes
-// on its two sides load the two guard zones of their own block's link
+// linked both ways and consecutive in storage; lanes before the list and past it
+// hold the guard zones of its first and last block.  At any other boundary (an
+// end of a chain, a neighbour stored elsewhere, links that do not lead back) the
+// lanes on its two sides load the two guard zones of their own block's link
 // themselves: blocks are at least 16 zones, so a lane has one such side at
 // most, and one more pass of the left face's arithmetic gives the right faces
 // of all chains that end in the window.  Links are read for blocks of the list
@@ -74,27 +75,35 @@ stage1d_kernel(EulerParams prm, Stage1DArgs a)
     double rate = 0.0;                      // fused CFL reduction
 
     if (lo < end) {
-        // block and zone of lo, then of each lane along the storage order; a
-        // lane before the list or past it holds a zone inside, of no use
+        // block and zone of lo, then of each lane along the storage order
         const int b0 = total < (1l << 31) ? (int)((unsigned)lo / (unsigned)n) : (int)(lo / n);
         const int p0 = (int)(lo - (long)b0 * n) + i - 2;      // the lane's zone counted from block b0's first
         int b = b0, z = p0;
         while (z >= n) { ++b; z -= n; }
         if (z < 0) { --b; z += n; }
         const bool there = b >= 0 && b < a.nblk;
-        const bool edge = !a.pe && i > 0 && z == 0 && b >= 0 && b <= a.nblk;   // a boundary before the lane's zone
+        const bool edge = !a.pe && i > 0 && z == 0 && b > 0 && there;       // a block boundary before the lane's zone
         int prev = -1, next = -1;                             // the links across it
-        if (edge) {
-            if (there) prev = a.nbr[2 * b];
-            if (b > 0) next = a.nbr[2 * (b - 1) + 1];
+        if (edge) { prev = a.nbr[2 * b]; next = a.nbr[2 * (b - 1) + 1]; }
+        const bool cut = edge && !(prev == b - 1 && next == b);
+        // lanes before the list and past it hold the guard zones of its first
+        // and its last block
+        size_t at = (size_t)b * NC * n + z, from = at;
+        bool behind = false;                                  // of a block with no row in the list
+        if (!there) {
+            const int eb = b < 0 ? 0 : a.nblk - 1, ez = b < 0 ? 0 : n - 1;
+            const int link = a.pe ? -1 : a.nbr[b < 0 ? 0 : 2 * a.nblk - 1];
+            const int gz = link < 0 ? ez : b < 0 ? z : min((b - a.nblk) * n + z, n - 1);
+            from = (size_t)(link < 0 ? eb : link) * NC * n + gz;
+            behind = link >= a.nblk && (b < 0 || gz < 2);
+            b = eb;
+            z = ez;
+            at = (size_t)b * NC * n + z;
         }
-        const bool cut = edge && !(there && b > 0 && prev == b - 1 && next == b);
-        if (!there) { b = b0; z = min(max(p0, 0), n - 1); }
-        const size_t at = (size_t)b * NC * n + z;
         double u[NC], u0[NC] = {};
         double dl = a.dl;
 #pragma unroll
-        for (int q = 0; q < NC; ++q) u[q] = a.u[at + (size_t)q * n];
+        for (int q = 0; q < NC; ++q) u[q] = a.u[from + (size_t)q * n];
         if (a.u0) {
 #pragma unroll
             for (int q = 0; q < NC; ++q) u0[q] = a.u0[at + (size_t)q * n];
@@ -138,11 +147,12 @@ stage1d_kernel(EulerParams prm, Stage1DArgs a)
                 if (first || last) {
                     R gq[NC];
 #pragma unroll
-                    for (int q = 0; q < NC; ++q) { g1[q] = away ? g1[q] : u[q]; g2[q] = away ? g2[q] : u[q]; }
-                    bool gok = Euler<R>::recover(g1, prm, gp);
-                    gok &= Euler<R>::recover(g2, prm, gq);
-                    // a guard zone behind the list has no lane of its own to report it
-                    if (away && link >= a.nblk && !gok) report_error(a.err, 1, b, z);
+                    for (int q = 0; q < NC; ++q) gp[q] = gq[q] = p[q];
+                    if (away) {
+                        bool gok = Euler<R>::recover(g1, prm, gp);
+                        gok &= Euler<R>::recover(g2, prm, gq);
+                        if (link >= a.nblk) ok &= gok;        // no lane of the list reports it
+                    }
 #pragma unroll
                     for (int q = 0; q < NC; ++q) {
                         const R h = plm_half(first ? gq[q] : p[q], gp[q], first ? p[q] : gq[q], theta);
@@ -191,11 +201,11 @@ stage1d_kernel(EulerParams prm, Stage1DArgs a)
             else wv[q] = u[q] - dfx[q] * (dt / dl);
             if (a.u0) wv[q] = u0[q] * a.rk_b + wv[q] * (1.0 - a.rk_b);
         }
+        if (!ok && (mine || behind)) report_error(a.err, 1, b, z);
         if (mine) {
             double* o = a.out + at;
 #pragma unroll
             for (int q = 0; q < NC; ++q) o[(size_t)q * n] = wv[q];
-            if (!ok) report_error(a.err, 1, b, z);
             if (a.rate_slot) rate = fmax(rate, Euler<double>::max_speed(wv, prm) * (1.0 / dl));
         }
     }
