@@ -21,8 +21,9 @@
 // with the CFL reduction 48.
 //
 // Zones of a window are one chain where every block boundary in it joins
-// blocks that are linked both ways and consecutive in storage (nearly always).
-// Else the window is cut there, and each part takes the two stages in turn
+// blocks that are linked both ways and consecutive in storage (nearly always);
+// lanes before the list and past it hold the guard zones of its first and last
+// block.  Else the window is cut there, and each part takes the two stages in turn
 // with its zones in their lanes; the lanes beside it hold its guard zones for
 // the while, found once for the whole window: blocks are at least 16 zones,
 // so a lane stands beside one cut at most.  The guard zones lie across the
@@ -63,31 +64,50 @@ rk2_fused_1d_kernel(EulerParams prm, Stage1DArgs a)
     double rate = 0.0;                      // fused CFL reduction
 
     if (lo < end) {
-        // block and zone of lo, then of each lane along the storage order; a
-        // lane before the list or past it holds a zone inside, of no use
+        // block and zone of lo, then of each lane along the storage order
         const int b0 = total < (1l << 31) ? (int)((unsigned)lo / (unsigned)n) : (int)(lo / n);
         const int p0 = (int)(lo - (long)b0 * n) + i - 4;      // the lane's zone counted from block b0's first
         int b = b0, z = p0;
         while (z >= n) { ++b; z -= n; }
         if (z < 0) { --b; z += n; }
         const bool there = b >= 0 && b < a.nblk;
-        const bool edge = i > 0 && z == 0 && b >= 0 && b <= a.nblk;   // a boundary before the lane's zone
+        const bool edge = i > 0 && z == 0 && b > 0 && there;  // a block boundary before the lane's zone
         int prev = -1, next = -1;                             // the links across it
-        if (edge) {
-            if (there) prev = a.nbr[2 * b];
-            if (b > 0) next = a.nbr[2 * (b - 1) + 1];
-        }
-        const bool cut = edge && !(there && b > 0 && prev == b - 1 && next == b);
-        if (!there) { b = b0; z = min(max(p0, 0), n - 1); }
-        const size_t at = (size_t)b * NC * n + z;
+        if (edge) { prev = a.nbr[2 * b]; next = a.nbr[2 * (b - 1) + 1]; }
+        const bool cut = edge && !(prev == b - 1 && next == b);
         const int stop = 4 + (int)(end - lo);                 // lanes 4 .. stop - 1 are the window's own
+
+        // the link of block eb past its lower or upper end; -1 where it leads
+        // nowhere or not back
+        auto link_of = [&] (int link, int eb, bool upper) {
+            if (link >= 0 && a.nbr[2 * link + (upper ? 0 : 1)] != eb) {
+                report_error(a.err, 4, eb, upper ? n : -1);
+                return -1;
+            }
+            return link;
+        };
+        // lanes before the list and past it hold the guard zones of its first
+        // and its last block
+        bool ends = false;                                    // at an outflow there
+        bool g4 = false, g2 = false;                          // one of four, two next to a block, of a block behind the list
+        if (!there) {
+            const bool upper = b > 0;
+            const int eb = upper ? a.nblk - 1 : 0, over = (b - a.nblk) * n + z;
+            const int link = link_of(a.nbr[upper ? 2 * eb + 1 : 0], eb, upper);
+            ends = link < 0;
+            g4 = link >= a.nblk && (upper ? over : n - 1 - z) < 4;
+            g2 = g4 && (upper ? over : n - 1 - z) < 2;
+            z = ends ? (upper ? n - 1 : 0) : upper ? min(over, n - 1) : z;
+            b = ends ? eb : link;
+        }
         // the state is fetched before the links are known (the latencies overlap)
+        const size_t at = (size_t)b * NC * n + z;
         double u0[NC], dl = a.dl;
 #pragma unroll
         for (int q = 0; q < NC; ++q) u0[q] = a.u[at + (size_t)q * n];
         if (a.dl_blk) dl = a.dl_blk[b];
 
-        const unsigned long long cuts = __ballot(cut);
+        const unsigned long long cuts = __ballot(cut), past = __ballot(ends), behind = __ballot(g4);
         int gb = b;                                           // the guard zone that the lane holds for a part
         size_t gat = at;                                      // beside it
         unsigned long long outflow = 0;
@@ -96,21 +116,17 @@ rk2_fused_1d_kernel(EulerParams prm, Stage1DArgs a)
             // lanes of one, the lane is beside the part on its other side
             const unsigned long long upto = (2ull << i) - 1, below = cuts & upto, above = cuts & ~upto;
             const int kd = below ? 63 - __builtin_clzll(below) : 0, ku = above ? __builtin_ctzll(above) : 64;
-            const bool starts = __shfl((int)there, ku & 63, 64);
             const bool up = below && i - kd < 4;              // past the end of the part below
-            const bool dn = above && ku - 1 - i < 4 && starts;
+            const bool dn = above && ku - 1 - i < 4;
             const int eb = __shfl(b, up ? kd - 1 : ku & 63, 64);      // that part's block
             const int from_below = __shfl(next, kd, 64), from_above = __shfl(prev, ku & 63, 64);
             int link = -1;
             if (up || dn) {
-                link = up ? from_below : from_above;
-                if (link >= 0 && a.nbr[2 * link + (up ? 0 : 1)] != eb) {
-                    report_error(a.err, 4, eb, up ? n : -1);
-                    link = -1;
-                }
+                link = link_of(up ? from_below : from_above, eb, up);
                 gb = link < 0 ? eb : link;
                 const int gz = link < 0 ? (up ? n - 1 : 0) : (up ? i - kd : n - ku + i);
                 gat = (size_t)gb * NC * n + gz;
+                if (gb >= a.nblk) { g4 = true; g2 = (up ? i - kd : ku - 1 - i) < 2; }
             }
             outflow = __ballot((up || dn) && link < 0);
         }
@@ -124,6 +140,9 @@ rk2_fused_1d_kernel(EulerParams prm, Stage1DArgs a)
             ka = kb;
             if (kb <= 4) continue;
             const bool in = i >= la && i < kb;
+            // the first and the last lane of the part's chain where an outflow is past it
+            const int low = la > 0 ? (outflow >> (la - 1) & 1 ? la : 0) : past & 1 ? __builtin_ctzll(~past) : 0;
+            const int high = kb < 64 ? (outflow >> kb & 1 ? kb - 1 : 63) : past >> 63 ? 63 - __builtin_clzll(~past) : 63;
             if (cuts) {
                 const double* src = a.u + (in ? at : gat);
 #pragma unroll
@@ -153,22 +172,23 @@ rk2_fused_1d_kernel(EulerParams prm, Stage1DArgs a)
 #pragma unroll
             for (int q = 0; q < NC; ++q) u1[q] = u0[q] - flux_difference(q) * dtdl;
             const bool ok1 = Euler<R>::recover(u1, prm, p);
-            if (cuts) {
+            if (cuts || past || behind) {
                 // a guard zone behind the list has no lane of its own to report it
-                if (!in && gb >= a.nblk && i >= la - 4 && i < kb + 4 && (!ok0 || (!ok1 && i >= la - 2 && i < kb + 2)))
-                    report_error(a.err, 1, b, z);
-                if (la > 0 && outflow >> (la - 1) & 1) {      // the lanes below take the edge zone's, the part's first
+                const int near = __shfl(b, in ? (i < 4 ? 4 : stop - 1) : i < la ? la : kb - 1, 64);
+                if (g4 && (in ? i < 4 || i >= stop : i >= la - 4 && i < kb + 4) && (!ok0 || (g2 && !ok1)))
+                    report_error(a.err, 1, near, i < stop - 1 && i < kb ? 0 : n - 1);
+                if (low > 0) {                                // the lanes below take the edge zone's
 #pragma unroll
                     for (int q = 0; q < NC; ++q) {
-                        const R v = __shfl(p[q], la, 64);
-                        if (i < la) p[q] = v;
+                        const R v = __shfl(p[q], low, 64);
+                        if (i < low) p[q] = v;
                     }
                 }
-                if (kb < 64 && outflow >> kb & 1) {           // and those above the last one's
+                if (high < 63) {                              // and those above the last one's
 #pragma unroll
                     for (int q = 0; q < NC; ++q) {
-                        const R v = __shfl(p[q], kb - 1, 64);
-                        if (i >= kb) p[q] = v;
+                        const R v = __shfl(p[q], high, 64);
+                        if (i > high) p[q] = v;
                     }
                 }
             }
