@@ -15,8 +15,8 @@
 // A workgroup per 64-zone block, a lane per zone, needed 69 and 65 faces of 64
 // lanes in the two stages, two nearly empty passes out of four, took two
 // slopes per face and met four barriers.  512 problems of 512 to 8192 zones in
-// blocks of 64: 55 to 45 us a step (some 530 VALU instructions per 56 zones, 965
-// per 64 before; 201 MB, 4.5 TB/s), with the CFL reduction at half that size 52 to
+// blocks of 64: 55 to 41 us a step (513 VALU instructions per 56 zones, 965 per 64
+// before; 193 MB, 4.8 TB/s), with the CFL reduction at half that size 52 to
 // 36, 300 problems in blocks of 16 16.7 to 8.9.  One-wave workgroups: 48 us,
 // with the CFL reduction 48.
 //
